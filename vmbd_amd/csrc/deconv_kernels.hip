@@ -125,7 +125,7 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
   for (int j = 0; j < NA; ++j) {
     float2 v[16];
     col_load<TH>(v, ins[j], p, c, NB, t, active, grp, row0, cx);
-    if (!ins[j].spec && wact) fft<TH, -1>(v, sl, t, T, tw);
+    if (!ins[j].spec && wact) fft<TH, -1>(v, sl, t, T);
     if (packed) {
 #pragma unroll
       for (int m = 0; m < 16; ++m) pk[j * SL + lds_pad(t + TPT * m)] = v[m];
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
       }
     }
   } else {
-    if (wact) fft<TH, +1>(Z, sl, t, T, tw);
+    if (wact) fft<TH, +1>(Z, sl, t, T);
     col_store_rows<TH, CS, true>(Z, sm, o, p, strip, NB, g.NBP, cc, t);
   }
 }

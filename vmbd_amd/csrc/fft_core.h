@@ -49,85 +49,175 @@ __device__ __forceinline__ void wave_sync() {
 
 // ---------------------------------------------------------------- small DFTs
 // All produce outputs in natural order in place; S = -1 forward, +1 inverse.
-template <int S>
-__device__ __forceinline__ void dft2(float2& a, float2& b) {
-  float2 t = a;
-  a = cadd(t, b);
-  b = csub(t, b);
-}
-
-template <int S>
-__device__ __forceinline__ void dft4(float2& a0, float2& a1, float2& a2, float2& a3) {
-  float2 t0 = cadd(a0, a2), t1 = csub(a0, a2);
-  float2 t2 = cadd(a1, a3), t3 = mul_si<S>(csub(a1, a3));
-  a0 = cadd(t0, t2);
-  a2 = csub(t0, t2);
-  a1 = cadd(t1, t3);
-  a3 = csub(t1, t3);
-}
-
+//
+// Every transform of the operator is bound by VALU issue or waits behind it,
+// and an FMA takes the issue slot of an addition, so both passes are written
+// to put their multiplications into FMAs.  Per 256-point transform and thread
+// (16 points): first pass 144 (from 160: constant twiddles factored out of
+// the sums), second pass 192 (from 160 + 60 for the separate products), 336
+// instead of 380 slots, with 8 twiddle registers pairs instead of 15.
 #define VMBD_R2H 0.70710678118654752440f
 #define VMBD_C8 0.92387953251128675613f  // cos(pi/8)
 #define VMBD_S8 0.38268343236508977173f  // sin(pi/8)
+#define VMBD_T8 0.41421356237309504880f  // tan(pi/8)
 
+// a + s * b, a + S * s * i * b (s real)
+__device__ __forceinline__ float2 cfma(float s, float2 b, float2 a) {
+  return make_float2(fmaf(s, b.x, a.x), fmaf(s, b.y, a.y));
+}
 template <int S>
-__device__ __forceinline__ void dft8(float2* v) {
-  // n = 2 n1 + n2, k = k1 + 4 k2
-  dft4<S>(v[0], v[2], v[4], v[6]);
-  dft4<S>(v[1], v[3], v[5], v[7]);
-  // twiddle w8^(k1) on the odd branch; branch k1 sits in slot 1+2*k1
-  v[3] = cmul(v[3], make_float2(VMBD_R2H, (float)S * VMBD_R2H));
-  v[5] = mul_si<S>(v[5]);
-  v[7] = cmul(v[7], make_float2(-VMBD_R2H, (float)S * VMBD_R2H));
-  float2 o[8];
-#pragma unroll
-  for (int k1 = 0; k1 < 4; ++k1) {
-    o[k1] = cadd(v[2 * k1], v[2 * k1 + 1]);
-    o[k1 + 4] = csub(v[2 * k1], v[2 * k1 + 1]);
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = o[i];
+__device__ __forceinline__ float2 cfma_si(float s, float2 b, float2 a) {
+  return make_float2(fmaf(-(float)S * s, b.y, a.x), fmaf((float)S * s, b.x, a.y));
+}
+// (1 + S i f) * a and (f + S i) * a
+template <int S>
+__device__ __forceinline__ float2 mul_1f(float2 a, float f) {
+  return make_float2(fmaf(-(float)S * f, a.y, a.x), fmaf((float)S * f, a.x, a.y));
+}
+template <int S>
+__device__ __forceinline__ float2 mul_f1(float2 a, float f) {
+  return make_float2(fmaf(f, a.x, -(float)S * a.y), fmaf(f, a.y, (float)S * a.x));
 }
 
-template <int S>
-__device__ __forceinline__ void dft16(float2* v) {
-  // n = 4 n1 + n2, k = k1 + 4 k2.  Step 1: DFT4 over n1 for each n2.
-#pragma unroll
-  for (int n2 = 0; n2 < 4; ++n2) dft4<S>(v[n2], v[n2 + 4], v[n2 + 8], v[n2 + 12]);
-  // now v[n2 + 4*k1] = Y[n2][k1]; twiddle by w16^(n2*k1)
-  const float2 w1 = make_float2(VMBD_C8, (float)S * VMBD_S8);
-  const float2 w2 = make_float2(VMBD_R2H, (float)S * VMBD_R2H);
-  const float2 w3 = make_float2(VMBD_S8, (float)S * VMBD_C8);
-  const float2 w6 = make_float2(-VMBD_R2H, (float)S * VMBD_R2H);
-  const float2 w9 = make_float2(-VMBD_C8, -(float)S * VMBD_S8);
-  v[1 + 4] = cmul(v[5], w1);
-  v[1 + 8] = cmul(v[9], w2);
-  v[1 + 12] = cmul(v[13], w3);
-  v[2 + 4] = cmul(v[6], w2);
-  v[2 + 8] = mul_si<S>(v[10]);
-  v[2 + 12] = cmul(v[14], w6);
-  v[3 + 4] = cmul(v[7], w3);
-  v[3 + 8] = cmul(v[11], w6);
-  v[3 + 12] = cmul(v[15], w9);
-  // Step 3: DFT4 over n2 for each k1 -> X[k1 + 4 k2]
-#pragma unroll
-  for (int k1 = 0; k1 < 4; ++k1) dft4<S>(v[4 * k1 + 0], v[4 * k1 + 1], v[4 * k1 + 2], v[4 * k1 + 3]);
-  // v[4*k1 + k2] = X[k1 + 4 k2]; transpose the 4x4 index grid to natural order
+// 4-point DFT of which the first K inputs are nonzero
+template <int S, int K = 4>
+__device__ __forceinline__ void dft4(float2& a0, float2& a1, float2& a2, float2& a3) {
+  if constexpr (K == 0) {
+    a0 = a1 = a2 = a3 = make_float2(0.f, 0.f);
+  } else if constexpr (K == 1) {
+    a1 = a2 = a3 = a0;
+  } else {
+    const float2 t0 = K > 2 ? cadd(a0, a2) : a0, t1 = K > 2 ? csub(a0, a2) : a0;
+    const float2 t2 = K > 3 ? cadd(a1, a3) : a1, t3 = mul_si<S>(K > 3 ? csub(a1, a3) : a1);
+    a0 = cadd(t0, t2);
+    a2 = csub(t0, t2);
+    a1 = cadd(t1, t3);
+    a3 = csub(t1, t3);
+  }
+}
+
+// 16-point DFT whose inputs r >= NZ are zero (not read)
+template <int S, int NZ = 16>
+__device__ __forceinline__ void dft16(float2 (&v)[16]) {
+  static_assert(NZ >= 3 && NZ <= 16, "NZ in [3,16]");
+  constexpr bool A3 = NZ > 3;  // the n2 = 3 branch has inputs
+  // n = 4 n1 + n2, k = k1 + 4 k2.  Step 1: DFT4 over n1 for each n2:
+  // v[n2 + 4 k1] = Y[n2][k1]
+  dft4<S, (NZ + 3) / 4>(v[0], v[4], v[8], v[12]);
+  dft4<S, (NZ + 2) / 4>(v[1], v[5], v[9], v[13]);
+  dft4<S, (NZ + 1) / 4>(v[2], v[6], v[10], v[14]);
+  dft4<S, NZ / 4>(v[3], v[7], v[11], v[15]);
+  // Step 2 and 3: a_n2 = Y[n2][k1] w16^(n2 k1), DFT4 over n2 -> X[k1 + 4 k2]
   float2 o[16];
-#pragma unroll
-  for (int k1 = 0; k1 < 4; ++k1)
-#pragma unroll
-    for (int k2 = 0; k2 < 4; ++k2) o[k1 + 4 * k2] = v[4 * k1 + k2];
+  float2 t0, t1, u, d;
+  {  // k1 = 0
+    t0 = cadd(v[0], v[2]);
+    t1 = csub(v[0], v[2]);
+    u = A3 ? cadd(v[1], v[3]) : v[1];
+    d = A3 ? csub(v[1], v[3]) : v[1];
+    o[0] = cadd(t0, u);
+    o[8] = csub(t0, u);
+    o[4] = cadd(t1, mul_si<S>(d));
+    o[12] = csub(t1, mul_si<S>(d));
+  }
+  {  // k1 = 1: w1 = C8 (1 + S i T8), w2 = R2H (1 + S i), w3 = C8 (T8 + S i)
+    const float2 p = mul_1f<S>(v[6], 1.f);
+    t0 = cfma(VMBD_R2H, p, v[4]);
+    t1 = cfma(-VMBD_R2H, p, v[4]);
+    const float2 q1 = mul_1f<S>(v[5], VMBD_T8);
+    u = d = q1;
+    if constexpr (A3) {
+      const float2 q3 = mul_f1<S>(v[7], VMBD_T8);
+      u = cadd(q1, q3);
+      d = csub(q1, q3);
+    }
+    o[1] = cfma(VMBD_C8, u, t0);
+    o[9] = cfma(-VMBD_C8, u, t0);
+    o[5] = cfma_si<S>(VMBD_C8, d, t1);
+    o[13] = cfma_si<S>(-VMBD_C8, d, t1);
+  }
+  {  // k1 = 2: w2, w4 = S i, w6 = R2H (-1 + S i) = S i w2
+    t0 = cadd(v[8], mul_si<S>(v[10]));
+    t1 = csub(v[8], mul_si<S>(v[10]));
+    const float2 p1 = mul_1f<S>(v[9], 1.f);
+    u = d = p1;
+    if constexpr (A3) {
+      const float2 p3 = mul_si<S>(mul_1f<S>(v[11], 1.f));
+      u = cadd(p1, p3);
+      d = csub(p1, p3);
+    }
+    o[2] = cfma(VMBD_R2H, u, t0);
+    o[10] = cfma(-VMBD_R2H, u, t0);
+    o[6] = cfma_si<S>(VMBD_R2H, d, t1);
+    o[14] = cfma_si<S>(-VMBD_R2H, d, t1);
+  }
+  {  // k1 = 3: w3 = C8 (T8 + S i), w6 = R2H S i (1 + S i), w9 = -C8 (1 + S i T8)
+    const float2 p = mul_si<S>(mul_1f<S>(v[14], 1.f));
+    t0 = cfma(VMBD_R2H, p, v[12]);
+    t1 = cfma(-VMBD_R2H, p, v[12]);
+    const float2 q1 = mul_f1<S>(v[13], VMBD_T8);
+    u = d = q1;
+    if constexpr (A3) {
+      const float2 q3 = mul_1f<S>(v[15], VMBD_T8);
+      u = csub(q1, q3);
+      d = cadd(q1, q3);
+    }
+    o[3] = cfma(VMBD_C8, u, t0);
+    o[11] = cfma(-VMBD_C8, u, t0);
+    o[7] = cfma_si<S>(VMBD_C8, d, t1);
+    o[15] = cfma_si<S>(-VMBD_C8, d, t1);
+  }
 #pragma unroll
   for (int i = 0; i < 16; ++i) v[i] = o[i];
 }
 
+// Radix-2 butterfly with its twiddle in the sums, six FMAs:
+// a' = a + W b, b' = a - W b = 2a - a'.  w: forward twiddle (conjugated for
+// S = +1); ROT: W = S i w.
+template <int S, bool ROT>
+__device__ __forceinline__ void bfly(float2 a, float2 b, float2 w, float2& hi, float2& lo) {
+  if constexpr (ROT) b = mul_si<S>(b);
+  const float wy = -(float)S * w.y;
+  const float2 t = make_float2(fmaf(-wy, b.y, fmaf(w.x, b.x, a.x)), fmaf(wy, b.x, fmaf(w.x, b.y, a.y)));
+  lo = make_float2(fmaf(2.f, a.x, -t.x), fmaf(2.f, a.y, -t.y));
+  hi = t;
+}
+
+// Twiddles of an R-point DFT of w^r x_r: level R (spans R/2) uses w e_R^k,
+// k < R/2, of which the second half is S i times the first; then level R/2
+// with w^2, and so on.  Kept per level: R/4 (one at R = 2), R/2 in all.
+template <int R>
+struct TwCount {
+  static constexpr int top = R > 2 ? R / 4 : 1;
+  static constexpr int n = R > 2 ? top + TwCount<(R > 2 ? R / 2 : 2)>::n : 1;
+};
+template <>
+struct TwCount<2> {
+  static constexpr int top = 1, n = 1;
+};
+
+// X[k] = sum_r x_r w^r e^{S 2 pi i r k / R}, decimation in time, natural order
 template <int R, int S>
-__device__ __forceinline__ void dftR(float2* v) {
-  if constexpr (R == 16) dft16<S>(v);
-  else if constexpr (R == 8) dft8<S>(v);
-  else if constexpr (R == 4) dft4<S>(v[0], v[1], v[2], v[3]);
-  else dft2<S>(v[0], v[1]);
+__device__ __forceinline__ void dft_tw(float2* x, const float2* w) {
+  if constexpr (R == 2) {
+    const float2 a = x[0], b = x[1];
+    bfly<S, false>(a, b, w[0], x[0], x[1]);
+  } else {
+    constexpr int H = R / 2;
+    float2 e[H], o[H];
+#pragma unroll
+    for (int j = 0; j < H; ++j) {
+      e[j] = x[2 * j];
+      o[j] = x[2 * j + 1];
+    }
+    dft_tw<H, S>(e, w + TwCount<R>::top);
+    dft_tw<H, S>(o, w + TwCount<R>::top);
+#pragma unroll
+    for (int k = 0; k < H / 2; ++k) {
+      bfly<S, false>(e[k], o[k], w[k], x[k], x[k + H]);
+      bfly<S, true>(e[k + H / 2], o[k + H / 2], w[k], x[k + H / 2], x[k + H / 2 + H]);
+    }
+  }
 }
 
 // LDS slot of element i inside a transform's slice (one pad slot per 16).
@@ -137,35 +227,6 @@ struct FftLds {
   static constexpr int floats2 = N + N / 16;  // float2 slots per transform
 };
 
-// w^r for r = 0..R-1 where w = twiddle base.
-template <int R>
-__device__ __forceinline__ void twiddle_powers(float2 w1, float2 w4, float2* p) {
-  p[0] = make_float2(1.f, 0.f);
-  p[1] = w1;
-  if constexpr (R > 2) {
-    p[2] = cmul(w1, w1);
-    p[3] = cmul(p[2], w1);
-  }
-  if constexpr (R > 4) {
-    p[4] = w4;
-    p[5] = cmul(w4, w1);
-    p[6] = cmul(w4, p[2]);
-    p[7] = cmul(w4, p[3]);
-  }
-  if constexpr (R > 8) {
-    float2 w8 = cmul(w4, w4);
-    p[8] = w8;
-    p[9] = cmul(w8, w1);
-    p[10] = cmul(w8, p[2]);
-    p[11] = cmul(w8, p[3]);
-    float2 w12 = cmul(w8, w4);
-    p[12] = w12;
-    p[13] = cmul(w12, w1);
-    p[14] = cmul(w12, p[2]);
-    p[15] = cmul(w12, p[3]);
-  }
-}
-
 // Radix plan of a length-N transform after the first radix-16 pass.
 template <int N>
 struct Plan {
@@ -173,87 +234,132 @@ struct Plan {
   static constexpr int R2 = (N > 256) ? N / 256 : 1;   // third pass radix
 };
 
-// Per-thread forward twiddles of the second pass (span 16): the thread's
-// 16/R1 butterflies j = t + b*TPT use w^(r*(j mod 16)), w = e^{-2 pi i/(16 R1)}.
-// They depend only on t, so a kernel computes them once and reuses them for
-// every transform it performs.  The (optional) third pass loads its twiddles.
+// Per-thread forward twiddles of the passes after the first, in the order of
+// TwCount.  Second pass (span 16): the thread's 16/R1 butterflies j = t + b*TPT
+// use w = e^{-2 pi i (j mod 16) / (16 R1)}.  Third pass (span 256): butterflies
+// j = t + b*TPT use w = e^{-2 pi i j / (256 R2)}, of which b and b + 4 (R2 = 2)
+// differ by a quarter turn, so four are kept.  They depend only on t: a kernel
+// sets them up once for every transform it performs.
 template <int N>
 struct Twiddles {
   static constexpr int R1 = Plan<N>::R1;
+  static constexpr int R2 = Plan<N>::R2;
   static constexpr int NB1 = (R1 > 1) ? 16 / R1 : 1;
-  static constexpr int CNT = (R1 > 1) ? NB1 * (R1 - 1) : 1;
-  float2 w[CNT];
+  static constexpr int C1 = (R1 > 1) ? TwCount<(R1 > 1 ? R1 : 2)>::n : 1;
+  static constexpr int C2 = (R2 > 1) ? TwCount<(R2 > 1 ? R2 : 2)>::n : 1;
+  float2 w[NB1 * C1];
+  float2 w3[(R2 > 1) ? 4 * C2 : 1];
 };
 
-// LOAD=true reads every twiddle from the table (best when a thread performs
-// several transforms); LOAD=false reads two and builds the powers by complex
-// multiplication (fewer memory instructions for one transform per thread).
-template <int N, bool LOAD = false>
-__device__ __forceinline__ void twiddles_init(Twiddles<N>& T, int t, const float2* __restrict__ tw) {
-  constexpr int TPT = N / 16;
-  constexpr int R1 = Plan<N>::R1;
-  if constexpr (R1 > 1) {
-    constexpr int NB1 = 16 / R1;
-    constexpr int STR = TW_LEN / (16 * R1);
+// twiddle array of an R-point DFT from w = tw[i] (table index i)
+template <int R>
+__device__ __forceinline__ void tw_load(float2* w, int i, const float2* __restrict__ tw) {
+  constexpr int top = TwCount<R>::top;
 #pragma unroll
-    for (int b = 0; b < NB1; ++b) {
-      const int k = (t + b * TPT) & 15;
-      if constexpr (LOAD) {
-#pragma unroll
-        for (int r = 1; r < R1; ++r) T.w[b * (R1 - 1) + r - 1] = tw[(k * r * STR) & (TW_LEN - 1)];
-      } else {
-        float2 p[R1];
-        twiddle_powers<R1>(tw[k * STR], tw[(4 * k * STR) & (TW_LEN - 1)], p);
-#pragma unroll
-        for (int r = 1; r < R1; ++r) T.w[b * (R1 - 1) + r - 1] = p[r];
-      }
-    }
+  for (int k = 0; k < top; ++k) w[k] = tw[(i + k * (TW_LEN / R)) & (TW_LEN - 1)];
+  if constexpr (R > 2) tw_load<R / 2>(w + top, 2 * i, tw);
+}
+// the same from w and w^4 by products
+template <int R>
+__device__ __forceinline__ void tw_powers(float2* w, float2 w1, float2 w4) {
+  const float2 e8 = make_float2(VMBD_R2H, -VMBD_R2H);
+  if constexpr (R == 2) {
+    w[0] = w1;
+  } else if constexpr (R == 4) {
+    w[0] = w1;
+    w[1] = cmul(w1, w1);
+  } else if constexpr (R == 8) {
+    w[0] = w1;
+    w[1] = cmul(w1, e8);
+    w[2] = cmul(w1, w1);
+    w[3] = w4;
+  } else {
+    w[0] = w1;
+    w[1] = cmul(w1, make_float2(VMBD_C8, -VMBD_S8));
+    w[2] = cmul(w1, e8);
+    w[3] = cmul(w1, make_float2(VMBD_S8, -VMBD_C8));
+    w[4] = cmul(w1, w1);
+    w[5] = cmul(w[4], e8);
+    w[6] = w4;
+    w[7] = cmul(w4, w4);
   }
 }
 
-// The same twiddles in two steps: twiddles_seed issues the table loads (two
-// per butterfly), twiddles_from_seed forms the powers, so the loads can be in
-// flight with other work while only the seeds hold registers.
+// table index of the second pass's w for butterfly b, of the third pass's w
+template <int N>
+__device__ __forceinline__ int tw_index1(int t, int b) {
+  return ((t + b * (N / 16)) & 15) * (TW_LEN / (16 * Plan<N>::R1));
+}
+template <int N>
+__device__ __forceinline__ int tw_index2(int t, int b) {
+  return (t + b * (N / 16)) * (TW_LEN / (256 * Plan<N>::R2));
+}
+
+// The twiddles in two steps: twiddles_seed issues the table loads (w and w^4
+// of each second-pass butterfly, w of the third pass's), twiddles_from_seed
+// forms the others, so the loads can be in flight with other work while only
+// the seeds hold registers.
 template <int N>
 struct TwSeed {
   static constexpr int NB1 = Twiddles<N>::NB1;
-  float2 w1[NB1], w4[NB1];
+  float2 w1[NB1], w4[NB1], w3[4];
 };
 template <int N>
 __device__ __forceinline__ void twiddles_seed(TwSeed<N>& S, int t, const float2* __restrict__ tw) {
-  constexpr int TPT = N / 16;
-  constexpr int R1 = Plan<N>::R1;
-  if constexpr (R1 > 1) {
-    constexpr int STR = TW_LEN / (16 * R1);
+  if constexpr (Plan<N>::R1 > 1) {
 #pragma unroll
     for (int b = 0; b < TwSeed<N>::NB1; ++b) {
-      const int k = (t + b * TPT) & 15;
-      S.w1[b] = tw[k * STR];
-      S.w4[b] = tw[(4 * k * STR) & (TW_LEN - 1)];
+      S.w1[b] = tw[tw_index1<N>(t, b)];
+      if constexpr (Plan<N>::R1 > 4) S.w4[b] = tw[4 * tw_index1<N>(t, b) & (TW_LEN - 1)];
     }
+  }
+  if constexpr (Plan<N>::R2 > 1) {
+#pragma unroll
+    for (int b = 0; b < 4; ++b) S.w3[b] = tw[tw_index2<N>(t, b)];
   }
 }
 template <int N>
 __device__ __forceinline__ void twiddles_from_seed(Twiddles<N>& T, const TwSeed<N>& S) {
-  constexpr int R1 = Plan<N>::R1;
+  constexpr int R1 = Plan<N>::R1, R2 = Plan<N>::R2;
   if constexpr (R1 > 1) {
 #pragma unroll
-    for (int b = 0; b < TwSeed<N>::NB1; ++b) {
-      float2 p[R1];
-      twiddle_powers<R1>(S.w1[b], S.w4[b], p);
+    for (int b = 0; b < TwSeed<N>::NB1; ++b) tw_powers<R1>(T.w + b * Twiddles<N>::C1, S.w1[b], S.w4[b]);
+  }
+  if constexpr (R2 > 1) {
 #pragma unroll
-      for (int r = 1; r < R1; ++r) T.w[b * (R1 - 1) + r - 1] = p[r];
-    }
+    for (int b = 0; b < 4; ++b) tw_powers<R2>(T.w3 + b * Twiddles<N>::C2, S.w3[b], S.w3[b]);
   }
 }
 
-// One Stockham pass after the first (Ns > 1).  Reads 16 values of the slice,
-// applies 16/R butterflies, writes 16 values (or keeps them in registers when
-// LAST: slot m = b + r*(16/R) holds X[t + TPT*m]).  Twiddles come from `pre`
-// (per-thread forward twiddles, conjugated for S=+1) or from the table.
-template <int N, int R, int NS, int S, bool LAST, bool PRE>
-__device__ __forceinline__ void stockham_pass(float2 (&v)[16], float2* sl, int t, const float2* pre,
-                                              const float2* __restrict__ tw) {
+// LOAD=true reads every twiddle from the table (best when a thread performs
+// several transforms); LOAD=false reads the seeds and builds the others
+// (fewer memory instructions for one transform per thread).
+template <int N, bool LOAD = false>
+__device__ __forceinline__ void twiddles_init(Twiddles<N>& T, int t, const float2* __restrict__ tw) {
+  if constexpr (LOAD) {
+    if constexpr (Plan<N>::R1 > 1) {
+#pragma unroll
+      for (int b = 0; b < Twiddles<N>::NB1; ++b)
+        tw_load<(Plan<N>::R1 > 1 ? Plan<N>::R1 : 2)>(T.w + b * Twiddles<N>::C1, tw_index1<N>(t, b), tw);
+    }
+    if constexpr (Plan<N>::R2 > 1) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        tw_load<(Plan<N>::R2 > 1 ? Plan<N>::R2 : 2)>(T.w3 + b * Twiddles<N>::C2, tw_index2<N>(t, b), tw);
+    }
+  } else {
+    TwSeed<N> S;
+    twiddles_seed<N>(S, t, tw);
+    twiddles_from_seed<N>(T, S);
+  }
+}
+
+// One Stockham pass after the first (NS > 1).  Reads 16 values of the slice,
+// applies 16/R butterflies with their twiddles (w: NB or, on a quarter turn
+// from the first four, 4 arrays of TwCount<R>::n), writes 16 values (or keeps
+// them in registers when LAST: slot m = b + r*(16/R) holds X[t + TPT*m]).
+template <int N, int R, int NS, int S, bool LAST>
+__device__ __forceinline__ void stockham_pass(float2 (&v)[16], float2* sl, int t, const float2* w) {
   constexpr int TPT = N / 16;
   constexpr int NB = 16 / R;
   float2 in[16];
@@ -269,23 +375,16 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[16], float2* sl, int t
     const int j = t + b * TPT;
     const int k = j & (NS - 1);
     float2* q = in + b * R;
-    if constexpr (PRE) {
-#pragma unroll
-      for (int r = 1; r < R; ++r) q[r] = (S < 0) ? cmul(q[r], pre[b * (R - 1) + r - 1]) : cmulc(q[r], pre[b * (R - 1) + r - 1]);
+    if constexpr (NS > 16 && R == 2) {
+      // third pass of 512 points: butterfly b + 4 on a quarter turn from b
+      const float2 x = q[0], y = q[1];
+      if (b < 4)
+        bfly<S, false>(x, y, w[b & 3], q[0], q[1]);
+      else
+        bfly<S, true>(x, y, w[b & 3], q[0], q[1]);
     } else {
-      constexpr int STR = TW_LEN / (NS * R);
-      float2 w1 = tw[k * STR];
-      float2 w4 = tw[(4 * k * STR) & (TW_LEN - 1)];
-      if (S > 0) {
-        w1 = cconj(w1);
-        w4 = cconj(w4);
-      }
-      float2 p[R];
-      twiddle_powers<R>(w1, w4, p);
-#pragma unroll
-      for (int r = 1; r < R; ++r) q[r] = cmul(q[r], p[r]);
+      dft_tw<R, S>(q, w + b * TwCount<R>::n);
     }
-    dftR<R, S>(q);
     if constexpr (LAST) {
 #pragma unroll
       for (int r = 0; r < R; ++r) v[b + r * NB] = q[r];
@@ -302,33 +401,25 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[16], float2* sl, int t
 // v: input mapping on entry, output mapping on exit.  S=-1 forward, +1 inverse
 // (unscaled).  Must be called by all TPT threads of the transform.
 // NZ < 16: the caller guarantees x[t + TPT*r] = 0 for r >= NZ; those slots are
-// taken as constant zeros, so the first pass shrinks to the arithmetic the
-// nonzero inputs need (outputs a caller never reads are removed the same way
-// by the compiler once the call is inlined).
+// not read, and the first pass shrinks to the arithmetic the nonzero inputs
+// need (outputs a caller never reads are removed by the compiler once the
+// call is inlined).
 template <int N, int S, int NZ = 16>
-__device__ __forceinline__ void fft(float2 (&v)[16], float2* sl, int t, const Twiddles<N>& T,
-                                    const float2* __restrict__ tw) {
+__device__ __forceinline__ void fft(float2 (&v)[16], float2* sl, int t, const Twiddles<N>& T) {
   static_assert(N >= 16 && N <= 1024 && (N & (N - 1)) == 0, "N must be a power of two in [16,1024]");
-  static_assert(NZ >= 1 && NZ <= 16, "NZ in [1,16]");
-  if constexpr (NZ < 16) {
-#pragma unroll
-    for (int r = NZ; r < 16; ++r) v[r] = make_float2(0.f, 0.f);
-  }
   // pass 0: radix 16, Ns = 1, j = t, no twiddles; output index t*16 + r
-  dft16<S>(v);
-  if constexpr (N == 16) {
-    return;
-  } else {
+  dft16<S, NZ>(v);
+  if constexpr (N > 16) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) sl[lds_pad(t * 16 + r)] = v[r];
     wave_sync();
     constexpr int R1 = Plan<N>::R1;
     constexpr int R2 = Plan<N>::R2;
     if constexpr (R2 == 1) {
-      stockham_pass<N, R1, 16, S, true, true>(v, sl, t, T.w, tw);
+      stockham_pass<N, R1, 16, S, true>(v, sl, t, T.w);
     } else {
-      stockham_pass<N, R1, 16, S, false, true>(v, sl, t, T.w, tw);
-      stockham_pass<N, R2, 256, S, true, false>(v, sl, t, nullptr, tw);
+      stockham_pass<N, R1, 16, S, false>(v, sl, t, T.w);
+      stockham_pass<N, R2, 256, S, true>(v, sl, t, T.w3);
     }
   }
 }

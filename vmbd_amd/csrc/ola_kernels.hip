@@ -157,12 +157,12 @@ __device__ __forceinline__ void rows_r2c_body(Geo g, RowSrc s, float2* __restric
 #pragma unroll
       for (int r = 0; r < 3; ++r) v[r] = sl[lds_pad(t + TPT * r)];
       wave_sync();
-      fft<TW, -1, (TW <= 256 ? 3 : 16)>(v, sl, t, T, tw);
+      fft<TW, -1, (TW <= 256 ? 3 : 16)>(v, sl, t, T);
     } else {
 #pragma unroll
       for (int r = 0; r < 16; ++r) v[r] = sl[lds_pad(t + TPT * r)];
       wave_sync();
-      fft<TW, -1>(v, sl, t, T, tw);
+      fft<TW, -1>(v, sl, t, T);
     }
     // natural-order spectrum of z = a + i b into the slice, then split
 #pragma unroll
@@ -503,14 +503,14 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
   constexpr bool PRUNE = !(TH >= 512 && OP == COL_ADJ2);
   if (PRUNE && (OP == COL_FWD || OP == COL_SPEC) && !a.spec && a.rlo + a.nr <= 3 * TPT) {
     col_load<TH, 3, XA>(A, a, p, c, NB, t, active, grp, row0, cx);
-    if (wact) fft<TH, -1, 3>(A, sl, t, T, tw);
+    if (wact) fft<TH, -1, 3>(A, sl, t, T);
   } else if (PRUNE && XA && !a.spec && a.rlo + a.nr <= 12 * TPT) {
     // image rows of a patch of at most 3/4 of the tile height
     col_load<TH, 12, XA>(A, a, p, c, NB, t, active, grp, row0, cx);
-    if (wact) fft<TH, -1, 12>(A, sl, t, T, tw);
+    if (wact) fft<TH, -1, 12>(A, sl, t, T);
   } else {
     col_load<TH, 16, XA>(A, a, p, c, NB, t, active, grp, row0, cx);
-    if (!a.spec && wact) fft<TH, -1>(A, sl, t, T, tw);
+    if (!a.spec && wact) fft<TH, -1>(A, sl, t, T);
   }
   if constexpr (OP == COL_SPEC) {
     if (active) {
@@ -527,35 +527,35 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
     float2 B[16];
     if (PRUNE && !b.spec && b.rlo + b.nr <= 3 * TPT) {
       col_load<TH, 3, XB>(B, b, p, c, NB, t, active, grp, row0, cx);
-      if (wact) fft<TH, -1, 3>(B, sl, t, T, tw);
+      if (wact) fft<TH, -1, 3>(B, sl, t, T);
     } else {
       col_load<TH, 16, XB>(B, b, p, c, NB, t, active, grp, row0, cx);
-      if (!b.spec && wact) fft<TH, -1>(B, sl, t, T, tw);
+      if (!b.spec && wact) fft<TH, -1>(B, sl, t, T);
     }
     {
       constexpr bool SPREAD = SPREAD1;
       VMBD_COL_PRODUCT(OP != COL_FWD, A, B);
     }
     if (OP == COL_ADJ1 && o1.nrows <= 3 * TPT) {
-      if (wact) fft<TH, +1>(B, sl, t, T, tw);
+      if (wact) fft<TH, +1>(B, sl, t, T);
       col_store_rows<TH, CS, true, 3, WGC>(B, sm, o1, p, strip, NB, g.NBP, cc, t);
     } else {
-      if (wact) fft<TH, +1>(B, sl, t, T, tw);
+      if (wact) fft<TH, +1>(B, sl, t, T);
       col_store_rows<TH, CS, OP != COL_ADJ2, 16, WGC>(B, sm, o1, p, strip, NB, g.NBP, cc, t);
     }
     if constexpr (OP == COL_ADJ2) {
       if (PRUNE && !c3.spec && c3.rlo + c3.nr <= 12 * TPT) {
         col_load<TH, 12, true>(B, c3, p, c, NB, t, active, grp, row0, cx);
-        if (wact) fft<TH, -1, 12>(B, sl, t, T, tw);
+        if (wact) fft<TH, -1, 12>(B, sl, t, T);
       } else {
         col_load<TH, 16, true>(B, c3, p, c, NB, t, active, grp, row0, cx);
-        if (!c3.spec && wact) fft<TH, -1>(B, sl, t, T, tw);
+        if (!c3.spec && wact) fft<TH, -1>(B, sl, t, T);
       }
       {
         constexpr bool SPREAD = SPREAD2;
         VMBD_COL_PRODUCT(true, A, B);
       }
-      if (wact) fft<TH, +1>(B, sl, t, T, tw);
+      if (wact) fft<TH, +1>(B, sl, t, T);
       if (PRUNE && o2.nrows <= 3 * TPT)
         col_store_rows<TH, CS, true, 3, WGC>(B, sm, o2, p, strip, NB, g.NBP, cc, t);
       else
@@ -849,7 +849,7 @@ __device__ __forceinline__ void c2r_ola_body(Geo g, OlaDst d, int i, int fr, flo
     // single-round launch holds slices for its items only
     if (act) {
       c2r_load<TW>(v, ra, rb, rok, rok && hasb, sl, t);
-      fft<TW, +1>(v, sl, t, T, tw);
+      fft<TW, +1>(v, sl, t, T);
     } else {
 #pragma unroll
       for (int mm = 0; mm < 16; ++mm) v[mm] = make_float2(0.f, 0.f);
@@ -1153,7 +1153,7 @@ __device__ __forceinline__ void c2r_sum_body(Geo g, OlaDst d, int i0, int fr, fl
     Twiddles<TW> T;
     twiddles_from_seed<TW>(T, S);
     c2r_stage<TW>(v, A, B, sl, t);
-    fft<TW, +1>(v, sl, t, T, tw);
+    fft<TW, +1>(v, sl, t, T);
   }
   __syncthreads();  // the slices become class rows; column weights staged
   {
@@ -1505,7 +1505,7 @@ __device__ __forceinline__ void c2r_stack_body(Geo g, const float2* __restrict__
   float2 v[16];
   float2* sl = fl + tr * SL;
   c2r_load<TW>(v, ra, rb, act, hasb, sl, t);
-  fft<TW, +1>(v, sl, t, T, tw);
+  fft<TW, +1>(v, sl, t, T);
   if (act) {
 #pragma unroll
     for (int mm = 0; mm < 16; ++mm) {

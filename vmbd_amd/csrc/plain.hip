@@ -131,7 +131,7 @@ __global__ __launch_bounds__(TB) void k_fft_rows(float2* data, long long rows, f
   float2 v[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) v[r] = act ? rp[t + TPT * r] : make_float2(0.f, 0.f);
-  fft<N, S>(v, sm + tr * SL, t, T, tw);
+  fft<N, S>(v, sm + tr * SL, t, T);
   if (act) {
 #pragma unroll
     for (int m = 0; m < 16; ++m) rp[t + TPT * m] = cscale(v[m], scale);
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(TB) void k_fft_cols(float2* data, int Tw, int strip
   __syncthreads();
   Twiddles<N> T;
   twiddles_init<N>(T, t, tw);
-  fft<N, S>(v, sm + cc * SL, t, T, tw);
+  fft<N, S>(v, sm + cc * SL, t, T);
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < 16; ++m) sm[(t + TPT * m) * (CS + 1) + cc] = cscale(v[m], scale);
