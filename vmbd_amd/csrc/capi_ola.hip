@@ -206,6 +206,7 @@ SharedRows residual_rows(const vmbd_plan* p, const Geo& g, const float* gres, in
   r.g = g;
   r.g.csf0 = 1;
   r.g.Pf = g.csf1;
+  r.g.dPf = g.dcsf1;
   r.g.P = (g.P / g.Pf) * g.csf1;
   return r;
 }
@@ -267,6 +268,7 @@ XRows x_rows(const vmbd_plan* p, const Geo& g, const float* x, bool alone) {
   r.s.czr = p->fac_czr;
   r.g.csf0 = 1;
   r.g.Pf = g.csf1;
+  r.g.dPf = g.dcsf1;
   r.g.P = (g.P / g.Pf) * g.csf1;
   r.in = ColIn{p->wsX, 0, g.sw0, 0, row_pitch(S0), 1};
   r.in.rsc = p->fac_rsc;
@@ -416,6 +418,8 @@ vmbd_plan* vmbd_plan_create(const vmbd_geom* gm, const float* win_table, int32_t
   g.csf1 = G.csf1;
   g.Pf = G.csf0 * G.csf1;
   g.P = g.Pf;
+  g.dPf = fast_div(g.Pf);
+  g.dcsf1 = fast_div(g.csf1);
   g.sw0 = G.sw0;
   g.sw1 = G.sw1;
   g.hop0 = G.nhop0;

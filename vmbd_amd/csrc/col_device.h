@@ -21,37 +21,71 @@ struct cmax {
 // (gfx950 vector memory accepts unaligned addresses)
 __device__ __forceinline__ void ld4(float (&d)[4], const float* p) { __builtin_memcpy(d, p, 16); }
 
-// NZ < 16: only slots r < NZ can hold stored rows (rlo + nr <= NZ*TPT); the
-// rest are zero without a load.  XS: the operand may be shared image rows
-// with patch-row factors (in.rsc); only those call sites carry that path.
-template <int TH, int NZ = 16, bool XS = false>
-__device__ __forceinline__ void col_load(float2 (&v)[16], const ColIn& in, int p, int c, int NB, int t, bool active,
-                                         int grp, int row0, const ColCtx& cx) {
-  constexpr int TPT = TH / 16;
-  if constexpr (NZ < 16) {
-#pragma unroll
-    for (int r = NZ; r < 16; ++r) v[r] = make_float2(0.f, 0.f);
+// Slots of a column against the operand's stored rows [rlo, rlo + nr): bit r
+// of `full` where all TPT rows of slot r are stored, of `part` where some
+// are.  Both are uniform, so the loads below branch on the scalar unit.
+struct ColSlots {
+  unsigned full, part;
+};
+template <int TPT>
+__device__ __forceinline__ ColSlots col_slots(int rlo, int nr) {
+  const int hi = rlo + nr;
+  const unsigned in = (1u << (hi / TPT)) - 1u, some = (1u << ((hi + TPT - 1) / TPT)) - 1u;
+  ColSlots m;
+  m.full = in & ~((1u << ((rlo + TPT - 1) / TPT)) - 1u);
+  m.part = some & ~((1u << (rlo / TPT)) - 1u) & ~m.full;
+  return m;
+}
+
+// Slot r of a column from base[vo + TPT*r] (T: float2 rows, or their float
+// factors): a full slot is a plain load at an immediate offset, a partial one
+// (at most two per column) takes a lane mask, the others are zero.
+template <int TPT, class T>
+__device__ __forceinline__ void col_slot(T& v, const T* base, unsigned vo, int t, int r, int rlo, int nr, ColSlots m) {
+  v = T{};
+  if (m.full >> r & 1) v = (base + vo)[TPT * r];
+  if (m.part >> r & 1) {
+    asm volatile("");  // keeps this block a scalar branch, not lane selects in every slot
+    const int rr = t + TPT * r - rlo;
+    if (rr >= 0 && rr < nr) v = (base + vo)[TPT * r];
   }
-  if (in.spec) {
-    const float2* col = in.p + ((size_t)p * NB + c) * TH;
+}
+
+// Column c of a cached spectrum.  Here and below, addresses are a uniform
+// base plus one 32-bit lane offset, and columns past the last bin read the
+// last one (their results are never stored): 6-8 VALU instructions per slot
+// less than with a masked 64-bit address of its own.
+template <int TH>
+__device__ __forceinline__ void col_load_spec(float2 (&v)[16], const ColIn& in, int p, int c, int NB, int t) {
+  constexpr int TPT = TH / 16;
+  const float2* base = in.p + (size_t)p * NB * TH;
+  const unsigned vo = (unsigned)min(c, NB - 2) * TH + t;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = active ? col[t + TPT * r] : make_float2(0.f, 0.f);
-  } else if (XS && in.rsc) {
-    // shared image rows, each scaled by its patch row's factor.  The factors
-    // are loaded unconditionally (index clamped into the table, so no load
-    // waits behind a branch) and applied once the column's loads are in.
-    const float2* col = in.p + ((size_t)grp * NB + c) * in.pitch + row0;
-    const float* rs = in.rsc + (size_t)cx.pm * in.nr;
+  for (int r = 0; r < 16; ++r) v[r] = (base + vo)[TPT * r];
+}
+
+// Column c of row-pass output in the FFT input mapping.  NZ < 16: only slots
+// r < NZ can hold stored rows (rlo + nr <= NZ*TPT); the others are left unset
+// (the transform does not read them).  XS: shared image rows, each scaled by
+// its patch row's factor in.rsc.
+template <int TH, int NZ = 16, bool XS = false>
+__device__ __forceinline__ void col_load(float2 (&v)[16], const ColIn& in, int p, int c, int NB, int t, int grp,
+                                         int row0, const ColCtx& cx) {
+  constexpr int TPT = TH / 16;
+  const float2* base =
+      (in.shared ? in.p + (size_t)grp * NB * in.pitch + row0 : in.p + (size_t)p * NB * in.pitch) - in.rlo;
+  const unsigned vo = (unsigned)min(c, NB - 2) * (unsigned)in.pitch + t;
+  const ColSlots m = col_slots<TPT>(in.rlo, in.nr);
+  if constexpr (!XS) {
+#pragma unroll
+    for (int r = 0; r < NZ; ++r) col_slot<TPT>(v[r], base, vo, t, r, in.rlo, in.nr, m);
+  } else {
+    const float* rs = in.rsc + (size_t)cx.pm * in.nr - in.rlo;
     float sc[NZ];
 #pragma unroll
     for (int r = 0; r < NZ; ++r) {
-      const int rr = t + TPT * r - in.rlo;
-      sc[r] = rs[min(max(rr, 0), in.nr - 1)];
-    }
-#pragma unroll
-    for (int r = 0; r < NZ; ++r) {
-      const int rr = t + TPT * r - in.rlo;
-      v[r] = (active && rr >= 0 && rr < in.nr) ? col[rr] : make_float2(0.f, 0.f);
+      col_slot<TPT>(sc[r], rs, (unsigned)t, t, r, in.rlo, in.nr, m);
+      col_slot<TPT>(v[r], base, vo, t, r, in.rlo, in.nr, m);
     }
 #pragma unroll
     for (int r = 0; r < NZ; ++r) {
@@ -86,20 +120,10 @@ __device__ __forceinline__ void col_load(float2 (&v)[16], const ColIn& in, int p
 #pragma unroll
         for (int r = 0; r < NZ; ++r) {
           const float dl = __shfl(tab[(TPT * r) / 64], (TPT * r) % 64 + t, 64);
-          if (active) {
-            v[r].x += dl * E.x;
-            v[r].y += dl * E.y;
-          }
+          v[r].x += dl * E.x;
+          v[r].y += dl * E.y;
         }
       }
-    }
-  } else {
-    const float2* col = in.shared ? in.p + ((size_t)grp * NB + c) * in.pitch + row0
-                                  : in.p + ((size_t)p * NB + c) * in.pitch;
-#pragma unroll
-    for (int r = 0; r < NZ; ++r) {
-      const int rr = t + TPT * r - in.rlo;
-      v[r] = (active && rr >= 0 && rr < in.nr) ? col[rr] : make_float2(0.f, 0.f);
     }
   }
 }
@@ -114,18 +138,42 @@ template <int TH, int CS, bool LAST = false, int MM = 16, int WGC = WG>
 __device__ __forceinline__ void col_store_rows(const float2 (&v)[16], float2* st, const ColOut& o, int p, int strip,
                                                int NB, int NBP, int cc, int t) {
   constexpr int TPT = TH / 16;
+  constexpr int RS = WGC / CS;  // rows stored per step (= TPT)
+  const int nrows = o.nrows;
   __syncthreads();  // all transforms of the workgroup are done with the slices
+  float2* sw = st + t * (CS + 1) + cc;
 #pragma unroll
   for (int m = 0; m < MM; ++m) {
-    const int r = t + TPT * m;
-    if (r < o.nrows) st[r * (CS + 1) + cc] = v[m];
+    if (TPT * (m + 1) <= nrows)  // uniform: no lane mask on whole slots
+      sw[TPT * m * (CS + 1)] = v[m];
+    else if (t + TPT * m < nrows)
+      sw[TPT * m * (CS + 1)] = v[m];
   }
   __syncthreads();
   const int c0 = strip * CS;
   const int ci = threadIdx.x & (CS - 1);
   if (c0 + ci < NB - 1) {  // bin NB-1 travels packed in bin 0
-    float2* dst = o.p + (size_t)p * o.nrows * NBP + c0 + ci;
-    for (int r = threadIdx.x / CS; r < o.nrows; r += WGC / CS) dst[(size_t)r * NBP] = st[r * (CS + 1) + ci];
+    const int r0 = threadIdx.x / CS;
+    float2* dst = o.p + (size_t)p * nrows * NBP + c0;
+    const unsigned vo = (unsigned)(r0 * NBP + ci);
+    const float2* sr = st + r0 * (CS + 1) + ci;
+    const size_t step = (size_t)RS * NBP;
+    int k = 0;
+    // four steps of whole rows at a time, their LDS reads together
+    for (; k + 4 * RS <= nrows; k += 4 * RS) {
+      float2 x[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = sr[i * RS * (CS + 1)];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) (dst + i * step)[vo] = x[i];
+      dst += 4 * step;
+      sr += 4 * RS * (CS + 1);
+    }
+    for (; k < nrows; k += RS) {
+      if (k + r0 < nrows) dst[vo] = sr[0];
+      dst += step;
+      sr += RS * (CS + 1);
+    }
   }
   if (!LAST) __syncthreads();  // staging drained before the slices are reused
 }

@@ -78,6 +78,8 @@ __device__ __forceinline__ float2 div_value(const float2 (&o)[4], int cx, int k,
 template <int OP>
 struct DivArity {
   static constexpr int n = (OP == DIV_X || OP == DIV_SPROD) ? 2 : 4;
+  // operand j is a cached spectrum
+  static constexpr bool spec(int j) { return (OP == DIV_X || OP == DIV_SPROD) ? j == 1 : OP == DIV_S && j >= 2; }
 };
 
 template <int TH, int OP>
@@ -95,16 +97,15 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
 
   const int NB = g.NB;
   const int strip = blockIdx.x;
-  const int p = (int)blockIdx.z * g.Pf + (int)blockIdx.y;
+  const int pfr = blockIdx.z, pk_ = blockIdx.y;
+  const int p = pfr * g.Pf + pk_;
   const int cc = threadIdx.x / TPT;
   const int t = threadIdx.x - cc * TPT;
   const int c = strip * CS + cc;
   const bool active = c < NB - 1;  // bins [0, NB-1); NB-1 travels packed in bin 0
   const bool packed = c == 0;
   const bool wact = strip * CS + (int)(threadIdx.x >> 6) * (64 / TPT) < NB - 1;
-  const int pfr = p / g.Pf;
-  const int pk_ = p - pfr * g.Pf;
-  const int pm = pk_ / g.csf1;
+  const int pm = div_by(pk_, g.dcsf1);
   const int grp = pfr * g.csf1 + (pk_ - pm * g.csf1);
   const int row0 = pm * g.hop0;
   const ColCtx cx{pm, pk_ - pm * g.csf1, pfr, g.hop0, g.Tw, tw};
@@ -124,8 +125,12 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
 #pragma unroll
   for (int j = 0; j < NA; ++j) {
     float2 v[16];
-    col_load<TH>(v, ins[j], p, c, NB, t, active, grp, row0, cx);
-    if (!ins[j].spec && wact) fft<TH, -1>(v, sl, t, T);
+    if (DivArity<OP>::spec(j)) {
+      col_load_spec<TH>(v, ins[j], p, c, NB, t);
+    } else {
+      col_load<TH>(v, ins[j], p, c, NB, t, grp, row0, cx);
+      if (wact) fft<TH, -1>(v, sl, t, T);
+    }
     if (packed) {
 #pragma unroll
       for (int m = 0; m < 16; ++m) pk[j * SL + lds_pad(t + TPT * m)] = v[m];
@@ -251,6 +256,10 @@ hipError_t launch_cols_div(const Geo& g, int op, const ColIn* a, int na, DivPara
                            float2* spec_out, const float2* tw, hipStream_t st) {
   const int need = (op == DIV_X || op == DIV_SPROD) ? 2 : 4;
   if (na != need || g.P <= 0) return hipErrorInvalidValue;
+  for (int j = 0; j < na; ++j) {  // spectra where the kernel reads spectra
+    const bool spec = op == DIV_X || op == DIV_SPROD ? j == 1 : op == DIV_S && j >= 2;
+    if ((a[j].spec != 0) != spec) return hipErrorInvalidValue;
+  }
   ColIn in[4] = {a[0], a[1], ColIn{}, ColIn{}};
   if (na == 4) {
     in[2] = a[2];

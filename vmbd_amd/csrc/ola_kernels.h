@@ -5,6 +5,23 @@
 
 namespace vmbd {
 
+// Division of 0 <= n < 2^31 by a divisor fixed on the host, as one high
+// product: m = ceil(2^(31+s) / d) with s = ceil(log2 d) is below 2^32, and its
+// excess over 2^(31+s)/d moves n*m / 2^(31+s) by less than 1/d.  Workgroup
+// uniform operands stay on the scalar unit (three instructions; the
+// compiler's division takes about 25 vector instructions each).
+struct FastDiv {
+  unsigned m, s;
+};
+inline FastDiv fast_div(int d) {
+  unsigned s = 0;
+  while (s < 31 && (1u << s) < (unsigned)d) ++s;
+  return FastDiv{(unsigned)(((1ull << (31 + s)) + (unsigned)d - 1) / (unsigned)d), s};
+}
+__host__ __device__ inline int div_by(int n, FastDiv d) {
+  return (int)((unsigned)(((unsigned long long)((unsigned)n << 1) * d.m) >> 32) >> d.s);
+}
+
 // Patch-grid geometry of one operator instance, passed by value to kernels.
 //   image x: H x W;  PSF stack f: P x sf0 x sf1;  patch k = m*csf1 + n at
 //   origin (m*hop0, n*hop1);  FFT tile Th x Tw;  half spectrum NB = Tw/2+1 slots
@@ -24,6 +41,7 @@ struct Geo {
   int ext0, ext1;
   int oc0, oc1;
   int sy0, sy1;
+  FastDiv dPf, dcsf1;  // division by Pf and csf1
 };
 
 // Source of the rows fed to the row transform (chop / pad / window fused).

@@ -450,13 +450,17 @@ struct ColsLds {
   static constexpr int v = (OP == COL_SPEC) ? CS * FftLds<TH>::floats2 : cmax<CS * FftLds<TH>::floats2, TH * (CS + 1)>::v;
 };
 
-// One workgroup of WGC threads of the column pass: strip `strip` of patch p
+// One workgroup of WGC threads of the column pass: strip `strip` of patch pk of frame pfr
 // (sm: ColsLds<TH, OP, WGC>::v float2 of LDS).
-template <int TH, int OP, int WGC = WG>
+// XS: the image operand (the forward's and the spectra's first, the
+// f-adjoint's second, the two-adjoint pass's third) is shared image rows.
+// BSPEC: the second operand is a cached spectrum.  Both are template
+// parameters, so a kernel holds the code of its own operands only.
+template <int TH, int OP, bool XS, bool BSPEC, int WGC = WG>
 // (parameters by value: with references the compiler keeps the column
 // descriptors in vector registers and spills at 256 points)
 __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, ColOut o1, ColOut o2,
-                                          float2* __restrict__ spec_out, int strip, int p, float2* sm,
+                                          float2* __restrict__ spec_out, int strip, int pk, int pfr, float2* sm,
                                           const float2* __restrict__ tw) {
   constexpr int TPT = TH / 16;
   constexpr int CS = WGC / TPT;  // columns per workgroup
@@ -480,16 +484,14 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
   // a wavefront whose columns all lie past the last bin skips its transforms
   const bool wact = strip * CS + (int)(threadIdx.x >> 6) * (64 / TPT) < NB - 1;
   // group and row offset of this patch in shared row transforms
-  const int pfr = p / g.Pf;
-  const int pk = p - pfr * g.Pf;
-  const int pm = pk / g.csf1;
+  const int p = pfr * g.Pf + pk;
+  const int pm = div_by(pk, g.dcsf1);
   const int grp = pfr * g.csf1 + (pk - pm * g.csf1);
   const int row0 = pm * g.hop0;
   const ColCtx cx{pm, pk - pm * g.csf1, pfr, g.hop0, g.Tw, tw};
-  // operands that may be shared image rows: the forward's and the spectra's
-  // first, the f-adjoint's second, the two-adjoint pass's third
-  constexpr bool XA = OP == COL_FWD || OP == COL_SPEC;
-  constexpr bool XB = OP == COL_ADJ1;
+  constexpr bool XA = XS && (OP == COL_FWD || OP == COL_SPEC);
+  constexpr bool XB = XS && OP == COL_ADJ1;
+  constexpr bool XC = XS && OP == COL_ADJ2;
   float2* sl = sm + cc * SL;
 
   Twiddles<TH> T;
@@ -501,22 +503,23 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
   // 3*TPT rows (f-adjoint) for the inverse transform's last pass.  Not in
   // the 512-point two-adjoint pass, whose registers the extra paths spill.
   constexpr bool PRUNE = !(TH >= 512 && OP == COL_ADJ2);
-  if (PRUNE && (OP == COL_FWD || OP == COL_SPEC) && !a.spec && a.rlo + a.nr <= 3 * TPT) {
-    col_load<TH, 3, XA>(A, a, p, c, NB, t, active, grp, row0, cx);
+  if (!XA && PRUNE && (OP == COL_FWD || OP == COL_SPEC) && a.rlo + a.nr <= 3 * TPT) {
+    col_load<TH, 3>(A, a, p, c, NB, t, grp, row0, cx);
     if (wact) fft<TH, -1, 3>(A, sl, t, T);
-  } else if (PRUNE && XA && !a.spec && a.rlo + a.nr <= 12 * TPT) {
+  } else if (PRUNE && (OP == COL_FWD || OP == COL_SPEC) && a.rlo + a.nr <= 12 * TPT) {
     // image rows of a patch of at most 3/4 of the tile height
-    col_load<TH, 12, XA>(A, a, p, c, NB, t, active, grp, row0, cx);
+    col_load<TH, 12, XA>(A, a, p, c, NB, t, grp, row0, cx);
     if (wact) fft<TH, -1, 12>(A, sl, t, T);
   } else {
-    col_load<TH, 16, XA>(A, a, p, c, NB, t, active, grp, row0, cx);
-    if (!a.spec && wact) fft<TH, -1>(A, sl, t, T);
+    col_load<TH, 16, XA>(A, a, p, c, NB, t, grp, row0, cx);
+    if (wact) fft<TH, -1>(A, sl, t, T);
   }
   if constexpr (OP == COL_SPEC) {
     if (active) {
-      float2* col = spec_out + ((size_t)p * NB + c) * TH;
+      float2* col = spec_out + (size_t)p * NB * TH;
+      const unsigned vo = (unsigned)(c * TH + t);
 #pragma unroll
-      for (int m = 0; m < 16; ++m) col[t + TPT * m] = A[m];
+      for (int m = 0; m < 16; ++m) (col + vo)[TPT * m] = A[m];
       if (packed) {  // bin NB-1 travels in bin 0: its column is written as zeros
         float2* coln = spec_out + ((size_t)p * NB + NB - 1) * TH;
 #pragma unroll
@@ -525,12 +528,14 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
     }
   } else {
     float2 B[16];
-    if (PRUNE && !b.spec && b.rlo + b.nr <= 3 * TPT) {
-      col_load<TH, 3, XB>(B, b, p, c, NB, t, active, grp, row0, cx);
+    if constexpr (BSPEC) {
+      col_load_spec<TH>(B, b, p, c, NB, t);
+    } else if (!XB && PRUNE && b.rlo + b.nr <= 3 * TPT) {
+      col_load<TH, 3>(B, b, p, c, NB, t, grp, row0, cx);
       if (wact) fft<TH, -1, 3>(B, sl, t, T);
     } else {
-      col_load<TH, 16, XB>(B, b, p, c, NB, t, active, grp, row0, cx);
-      if (!b.spec && wact) fft<TH, -1>(B, sl, t, T);
+      col_load<TH, 16, XB>(B, b, p, c, NB, t, grp, row0, cx);
+      if (wact) fft<TH, -1>(B, sl, t, T);
     }
     {
       constexpr bool SPREAD = SPREAD1;
@@ -544,12 +549,12 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
       col_store_rows<TH, CS, OP != COL_ADJ2, 16, WGC>(B, sm, o1, p, strip, NB, g.NBP, cc, t);
     }
     if constexpr (OP == COL_ADJ2) {
-      if (PRUNE && !c3.spec && c3.rlo + c3.nr <= 12 * TPT) {
-        col_load<TH, 12, true>(B, c3, p, c, NB, t, active, grp, row0, cx);
+      if (PRUNE && c3.rlo + c3.nr <= 12 * TPT) {
+        col_load<TH, 12, XC>(B, c3, p, c, NB, t, grp, row0, cx);
         if (wact) fft<TH, -1, 12>(B, sl, t, T);
       } else {
-        col_load<TH, 16, true>(B, c3, p, c, NB, t, active, grp, row0, cx);
-        if (!c3.spec && wact) fft<TH, -1>(B, sl, t, T);
+        col_load<TH, 16, XC>(B, c3, p, c, NB, t, grp, row0, cx);
+        if (wact) fft<TH, -1>(B, sl, t, T);
       }
       {
         constexpr bool SPREAD = SPREAD2;
@@ -569,18 +574,38 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
 // workgroups per CU.  Strips of one patch are consecutive workgroups; each
 // writes whole 128-byte lines of its rows (16 bins, row pitch NBP a multiple
 // of 16).
-template <int TH, int OP, int WGC>
+template <int TH, int OP, bool XS, bool BSPEC, int WGC>
 __global__ __launch_bounds__(WGC, (TH >= 256 ? 4 * WG / WGC : 1)) void k_cols(Geo g, ColIn a, ColIn b, ColIn c3,
                                                                              ColOut o1, ColOut o2,
                                                                              float2* __restrict__ spec_out,
                                                                              const float2* __restrict__ tw) {
   __shared__ float2 sm[ColsLds<TH, OP, WGC>::v];
   // frame blockIdx.z, patch blockIdx.y
-  cols_body<TH, OP, WGC>(g, a, b, c3, o1, o2, spec_out, blockIdx.x, (int)blockIdx.z * g.Pf + (int)blockIdx.y, sm,
-                         tw);
+  cols_body<TH, OP, XS, BSPEC, WGC>(g, a, b, c3, o1, o2, spec_out, blockIdx.x, blockIdx.y, blockIdx.z, sm, tw);
 }
 
 #undef VMBD_COL_PRODUCT
+
+// the template arguments of a launch's operands (launch_cols checked them)
+template <int TH, int OP, int WGC>
+static void cols_op(const Geo& g, const ColIn& a, const ColIn& b, const ColIn& c, const ColOut& o1, const ColOut& o2,
+                    float2* spec_out, const float2* tw, hipStream_t st, const dim3& grid) {
+  const bool xs = (OP == COL_ADJ1 ? b.rsc : OP == COL_ADJ2 ? c.rsc : a.rsc) != nullptr;
+  auto go = [&](auto k) { hipLaunchKernelGGL(k, grid, dim3(WGC), 0, st, g, a, b, c, o1, o2, spec_out, tw); };
+  if constexpr (OP == COL_FWD) {
+    if (b.spec)
+      xs ? go(k_cols<TH, OP, true, true, WGC>) : go(k_cols<TH, OP, false, true, WGC>);
+    else
+      xs ? go(k_cols<TH, OP, true, false, WGC>) : go(k_cols<TH, OP, false, false, WGC>);
+  } else if constexpr (OP == COL_ADJ1) {
+    if (b.spec)
+      go(k_cols<TH, OP, false, true, WGC>);
+    else
+      xs ? go(k_cols<TH, OP, true, false, WGC>) : go(k_cols<TH, OP, false, false, WGC>);
+  } else {
+    xs ? go(k_cols<TH, OP, true, false, WGC>) : go(k_cols<TH, OP, false, false, WGC>);
+  }
+}
 
 template <int TH, int WGC>
 static hipError_t cols_wg(const Geo& g, int op, const ColIn& a, const ColIn& b, const ColIn& c, const ColOut& o1,
@@ -591,20 +616,11 @@ static hipError_t cols_wg(const Geo& g, int op, const ColIn& a, const ColIn& b, 
   static const char* names[4] = {"cols_spec", "cols_fwd", "cols_adj1", "cols_adj2"};
   ProfScope ps(names[op & 3], st);
   switch (op) {
-    case COL_SPEC:
-      hipLaunchKernelGGL((k_cols<TH, COL_SPEC, WGC>), grid, dim3(WGC), 0, st, g, a, b, c, o1, o2, spec_out, tw);
-      break;
-    case COL_FWD:
-      hipLaunchKernelGGL((k_cols<TH, COL_FWD, WGC>), grid, dim3(WGC), 0, st, g, a, b, c, o1, o2, spec_out, tw);
-      break;
-    case COL_ADJ1:
-      hipLaunchKernelGGL((k_cols<TH, COL_ADJ1, WGC>), grid, dim3(WGC), 0, st, g, a, b, c, o1, o2, spec_out, tw);
-      break;
-    case COL_ADJ2:
-      hipLaunchKernelGGL((k_cols<TH, COL_ADJ2, WGC>), grid, dim3(WGC), 0, st, g, a, b, c, o1, o2, spec_out, tw);
-      break;
-    default:
-      return hipErrorInvalidValue;
+    case COL_SPEC: cols_op<TH, COL_SPEC, WGC>(g, a, b, c, o1, o2, spec_out, tw, st, grid); break;
+    case COL_FWD: cols_op<TH, COL_FWD, WGC>(g, a, b, c, o1, o2, spec_out, tw, st, grid); break;
+    case COL_ADJ1: cols_op<TH, COL_ADJ1, WGC>(g, a, b, c, o1, o2, spec_out, tw, st, grid); break;
+    case COL_ADJ2: cols_op<TH, COL_ADJ2, WGC>(g, a, b, c, o1, o2, spec_out, tw, st, grid); break;
+    default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
@@ -619,6 +635,8 @@ static hipError_t cols_t(const Geo& g, int op, const ColIn& a, const ColIn& b, c
 hipError_t launch_cols(const Geo& g, int op, const ColIn& a, const ColIn& b, const ColIn& c, const ColOut& o1,
                        const ColOut& o2, float2* spec_out, const float2* tw, hipStream_t st, int wgc) {
   if (wgc != 0 && wgc != 128 && wgc != WG) return hipErrorInvalidValue;
+  // a cached spectrum is the second operand of the forward and of one adjoint
+  if (a.spec || c.spec || (b.spec && op != COL_FWD && op != COL_ADJ1)) return hipErrorInvalidValue;
   switch (g.Th) {
     case 16: return cols_t<16>(g, op, a, b, c, o1, o2, spec_out, tw, st, wgc);
     case 32: return cols_t<32>(g, op, a, b, c, o1, o2, spec_out, tw, st, wgc);
@@ -1599,10 +1617,22 @@ __global__ __launch_bounds__(WG, (TH >= 256 ? 4 : 1)) void k_batch_cols(const Ba
   const int strips = (B.g.NB - 1 + CS - 1) / CS;
   const int p = lb / strips;
   if (p >= B.g.P) return;
+  const int strip = lb - p * strips;
+  const int pfr = div_by(p, B.g.dPf);
+  const int pk = p - pfr * B.g.Pf;
   if constexpr (OP == COL_FWD)
-    cols_body<TH, COL_FWD>(B.g, B.cf_a, B.cf_b, B.cf_b, B.cf_o, B.cf_o, nullptr, lb - p * strips, p, sm, B.tw);
+    if (B.cf_a.rsc)
+      cols_body<TH, COL_FWD, true, false>(B.g, B.cf_a, B.cf_b, B.cf_b, B.cf_o, B.cf_o, nullptr, strip, pk, pfr, sm,
+                                          B.tw);
+    else
+      cols_body<TH, COL_FWD, false, false>(B.g, B.cf_a, B.cf_b, B.cf_b, B.cf_o, B.cf_o, nullptr, strip, pk, pfr, sm,
+                                           B.tw);
+  else if (B.ca_c.rsc)
+    cols_body<TH, COL_ADJ2, true, false>(B.g, B.ca_a, B.ca_b, B.ca_c, B.ca_o1, B.ca_o2, nullptr, strip, pk, pfr, sm,
+                                         B.tw);
   else
-    cols_body<TH, COL_ADJ2>(B.g, B.ca_a, B.ca_b, B.ca_c, B.ca_o1, B.ca_o2, nullptr, lb - p * strips, p, sm, B.tw);
+    cols_body<TH, COL_ADJ2, false, false>(B.g, B.ca_a, B.ca_b, B.ca_c, B.ca_o1, B.ca_o2, nullptr, strip, pk, pfr, sm,
+                                          B.tw);
 }
 
 // WGS < WG: every group of the launch holds its row in one round of WGS
