@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -344,17 +345,24 @@ OlaDst dst_adjoint_x(const vmbd_plan* p, float* xbar) {
 
 // row transforms of x and f: one launch over both (one geometry, or, with
 // the image rows shared per patch column, a geometry per job)
+// One launch of the row transforms of up to four operands, each over the
+// patches of its own geometry
+struct RowOp {
+  const Geo& g;
+  const RowSrc& s;
+  float2* out;
+};
+hipError_t launch_rows(const vmbd_plan* p, const Geo& g, std::initializer_list<RowOp> ops, hipStream_t st,
+                       const char* name) {
+  RowJobs jobs{};
+  for (const RowOp& o : ops)
+    if (!row_job(jobs, o.g, o.s, o.out)) return hipErrorInvalidValue;
+  return launch_rows_r2c(g, jobs, p->tw, st, name);
+}
+
 hipError_t launch_xf_rows(const vmbd_plan* p, const Geo& g, const XRows& xr, const RowSrc& sf, hipStream_t st) {
-  if (!xr.shared) {
-    RowSrc srcs[2] = {xr.s, sf};
-    float2* outs[2] = {p->wsX, p->wsF};
-    return launch_rows_r2c_multi(g, srcs, outs, 2, p->tw, st);
-  }
-  // the shared image rows (one geometry per patch column) beside the PSF rows
-  const RowSrc srcs[2] = {xr.s, sf};
-  float2* outs[2] = {p->wsX, p->wsF};
-  const int P[2] = {xr.g.P, g.P}, Pf[2] = {xr.g.Pf, g.Pf};
-  return launch_rows_r2c_geo(g, srcs, outs, P, Pf, 2, p->tw, st, "rows_r2c_x_psf");
+  return launch_rows(p, g, {{xr.g, xr.s, p->wsX}, {g, sf, p->wsF}}, st,
+                     xr.shared ? "rows_r2c_x_psf" : "rows_r2c_multi");
 }
 
 #define VMBD_LAUNCH(expr)                                            \
@@ -420,6 +428,8 @@ vmbd_plan* vmbd_plan_create(const vmbd_geom* gm, const float* win_table, int32_t
   g.P = g.Pf;
   g.dPf = fast_div(g.Pf);
   g.dcsf1 = fast_div(g.csf1);
+  g.dNP2 = fast_div((g.csf1 + 1) / 2);
+  g.dhop0 = fast_div(G.nhop0);
   g.sw0 = G.sw0;
   g.sw1 = G.sw1;
   g.hop0 = G.nhop0;
@@ -802,8 +812,7 @@ int vmbd_ola_adjoint_x(vmbd_plan* p, int32_t nframes, const float* gres, const f
   p->rows_frames = 0;
   const SharedRows sr = residual_rows(p, g, gres, exact);
   const RowSrc sf = src_psf(p, f);
-  VMBD_LAUNCH(launch_rows_r2c(sr.g, sr.s, p->wsG, p->tw, st));
-  VMBD_LAUNCH(launch_rows_r2c(g, sf, p->wsF, p->tw, st, "rows_r2c_psf"));
+  VMBD_LAUNCH(launch_rows(p, g, {{sr.g, sr.s, p->wsG}, {g, sf, p->wsF}}, st, "rows_r2c_res_psf"));
   ColOut o1{p->Y1, g.sw0}, o2{nullptr, 0};
   ColIn none{};
   VMBD_LAUNCH(launch_cols(g, COL_ADJ1, shared_in(p->wsG, sr), raw_in(p->wsF, sf), none, o1, o2, nullptr, p->tw, st, p->tune.col_threads));
@@ -822,8 +831,7 @@ int vmbd_ola_adjoint_f(vmbd_plan* p, int32_t nframes, const float* gres, const f
   const SharedRows sr = residual_rows(p, g, gres, exact);
   // the form of vmbd_ola_adjoint_xf, so that both give f-bar bit for bit
   const XRows xr = x_rows(p, g, x, false);
-  VMBD_LAUNCH(launch_rows_r2c(sr.g, sr.s, p->wsG, p->tw, st));
-  VMBD_LAUNCH(launch_rows_r2c(xr.g, xr.s, p->wsX, p->tw, st, "rows_r2c_x"));
+  VMBD_LAUNCH(launch_rows(p, g, {{sr.g, sr.s, p->wsG}, {xr.g, xr.s, p->wsX}}, st, "rows_r2c_res_x"));
   ColOut o1{p->Y2, g.sf0}, o2{nullptr, 0};
   ColIn none{};
   VMBD_LAUNCH(launch_cols(g, COL_ADJ1, shared_in(p->wsG, sr), xr.in, none, o1, o2, nullptr, p->tw, st, p->tune.col_threads));
@@ -846,7 +854,7 @@ int vmbd_ola_adjoint_xf(vmbd_plan* p, int32_t nframes, const float* gres, const 
   const SharedRows sr = residual_rows(p, g, gres, exact);
   const XRows xr = x_rows(p, g, x, false);
   const RowSrc sf = src_psf(p, f);
-  VMBD_LAUNCH(launch_rows_r2c(sr.g, sr.s, p->wsG, p->tw, st));
+  VMBD_LAUNCH(launch_rows(p, g, {{sr.g, sr.s, p->wsG}}, st, "rows_r2c"));
   if (!reuse) {
     p->rows_frames = 0;
     VMBD_LAUNCH(launch_xf_rows(p, g, xr, sf, st));
@@ -903,11 +911,11 @@ int vmbd_spectra(vmbd_plan* p, int32_t nframes, int32_t kind, const float* z, vo
   ColIn in;
   if (kind == VMBD_CACHE_PSF) {
     const RowSrc s = src_psf(p, z);
-    VMBD_LAUNCH(launch_rows_r2c(g, s, p->wsF, p->tw, st, "rows_r2c_psf"));
+    VMBD_LAUNCH(launch_rows(p, g, {{g, s, p->wsF}}, st, "rows_r2c_psf"));
     in = raw_in(p->wsF, s);
   } else {
     const XRows xr = x_rows(p, g, z, true);
-    VMBD_LAUNCH(launch_rows_r2c(xr.g, xr.s, p->wsX, p->tw, st, "rows_r2c_x"));
+    VMBD_LAUNCH(launch_rows(p, g, {{xr.g, xr.s, p->wsX}}, st, "rows_r2c_x"));
     in = xr.in;
   }
   ColOut none_o{nullptr, 0};
@@ -930,11 +938,11 @@ int vmbd_ola_forward_cached_ex(vmbd_plan* p, int32_t nframes, int32_t kind, cons
   ColIn in;
   if (kind == VMBD_CACHE_PSF) {
     const XRows xr = x_rows(p, g, u, true);
-    VMBD_LAUNCH(launch_rows_r2c(xr.g, xr.s, p->wsX, p->tw, st, "rows_r2c_x"));
+    VMBD_LAUNCH(launch_rows(p, g, {{xr.g, xr.s, p->wsX}}, st, "rows_r2c_x"));
     in = xr.in;
   } else {
     const RowSrc s = src_psf(p, u);
-    VMBD_LAUNCH(launch_rows_r2c(g, s, p->wsF, p->tw, st, "rows_r2c_psf"));
+    VMBD_LAUNCH(launch_rows(p, g, {{g, s, p->wsF}}, st, "rows_r2c_psf"));
     in = raw_in(p->wsF, s);
   }
   ColOut o1{p->Y1, g.ext0}, o2{nullptr, 0};
@@ -962,7 +970,7 @@ int vmbd_ola_adjoint_cached_ex(vmbd_plan* p, int32_t nframes, int32_t kind, cons
   hipStream_t st = (hipStream_t)stream;
   const Geo g = call_geo(p, nframes);
   const SharedRows sr = residual_rows(p, g, gres, exact);
-  VMBD_LAUNCH(launch_rows_r2c(sr.g, sr.s, p->wsG, p->tw, st));
+  VMBD_LAUNCH(launch_rows(p, g, {{sr.g, sr.s, p->wsG}}, st, "rows_r2c"));
   ColIn none{};
   ColOut o2{nullptr, 0};
   if (kind == VMBD_CACHE_PSF) {
@@ -1077,7 +1085,7 @@ int vmbd_deconv_direct(vmbd_plan* p, int32_t kind, const void* spec, const float
   // the observation's patch at the mode offset times the window at tile
   // offset 0 (olaGPU.py:577-581)
   const RowSrc s = windowed(p, src_chop(p, y, g.sy0, g.sy1, g.oc0, g.oc1), 0, 0);
-  VMBD_LAUNCH(launch_rows_r2c(g, s, p->wsX, p->tw, st));
+  VMBD_LAUNCH(launch_rows(p, g, {{g, s, p->wsX}}, st, "rows_r2c"));
   const ColIn in[2] = {raw_in(p->wsX, s), spec_in(spec, g.Th)};
   const DivParams prm{alpha, beta, 0.f};
   if (kind == VMBD_CACHE_PSF) {
@@ -1103,7 +1111,9 @@ int vmbd_deconv_gdirect(vmbd_plan* p, const float* xx, const float* xy, const fl
   const RowSrc srcs[4] = {src_chop(p, xx, g.H, g.W - 1, 0, 0), src_chop(p, yx, g.sy0, g.sy1 - 1, g.oc0, g.oc1),
                           src_chop(p, xy, g.H - 1, g.W, 0, 0), src_chop(p, yy, g.sy0 - 1, g.sy1, g.oc0, g.oc1)};
   float2* outs[4] = {work_rows(p, work, 0), work_rows(p, work, 1), work_rows(p, work, 2), work_rows(p, work, 3)};
-  VMBD_LAUNCH(launch_rows_r2c_multi(g, srcs, outs, 4, p->tw, st));
+  VMBD_LAUNCH(launch_rows(
+      p, g, {{g, srcs[0], outs[0]}, {g, srcs[1], outs[1]}, {g, srcs[2], outs[2]}, {g, srcs[3], outs[3]}}, st,
+      "rows_r2c_multi"));
   const ColIn in[4] = {raw_in(outs[0], srcs[0]), raw_in(outs[1], srcs[1]), raw_in(outs[2], srcs[2]),
                        raw_in(outs[3], srcs[3])};
   VMBD_LAUNCH(launch_cols_div(g, DIV_G, in, 4, DivParams{alpha, beta, 0.f}, ColOut{p->Y2, g.sf0}, nullptr, p->tw,
@@ -1126,7 +1136,7 @@ int vmbd_deconv_sparse_setup(vmbd_plan* p, const void* spec, const float* y, con
   const RowSrc srcs[2] = {windowed(p, src_chop(p, y, g.sy0, g.sy1, g.oc0, g.oc1), g.oc0, g.oc1),
                           windowed(p, src_chop(p, c, g.sy0, g.sy1, g.oc0, g.oc1), g.oc0, g.oc1)};
   float2* outs[2] = {work_rows(p, work, 0), work_rows(p, work, 1)};
-  VMBD_LAUNCH(launch_rows_r2c_multi(g, srcs, outs, 2, p->tw, st));
+  VMBD_LAUNCH(launch_rows(p, g, {{g, srcs[0], outs[0]}, {g, srcs[1], outs[1]}}, st, "rows_r2c_multi"));
   // F^H y, kept as a spectrum for every half-quadratic step (olaGPU.py:690-692)
   const ColIn yin[2] = {raw_in(outs[0], srcs[0]), spec_in(spec, g.Th)};
   VMBD_LAUNCH(launch_cols_div(g, DIV_SPROD, yin, 2, DivParams{0.f, 0.f, 0.f}, ColOut{nullptr, 0}, (float2*)ftpy,
@@ -1159,7 +1169,7 @@ int vmbd_deconv_sparse_step(vmbd_plan* p, const void* spec, const void* ftpy, co
   // shrunk gradients at offset 0 (olaGPU.py:700-712)
   const RowSrc srcs[2] = {src_chop(p, wx, wx_rows, wx_cols, 0, 0), src_chop(p, wy, wy_rows, wy_cols, 0, 0)};
   float2* outs[2] = {work_rows(p, work, 0), work_rows(p, work, 1)};
-  VMBD_LAUNCH(launch_rows_r2c_multi(g, srcs, outs, 2, p->tw, st));
+  VMBD_LAUNCH(launch_rows(p, g, {{g, srcs[0], outs[0]}, {g, srcs[1], outs[1]}}, st, "rows_r2c_multi"));
   const ColIn in[4] = {raw_in(outs[0], srcs[0]), raw_in(outs[1], srcs[1]), spec_in(ftpy, g.Th), spec_in(spec, g.Th)};
   VMBD_LAUNCH(launch_cols_div(g, DIV_S, in, 4, DivParams{alpha, beta, gamma}, ColOut{p->Y1, g.sw0}, nullptr, p->tw,
                               st));
@@ -1194,46 +1204,23 @@ namespace {
 
 // the step's parameters of one group: vmbd_ola_forward followed by
 // vmbd_ola_adjoint_xf reusing the forward's row transforms
-BatchGroup batch_group(vmbd_plan* p, int nframes, const float* x, const float* f, const float* gres, float* y,
-                       float* xbar, float* fbar, int exact) {
-  BatchGroup B{};
+bool batch_group(BatchGroup& B, vmbd_plan* p, int nframes, const float* x, const float* f, const float* gres, float* y,
+                 float* xbar, float* fbar, int exact) {
+  B = BatchGroup{};
   const Geo g = call_geo(p, nframes);
   B.g = g;
   B.tw = p->tw;
   const XRows xr = x_rows(p, g, x, false);
   const RowSrc sf = src_psf(p, f);
-  const int TPW = WG / (g.Tw / 16);
-  auto blocks = [&](const RowSrc& s) { return ((s.rhi - s.rlo + 1) / 2 + TPW - 1) / TPW; };
-  if (xr.shared) {  // the image rows in a pass of their own (their geometry)
-    B.rows_fwd.n = 1;
-    B.rows_fwd.s[0] = sf;
-    B.rows_fwd.out[0] = p->wsF;
-    B.rows_fwd.blk_end[0] = blocks(sf);
-    B.gx = xr.g;
-    B.rows_x.n = 1;
-    B.rows_x.s[0] = xr.s;
-    B.rows_x.out[0] = p->wsX;
-    B.rows_x.blk_end[0] = blocks(xr.s);
-  } else {
-    B.rows_fwd.n = 2;
-    B.rows_fwd.s[0] = xr.s;
-    B.rows_fwd.s[1] = sf;
-    B.rows_fwd.out[0] = p->wsX;
-    B.rows_fwd.out[1] = p->wsF;
-    B.rows_fwd.blk_end[0] = blocks(xr.s);
-    B.rows_fwd.blk_end[1] = B.rows_fwd.blk_end[0] + blocks(sf);
-  }
+  // shared image rows take a pass of their own, others run beside the PSF rows
+  bool ok = row_job(xr.shared ? B.rows_x : B.rows_fwd, xr.g, xr.s, p->wsX) && row_job(B.rows_fwd, g, sf, p->wsF);
   B.cf_a = xr.in;
   B.cf_b = raw_in(p->wsF, sf);
   B.cf_o = ColOut{p->Y1, g.ext0};
   B.ola_fwd = dst_forward(p, y);
   ola_fit_rows(B.ola_fwd, (long long)B.ola_fwd.O0 * nframes);
   const SharedRows sr = residual_rows(p, g, gres, exact);
-  B.gres = sr.g;
-  B.rows_res.n = 1;
-  B.rows_res.s[0] = sr.s;
-  B.rows_res.out[0] = p->wsG;
-  B.rows_res.blk_end[0] = blocks(sr.s);
+  ok = ok && row_job(B.rows_res, sr.g, sr.s, p->wsG);
   B.ca_a = shared_in(p->wsG, sr);
   B.ca_b = raw_in(p->wsF, sf);
   B.ca_c = xr.in;
@@ -1248,7 +1235,7 @@ BatchGroup batch_group(vmbd_plan* p, int nframes, const float* x, const float* f
   B.st_ncols = g.sf1;
   B.st_out = fbar;
   B.st_scale = inv_scale(g);
-  return B;
+  return ok;
 }
 
 void batch_free(vmbd_batch* b) {
@@ -1282,7 +1269,10 @@ vmbd_batch* vmbd_batch_create(vmbd_plan* const* plans, int32_t n, const int32_t*
       vmbd_fail(VMBD_E_ARG, "vmbd_batch_create: null buffer of plan %d", i);
       return nullptr;
     }
-    host[i] = batch_group(plans[i], nframes[i], x[i], f[i], g[i], y[i], xbar[i], fbar[i], exact);
+    if (!batch_group(host[i], plans[i], nframes[i], x[i], f[i], g[i], y[i], xbar[i], fbar[i], exact)) {
+      vmbd_fail(VMBD_E_ARG, "vmbd_batch_create: plan %d has more row blocks than one launch holds", i);
+      return nullptr;
+    }
   }
   vmbd_batch* b = new vmbd_batch();
   b->device = dev;

@@ -247,8 +247,17 @@ struct Twiddles {
   static constexpr int NB1 = (R1 > 1) ? 16 / R1 : 1;
   static constexpr int C1 = (R1 > 1) ? TwCount<(R1 > 1 ? R1 : 2)>::n : 1;
   static constexpr int C2 = (R2 > 1) ? TwCount<(R2 > 1 ? R2 : 2)>::n : 1;
-  float2 w[NB1 * C1];
-  float2 w3[(R2 > 1) ? 4 * C2 : 1];
+  static constexpr int N2 = NB1 * C1, N3 = (R2 > 1) ? 4 * C2 : 1;
+  float2 w[N2];
+  float2 w3[N3];
+  __device__ __forceinline__ void second(float2 (&o)[N2], int) const {
+#pragma unroll
+    for (int i = 0; i < N2; ++i) o[i] = w[i];
+  }
+  __device__ __forceinline__ void third(float2 (&o)[N3], int) const {
+#pragma unroll
+    for (int i = 0; i < N3; ++i) o[i] = w3[i];
+  }
 };
 
 // twiddle array of an R-point DFT from w = tw[i] (table index i)
@@ -354,15 +363,52 @@ __device__ __forceinline__ void twiddles_init(Twiddles<N>& T, int t, const float
   }
 }
 
+// The same twiddles in LDS, shared by the transforms of a workgroup and read
+// by the pass that uses them: a kernel that keeps the registers for its
+// operands (slot i of thread t at i*TPT + t: consecutive lanes, no conflicts).
+template <int N>
+struct TwiddlesLds {
+  using T = Twiddles<N>;
+  static constexpr int TPT = N / 16;
+  static constexpr int floats2 = TPT * (T::N2 + (T::R2 > 1 ? T::N3 : 0));
+  const float2* p;
+  // fills the table (the caller's barrier follows)
+  static __device__ __forceinline__ void fill(float2* p, const float2* __restrict__ tw) {
+    if ((int)threadIdx.x < TPT) {
+      T r;
+      twiddles_init<N, true>(r, threadIdx.x, tw);
+#pragma unroll
+      for (int i = 0; i < T::N2; ++i) p[i * TPT + threadIdx.x] = r.w[i];
+      if constexpr (T::R2 > 1) {
+#pragma unroll
+        for (int i = 0; i < T::N3; ++i) p[(T::N2 + i) * TPT + threadIdx.x] = r.w3[i];
+      }
+    }
+  }
+  __device__ __forceinline__ void second(float2 (&o)[T::N2], int t) const {
+#pragma unroll
+    for (int i = 0; i < T::N2; ++i) o[i] = p[i * TPT + t];
+  }
+  __device__ __forceinline__ void third(float2 (&o)[T::N3], int t) const {
+#pragma unroll
+    for (int i = 0; i < T::N3; ++i) o[i] = p[(T::N2 + i) * TPT + t];
+  }
+};
+
 // One Stockham pass after the first (NS > 1).  Reads 16 values of the slice,
-// applies 16/R butterflies with their twiddles (w: NB or, on a quarter turn
-// from the first four, 4 arrays of TwCount<R>::n), writes 16 values (or keeps
+// applies 16/R butterflies with their twiddles (from T: NB or, on a quarter
+// turn from the first four, 4 arrays of TwCount<R>::n), writes 16 values (or keeps
 // them in registers when LAST: slot m = b + r*(16/R) holds X[t + TPT*m]).
-template <int N, int R, int NS, int S, bool LAST>
-__device__ __forceinline__ void stockham_pass(float2 (&v)[16], float2* sl, int t, const float2* w) {
+template <int N, int R, int NS, int S, bool LAST, class TWD>
+__device__ __forceinline__ void stockham_pass(float2 (&v)[16], float2* sl, int t, const TWD& T) {
   constexpr int TPT = N / 16;
   constexpr int NB = 16 / R;
   float2 in[16];
+  float2 w[NS > 16 ? Twiddles<N>::N3 : Twiddles<N>::N2];
+  if constexpr (NS > 16)
+    T.third(w, t);
+  else
+    T.second(w, t);
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
     const int j = t + b * TPT;
@@ -404,8 +450,8 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[16], float2* sl, int t
 // not read, and the first pass shrinks to the arithmetic the nonzero inputs
 // need (outputs a caller never reads are removed by the compiler once the
 // call is inlined).
-template <int N, int S, int NZ = 16>
-__device__ __forceinline__ void fft(float2 (&v)[16], float2* sl, int t, const Twiddles<N>& T) {
+template <int N, int S, int NZ = 16, class TWD>
+__device__ __forceinline__ void fft(float2 (&v)[16], float2* sl, int t, const TWD& T) {
   static_assert(N >= 16 && N <= 1024 && (N & (N - 1)) == 0, "N must be a power of two in [16,1024]");
   // pass 0: radix 16, Ns = 1, j = t, no twiddles; output index t*16 + r
   dft16<S, NZ>(v);
@@ -416,10 +462,10 @@ __device__ __forceinline__ void fft(float2 (&v)[16], float2* sl, int t, const Tw
     constexpr int R1 = Plan<N>::R1;
     constexpr int R2 = Plan<N>::R2;
     if constexpr (R2 == 1) {
-      stockham_pass<N, R1, 16, S, true>(v, sl, t, T.w);
+      stockham_pass<N, R1, 16, S, true>(v, sl, t, T);
     } else {
-      stockham_pass<N, R1, 16, S, false>(v, sl, t, T.w);
-      stockham_pass<N, R2, 256, S, true>(v, sl, t, T.w3);
+      stockham_pass<N, R1, 16, S, false>(v, sl, t, T);
+      stockham_pass<N, R2, 256, S, true>(v, sl, t, T);
     }
   }
 }

@@ -41,7 +41,7 @@ struct Geo {
   int ext0, ext1;
   int oc0, oc1;
   int sy0, sy1;
-  FastDiv dPf, dcsf1;  // division by Pf and csf1
+  FastDiv dPf, dcsf1, dNP2, dhop0;  // division by Pf, csf1, its pairs (csf1+1)/2, hop0
 };
 
 // Source of the rows fed to the row transform (chop / pad / window fused).
@@ -69,13 +69,26 @@ struct RowSrc {
   const int* czr;
 };
 
-// Up to four row-transform jobs fused in one launch: blocks [0, blk_end[0])
-// run job 0, [blk_end[0], blk_end[1]) job 1, ...
+// Up to four row-transform jobs in one launch, each over patches of its own
+// (the shared image rows of a patch column beside the PSF rows of every
+// patch).  A job's work units are its blocks of row pairs, one per patch and
+// block; every XCD runs an equal share of each job, slots [u[j-1].send,
+// u[j].send) of its workgroups.  The divisors of the unit number are set up
+// on the host.
 constexpr int ROW_JOBS_MAX = 4;
+struct RowUnits {
+  int P, Pf;   // patches of the launch and of a frame
+  int nb;      // row blocks per patch
+  int n;       // units (P * nb)
+  int send;    // slots per XCD, ceil(n / 8), of this job and the ones before it
+  int TP;      // patches of a tile: one XCD's share
+  int nfull, Tl;  // tiles of TP patches, patches of the last, shorter one
+  FastDiv dTile, dTP, dTl, dPf;  // division by TP*nb, TP, Tl, Pf
+};
 struct RowJobs {
   RowSrc s[ROW_JOBS_MAX];
   float2* out[ROW_JOBS_MAX];
-  int blk_end[ROW_JOBS_MAX];
+  RowUnits u[ROW_JOBS_MAX];
   int n;
 };
 
@@ -199,22 +212,14 @@ struct DivParams {
 };
 
 // Launchers (ola_kernels.hip).  Return hipError_t of the launch.
-// Jobs of different patch counts in one launch (the shared image rows of a
-// patch column beside the PSF rows of every patch): job j has P[j] units of
-// its own geometry's patches (Pf[j] per frame); at most two jobs.
-struct RowJobGeo {
-  int P[2], Pf[2];
-  int nb[2];    // row blocks per patch
-  int uend[2];  // cumulative work units, P[j] * nb[j]
-};
-hipError_t launch_rows_r2c_geo(const Geo& g, const RowSrc* s, float2* const* out, const int* P, const int* Pf, int n,
-                               const float2* tw, hipStream_t st, const char* name);
-// name: the launch's label in the library's kernel timing (default rows_r2c)
-hipError_t launch_rows_r2c(const Geo& g, const RowSrc& s, float2* out, const float2* tw, hipStream_t st,
-                           const char* name = nullptr);
-// several row-transform jobs in one launch (n <= ROW_JOBS_MAX)
-hipError_t launch_rows_r2c_multi(const Geo& g, const RowSrc* s, float2* const* out, int n, const float2* tw,
-                                 hipStream_t st);
+// Appends the rows of s over g's patches to a launch's jobs (nothing when it
+// has no rows); false when the launch's units would not fit an int.
+bool row_job(RowJobs& jobs, const Geo& g, const RowSrc& s, float2* out);
+// workgroups of a launch (a multiple of the XCDs)
+int row_blocks(const RowJobs& jobs);
+// One launch of the jobs' row transforms (tile width g.Tw, hops and patch
+// columns of g).  name: the launch's label in the library's kernel timing.
+hipError_t launch_rows_r2c(const Geo& g, const RowJobs& jobs, const float2* tw, hipStream_t st, const char* name);
 // wgc: threads per column-pass workgroup (128 or 256; 0 = 256): the column
 // strip of a workgroup is wgc / (Th/16) columns wide
 hipError_t launch_cols(const Geo& g, int op, const ColIn& a, const ColIn& b, const ColIn& c, const ColOut& o1,
@@ -239,9 +244,8 @@ hipError_t launch_rows_c2r_stack(const Geo& g, const float2* src, int srow, floa
 // for one group, built once when the batch binds its buffers.
 constexpr int BATCH_MAX_GROUPS = 16;
 struct BatchGroup {
-  Geo g;     // call geometry (P = frames * Pf)
-  Geo gres;  // geometry of the shared residual rows
-  Geo gx;    // geometry of the image rows shared per patch column (rows_x.n > 0)
+  Geo g;  // call geometry (P = frames * Pf)
+  // rows_x: the image rows where they are shared per patch column
   RowJobs rows_fwd, rows_res, rows_x;
   ColIn cf_a, cf_b;
   ColOut cf_o;

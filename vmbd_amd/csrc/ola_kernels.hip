@@ -28,6 +28,7 @@
 // the footprint at 35-40 KB and allows four workgroups per CU.
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "col_device.h"
 #include "fft_core.h"
@@ -49,11 +50,11 @@ struct RowsLds {
   static constexpr int v = cmax<TPW * FftLds<TW>::floats2, 2 * TPW * (TW / 2 + 1)>::v;
 };
 
-// One workgroup of the row pass: row pairs [q0, q0 + TPW) of patch pu of
-// source s into out (sm: RowsLds<TW>::v float2 of LDS).
+// One workgroup of the row pass: row pairs [q0, q0 + TPW) of patch p (patch
+// k of frame fr) of source s into out (sm: RowsLds<TW>::v float2 of LDS).
 template <int TW>
-__device__ __forceinline__ void rows_r2c_body(Geo g, RowSrc s, float2* __restrict__ out, int pu, int q0, float2* sm,
-                                              const float2* __restrict__ tw) {
+__device__ __forceinline__ void rows_r2c_body(Geo g, RowSrc s, float2* __restrict__ out, int p, int fr, int k, int q0,
+                                              float2* sm, const float2* __restrict__ tw) {
   constexpr int TPT = TW / 16;
   constexpr int TPW = WG / TPT;
   constexpr int NBN = TW / 2 + 1;
@@ -66,11 +67,8 @@ __device__ __forceinline__ void rows_r2c_body(Geo g, RowSrc s, float2* __restric
   const int NQ = (nr + 1) >> 1;
   const int q = q0 + tr;
   const bool active = q < NQ;
-  const int p = pu;
   const int r0 = s.rlo + 2 * q;
-  const int fr = p / g.Pf;
-  const int k = p - fr * g.Pf;
-  const int m = k / g.csf1;
+  const int m = div_by(k, g.dcsf1);
   const int n = k - m * g.csf1;
   const int o0 = (s.origin ? m * g.hop0 : 0) - s.sh0;
   const int o1 = (s.origin ? n * g.hop1 : 0) - s.sh1;
@@ -214,156 +212,90 @@ __device__ __forceinline__ void rows_r2c_body(Geo g, RowSrc s, float2* __restric
     }
 }
 
-// 1-D grid over work units (patch, row block), row blocks of all jobs
-// job-major.  Workgroup ids are dealt round-robin to the NXCD XCDs; XCD j
-// runs the contiguous units [start_j, start_j + count_j).  Units are ordered
-// in tiles of TP = ceil(P / NXCD) consecutive patches (one XCD's share),
-// row-block-major inside a tile, so neighbouring patches, which read the
-// same pixels, run on one XCD at the same time and share its L2.  The map
-// id -> (patch, row block) is a bijection whatever the hardware placement.
-// blk: the workgroup's id among the launch's g.P * (row blocks) (its XCD is
-// blk mod NXCD).  Returns the patch, the job and its first row pair.
+// 1-D grid over the jobs' work units (patch, row block).  Workgroup ids are
+// dealt round-robin to the NXCD XCDs; of every job, XCD j runs the contiguous
+// units [start_j, start_j + count_j) (equal shares: with the jobs' units in
+// one sequence, some XCDs had image rows only and others PSF rows only).  A
+// job's units are ordered in tiles of TP = ceil(P / NXCD) consecutive
+// patches, row-block-major inside a tile, so neighbouring patches, which read
+// the same pixels, run on one XCD at the same time and share its L2.  The map
+// id -> (job, patch, row block) is a bijection whatever the hardware
+// placement, apart from ids past an XCD's share, which have no unit.
 template <int TW>
-__device__ __forceinline__ void rows_unit(const Geo& g, const RowJobs& jobs, int blk, int& pu, int& ji, int& q0) {
+__device__ __forceinline__ void rows_r2c_unit(const Geo& g, const RowJobs& jobs, int blk, float2* sm,
+                                              const float2* __restrict__ tw) {
   constexpr int TPW = WG / (TW / 16);
-  const int nblk = jobs.blk_end[jobs.n - 1];
-  const int total = g.P * nblk;
   const int xcd = blk % NXCD;
-  const int u = xcd * (total / NXCD) + min(xcd, total % NXCD) + blk / NXCD;
-  const int TP = (g.P + NXCD - 1) / NXCD;
-  const int tile = u / (TP * nblk);
-  const int ur = u - tile * TP * nblk;
-  const int Tt = min(TP, g.P - tile * TP);
-  const int by = ur / Tt;
-  pu = tile * TP + (ur - by * Tt);
-  ji = 0;
-  int blk0 = 0;
+  int ji = 0, slot = blk / NXCD, s0 = 0;
 #pragma unroll
   for (int jj = 0; jj < ROW_JOBS_MAX - 1; ++jj)
-    if (jobs.n > jj + 1 && by >= jobs.blk_end[jj]) {
+    if (jobs.n > jj + 1 && slot >= jobs.u[jj].send) {
       ji = jj + 1;
-      blk0 = jobs.blk_end[jj];
+      s0 = jobs.u[jj].send;
     }
-  q0 = (by - blk0) * TPW;
+  const RowUnits U = jobs.u[ji];
+  slot -= s0;
+  if (slot >= U.n / NXCD + (xcd < U.n % NXCD)) return;
+  const int u = xcd * (U.n / NXCD) + min(xcd, U.n % NXCD) + slot;
+  const int tile = div_by(u, U.dTile);
+  const int ur = u - tile * (U.TP * U.nb);
+  const int by = tile < U.nfull ? div_by(ur, U.dTP) : div_by(ur, U.dTl);
+  const int p = tile * U.TP + (ur - by * (tile < U.nfull ? U.TP : U.Tl));
+  const int fr = div_by(p, U.dPf);
+  rows_r2c_body<TW>(g, jobs.s[ji], jobs.out[ji], p, fr, p - fr * U.Pf, by * TPW, sm, tw);
 }
 
 template <int TW>
 __global__ __launch_bounds__(WG) void k_rows_r2c(Geo g, RowJobs jobs, const float2* __restrict__ tw) {
   __shared__ float2 sm[RowsLds<TW>::v];
-
-  int pu, ji, q0;
-  rows_unit<TW>(g, jobs, (int)blockIdx.x, pu, ji, q0);
-  const RowSrc s = jobs.s[ji];
-  rows_r2c_body<TW>(g, s, jobs.out[ji], pu, q0, sm, tw);
+  rows_r2c_unit<TW>(g, jobs, (int)blockIdx.x, sm, tw);
 }
 
-// Row jobs with a patch count of their own: the units of job 0, then of
-// job 1, each in the tile order of rows_unit over its own patches; the XCD
-// of workgroup b runs a contiguous range of them.
-template <int TW>
-__global__ __launch_bounds__(WG) void k_rows_r2c_geo(Geo g, RowJobs jobs, RowJobGeo jg,
-                                                     const float2* __restrict__ tw) {
-  __shared__ float2 sm[RowsLds<TW>::v];
-  constexpr int TPW = WG / (TW / 16);
-  const int blk = (int)blockIdx.x;
-  const int total = jobs.n > 1 ? jg.uend[1] : jg.uend[0];
-  const int xcd = blk % NXCD;
-  const int u = xcd * (total / NXCD) + min(xcd, total % NXCD) + blk / NXCD;
-  const bool j1 = jobs.n > 1 && u >= jg.uend[0];
-  const int ul = j1 ? u - jg.uend[0] : u;
-  const int P = j1 ? jg.P[1] : jg.P[0];
-  const int nb = j1 ? jg.nb[1] : jg.nb[0];
-  const int TP = (P + NXCD - 1) / NXCD;
-  const int tile = ul / (TP * nb);
-  const int ur = ul - tile * TP * nb;
-  const int Tt = min(TP, P - tile * TP);
-  const int by = ur / Tt;
-  const int pu = tile * TP + (ur - by * Tt);
-  Geo gj = g;
-  gj.P = P;
-  gj.Pf = j1 ? jg.Pf[1] : jg.Pf[0];
-  rows_r2c_body<TW>(gj, j1 ? jobs.s[1] : jobs.s[0], j1 ? jobs.out[1] : jobs.out[0], pu, by * TPW, sm, tw);
+bool row_job(RowJobs& jobs, const Geo& g, const RowSrc& s, float2* out) {
+  const int TPW = WG / (g.Tw / 16);
+  const int nb = ((s.rhi - s.rlo + 1) / 2 + TPW - 1) / TPW;
+  if (nb <= 0 || g.P <= 0) return true;
+  const long long n = (long long)g.P * nb;
+  const long long send = (jobs.n ? jobs.u[jobs.n - 1].send : 0) + (n + NXCD - 1) / NXCD;
+  if (jobs.n == ROW_JOBS_MAX || send * NXCD > INT_MAX) return false;
+  RowUnits& u = jobs.u[jobs.n];
+  jobs.s[jobs.n] = s;
+  jobs.out[jobs.n++] = out;
+  u.P = g.P;
+  u.Pf = g.Pf;
+  u.nb = nb;
+  u.n = (int)n;
+  u.send = (int)send;
+  u.TP = (g.P + NXCD - 1) / NXCD;
+  u.nfull = g.P / u.TP;
+  u.Tl = std::max(1, g.P - u.nfull * u.TP);
+  u.dTile = fast_div(u.TP * nb);
+  u.dTP = fast_div(u.TP);
+  u.dTl = fast_div(u.Tl);
+  u.dPf = fast_div(g.Pf);
+  return true;
 }
 
+int row_blocks(const RowJobs& jobs) { return jobs.n ? jobs.u[jobs.n - 1].send * NXCD : 0; }
+
 template <int TW>
-static hipError_t rows_r2c_geo_t(const Geo& g, const RowSrc* s, float2* const* out, const int* P, const int* Pf, int n,
-                                 const float2* tw, hipStream_t st, const char* name) {
-  constexpr int TPW = WG / (TW / 16);
-  RowJobs jobs{};
-  RowJobGeo jg{};
-  jobs.n = n;
-  long long units = 0;
-  for (int i = 0; i < n; ++i) {
-    jobs.s[i] = s[i];
-    jobs.out[i] = out[i];
-    jg.P[i] = P[i];
-    jg.Pf[i] = Pf[i];
-    jg.nb[i] = ((s[i].rhi - s[i].rlo + 1) / 2 + TPW - 1) / TPW;
-    units += (long long)P[i] * jg.nb[i];
-    if (jg.nb[i] <= 0 || P[i] <= 0 || units > INT_MAX) return hipErrorInvalidValue;
-    jg.uend[i] = (int)units;
-  }
-  ProfScope ps(name ? name : "rows_r2c_multi", st);
-  hipLaunchKernelGGL(k_rows_r2c_geo<TW>, dim3((unsigned)units), dim3(WG), 0, st, g, jobs, jg, tw);
+static hipError_t rows_r2c_t(const Geo& g, const RowJobs& jobs, const float2* tw, hipStream_t st, const char* name) {
+  ProfScope ps(name, st);
+  hipLaunchKernelGGL(k_rows_r2c<TW>, dim3((unsigned)row_blocks(jobs)), dim3(WG), 0, st, g, jobs, tw);
   return hipGetLastError();
 }
 
-hipError_t launch_rows_r2c_geo(const Geo& g, const RowSrc* s, float2* const* out, const int* P, const int* Pf, int n,
-                               const float2* tw, hipStream_t st, const char* name) {
-  if (n < 1 || n > 2) return hipErrorInvalidValue;
+hipError_t launch_rows_r2c(const Geo& g, const RowJobs& jobs, const float2* tw, hipStream_t st, const char* name) {
+  if (jobs.n == 0) return hipSuccess;
   switch (g.Tw) {
-    case 16: return rows_r2c_geo_t<16>(g, s, out, P, Pf, n, tw, st, name);
-    case 32: return rows_r2c_geo_t<32>(g, s, out, P, Pf, n, tw, st, name);
-    case 64: return rows_r2c_geo_t<64>(g, s, out, P, Pf, n, tw, st, name);
-    case 128: return rows_r2c_geo_t<128>(g, s, out, P, Pf, n, tw, st, name);
-    case 256: return rows_r2c_geo_t<256>(g, s, out, P, Pf, n, tw, st, name);
-    case 512: return rows_r2c_geo_t<512>(g, s, out, P, Pf, n, tw, st, name);
+    case 16: return rows_r2c_t<16>(g, jobs, tw, st, name);
+    case 32: return rows_r2c_t<32>(g, jobs, tw, st, name);
+    case 64: return rows_r2c_t<64>(g, jobs, tw, st, name);
+    case 128: return rows_r2c_t<128>(g, jobs, tw, st, name);
+    case 256: return rows_r2c_t<256>(g, jobs, tw, st, name);
+    case 512: return rows_r2c_t<512>(g, jobs, tw, st, name);
     default: return hipErrorInvalidValue;
   }
-}
-
-template <int TW>
-static hipError_t rows_r2c_t(const Geo& g, const RowSrc* s, float2* const* out, int n, const float2* tw,
-                             hipStream_t st, const char* name) {
-  constexpr int TPW = WG / (TW / 16);
-  RowJobs jobs{};
-  jobs.n = n;
-  int blocks = 0;
-  for (int i = 0; i < n; ++i) {
-    jobs.s[i] = s[i];
-    jobs.out[i] = out[i];
-    const int nq = (s[i].rhi - s[i].rlo + 1) / 2;
-    blocks += (nq + TPW - 1) / TPW;
-    jobs.blk_end[i] = blocks;
-  }
-  if (blocks <= 0 || g.P <= 0) return hipSuccess;
-  ProfScope ps(name ? name : n == 1 ? "rows_r2c" : "rows_r2c_multi", st);
-  hipLaunchKernelGGL(k_rows_r2c<TW>, dim3((unsigned)(g.P * blocks)), dim3(WG), 0, st, g, jobs, tw);
-  return hipGetLastError();
-}
-
-static hipError_t rows_r2c_any(const Geo& g, const RowSrc* s, float2* const* out, int n, const float2* tw,
-                               hipStream_t st, const char* name) {
-  if (n < 1 || n > ROW_JOBS_MAX) return hipErrorInvalidValue;
-  switch (g.Tw) {
-    case 16: return rows_r2c_t<16>(g, s, out, n, tw, st, name);
-    case 32: return rows_r2c_t<32>(g, s, out, n, tw, st, name);
-    case 64: return rows_r2c_t<64>(g, s, out, n, tw, st, name);
-    case 128: return rows_r2c_t<128>(g, s, out, n, tw, st, name);
-    case 256: return rows_r2c_t<256>(g, s, out, n, tw, st, name);
-    case 512: return rows_r2c_t<512>(g, s, out, n, tw, st, name);
-    default: return hipErrorInvalidValue;
-  }
-}
-
-hipError_t launch_rows_r2c_multi(const Geo& g, const RowSrc* s, float2* const* out, int n, const float2* tw,
-                                 hipStream_t st) {
-  return rows_r2c_any(g, s, out, n, tw, st, nullptr);
-}
-
-hipError_t launch_rows_r2c(const Geo& g, const RowSrc& s, float2* out, const float2* tw, hipStream_t st,
-                           const char* name) {
-  return rows_r2c_any(g, &s, &out, 1, tw, st, name);
 }
 
 // ----------------------------------------------------------------------------
@@ -375,68 +307,66 @@ hipError_t launch_rows_r2c(const Geo& g, const RowSrc& s, float2* out, const flo
 // lanes of wavefront 0 of strip 0) carries two real row bins, 0 and TW/2: its
 // transforms are P = D + i N of two Hermitian spectra D, N, taken apart with
 // P(-k) (D = (P(k) + conj P(-k)) / 2, N = (P(k) - conj P(-k)) / 2i),
-// multiplied bin by bin and put together as D' + i N'.  Its operands go to
-// LDS (its own slice and the next column's, which belongs to the same
-// wavefront and is idle between the transforms); after the plain product of
-// every column, all 64 lanes of that wavefront form the packed product in
-// place, each taking pairs of frequencies (k, TH-k), and its lanes read their
-// slots back (SPREAD; otherwise the column's own lanes form it, 16 slots each).  Written
-// as a macro: the same code behind a function boundary takes 32 more VGPRs
-// (four wavefronts per SIMD become three).
+// multiplied bin by bin and put together as D' + i N'.  At k = 0 all four are
+// real, so the lane that holds it multiplies the parts.  For the other k the
+// operands go to LDS (the column's own slice and the next column's, which
+// belongs to the same wavefront and is idle between the transforms); after
+// the plain product of every column, all 64 lanes of that wavefront form the
+// packed product in place, each taking pairs of frequencies (k, TH-k), and
+// its lanes read their slots back.  This path is on the critical path of a
+// small launch (every workgroup of strip 0 waits for it), so up to two pairs
+// per lane are read together: 2300 -> 900 cycles of a 21000-cycle workgroup
+// (one 1024^2 frame) against one pair at a time over TH/2 + 1 frequencies.
+// Written as a macro: the same code behind a function boundary takes 32 more
+// VGPRs (four wavefronts per SIMD become three).
 #define VMBD_COL_PRODUCT(CONJ, A, B)                                                                \
   do {                                                                                              \
-    if (packed) {                                                                                   \
-      _Pragma("unroll") for (int m = 0; m < 16; ++m) {                                              \
-        sm[lds_pad(t + TPT * m)] = A[m];                                                            \
-        sm[SL + lds_pad(t + TPT * m)] = B[m];                                                       \
+    float2 z0_;                                                                                     \
+    if (pwave) {                                                                                    \
+      z0_ = make_float2(A[0].x * B[0].x, A[0].y * B[0].y);                                          \
+      if (packed) {                                                                                 \
+        _Pragma("unroll") for (int m = 0; m < 16; ++m) {                                            \
+          sm[lds_pad(t + TPT * m)] = A[m];                                                          \
+          sm[SL + lds_pad(t + TPT * m)] = B[m];                                                     \
+        }                                                                                           \
       }                                                                                             \
     }                                                                                               \
     _Pragma("unroll") for (int m = 0; m < 16; ++m) B[m] =                                           \
         (CONJ) ? cmulc(A[m], B[m]) : cmul(A[m], B[m]);                                              \
-    if (SPREAD && pwave) {                                                                          \
-      /* frequencies k <= TH/2 with their mirror TH-k: one lane reads both */                      \
-      /* pairs of both operands and writes both products in place         */                       \
-      constexpr int NP_ = TH / 128 + 1;                                                             \
+    if (pwave) {                                                                                    \
+      /* frequencies 1 <= k <= TH/2 with their mirror TH-k: one lane reads */                      \
+      /* both pairs of both operands and writes both products in place     */                      \
+      constexpr int U_ = TH == 256 ? 2 : 1; /* pairs in flight per lane */                          \
       const int lane_ = threadIdx.x & 63;                                                           \
       wave_sync();                                                                                  \
-      _Pragma("unroll 1") for (int j = 0; j < NP_; ++j) {                                           \
-        const int k_ = lane_ + 64 * j;                                                              \
-        if (k_ <= TH / 2) {                                                                         \
-          const int kr_ = (TH - k_) & (TH - 1);                                                     \
-          const float2 a_ = sm[lds_pad(k_)], ar_ = sm[lds_pad(kr_)];                                \
-          const float2 b_ = sm[SL + lds_pad(k_)], br_ = sm[SL + lds_pad(kr_)];                      \
-          const float2 ad_ = make_float2(0.5f * (a_.x + ar_.x), 0.5f * (a_.y - ar_.y));             \
-          const float2 an_ = make_float2(0.5f * (a_.y + ar_.y), 0.5f * (ar_.x - a_.x));             \
-          const float2 bd_ = make_float2(0.5f * (b_.x + br_.x), 0.5f * (b_.y - br_.y));             \
-          const float2 bn_ = make_float2(0.5f * (b_.y + br_.y), 0.5f * (br_.x - b_.x));             \
+      _Pragma("unroll 1") for (int j = 0; j < TH / 2; j += 64 * U_) {                               \
+        float2 a_[U_], ar_[U_], b_[U_], br_[U_];                                                    \
+        _Pragma("unroll") for (int q = 0; q < U_; ++q) {                                            \
+          const int k_ = 1 + ((lane_ + j + 64 * q) & (TH / 2 - 1)), kr_ = TH - k_;                  \
+          a_[q] = sm[lds_pad(k_)];                                                                  \
+          ar_[q] = sm[lds_pad(kr_)];                                                                \
+          b_[q] = sm[SL + lds_pad(k_)];                                                             \
+          br_[q] = sm[SL + lds_pad(kr_)];                                                           \
+        }                                                                                           \
+        wave_sync(); /* below 128 points several lanes form the same pair */                       \
+        _Pragma("unroll") for (int q = 0; q < U_; ++q) {                                            \
+          const int k_ = 1 + ((lane_ + j + 64 * q) & (TH / 2 - 1)), kr_ = TH - k_;                  \
+          const float2 ad_ = make_float2(0.5f * (a_[q].x + ar_[q].x), 0.5f * (a_[q].y - ar_[q].y)); \
+          const float2 an_ = make_float2(0.5f * (a_[q].y + ar_[q].y), 0.5f * (ar_[q].x - a_[q].x)); \
+          const float2 bd_ = make_float2(0.5f * (b_[q].x + br_[q].x), 0.5f * (b_[q].y - br_[q].y)); \
+          const float2 bn_ = make_float2(0.5f * (b_[q].y + br_[q].y), 0.5f * (br_[q].x - b_[q].x)); \
           const float2 pd_ = (CONJ) ? cmulc(ad_, bd_) : cmul(ad_, bd_);                            \
           const float2 pn_ = (CONJ) ? cmulc(an_, bn_) : cmul(an_, bn_);                            \
           /* at -k: D(-k) = conj D(k), N(-k) = conj N(k) */                                         \
           const float2 pdr_ = cconj(pd_), pnr_ = cconj(pn_);                                        \
+          sm[lds_pad(kr_)] = make_float2(pdr_.x - pnr_.y, pdr_.y + pnr_.x);                         \
           sm[lds_pad(k_)] = make_float2(pd_.x - pn_.y, pd_.y + pn_.x);                              \
-          if (kr_ != k_) sm[lds_pad(kr_)] = make_float2(pdr_.x - pnr_.y, pdr_.y + pnr_.x);          \
         }                                                                                           \
       }                                                                                             \
       wave_sync();                                                                                  \
       if (packed) {                                                                                 \
         _Pragma("unroll") for (int m = 0; m < 16; ++m) B[m] = sm[lds_pad(t + TPT * m)];             \
-      }                                                                                             \
-      wave_sync(); /* the slices are written next by the inverse transform */                      \
-    }                                                                                               \
-    if (!SPREAD && packed) {                                                                        \
-      wave_sync();                                                                                  \
-      _Pragma("unroll") for (int m = 0; m < 16; ++m) {                                              \
-        const int k_ = t + TPT * m;                                                                 \
-        const int kr_ = (TH - k_) & (TH - 1);                                                       \
-        const float2 a_ = sm[lds_pad(k_)], ar_ = sm[lds_pad(kr_)];                                  \
-        const float2 b_ = sm[SL + lds_pad(k_)], br_ = sm[SL + lds_pad(kr_)];                        \
-        const float2 ad_ = make_float2(0.5f * (a_.x + ar_.x), 0.5f * (a_.y - ar_.y));               \
-        const float2 an_ = make_float2(0.5f * (a_.y + ar_.y), 0.5f * (ar_.x - a_.x));               \
-        const float2 bd_ = make_float2(0.5f * (b_.x + br_.x), 0.5f * (b_.y - br_.y));               \
-        const float2 bn_ = make_float2(0.5f * (b_.y + br_.y), 0.5f * (br_.x - b_.x));               \
-        const float2 pd_ = (CONJ) ? cmulc(ad_, bd_) : cmul(ad_, bd_);                              \
-        const float2 pn_ = (CONJ) ? cmulc(an_, bn_) : cmul(an_, bn_);                              \
-        B[m] = make_float2(pd_.x - pn_.y, pd_.y + pn_.x);                                           \
+        if (t == 0) B[0] = z0_;                                                                     \
       }                                                                                             \
       wave_sync(); /* the slices are written next by the inverse transform */                      \
     }                                                                                               \
@@ -447,7 +377,16 @@ hipError_t launch_rows_r2c(const Geo& g, const RowSrc& s, float2* out, const flo
 template <int TH, int OP, int WGC = WG>
 struct ColsLds {
   static constexpr int CS = WGC / (TH / 16);
-  static constexpr int v = (OP == COL_SPEC) ? CS * FftLds<TH>::floats2 : cmax<CS * FftLds<TH>::floats2, TH * (CS + 1)>::v;
+  static constexpr int work =
+      (OP == COL_SPEC) ? CS * FftLds<TH>::floats2 : cmax<CS * FftLds<TH>::floats2, TH * (CS + 1)>::v;
+  // the 512-point two-adjoint pass keeps its first operand's spectrum through
+  // both products and the twiddles of three passes: those live in LDS, behind
+  // the work area (in registers 25 of them spilled per lane; a 768 x 1024
+  // group of 6 x 12 patches: 322 us with the table, 376 without).  At 256
+  // points 6 registers spill and the table costs more than that (one 1024^2
+  // frame 21.0 us with it, 20.2 without).
+  static constexpr bool twl = OP == COL_ADJ2 && TH >= 512;
+  static constexpr int v = work + (twl ? TwiddlesLds<TH>::floats2 : 0);
 };
 
 // One workgroup of WGC threads of the column pass: strip `strip` of patch pk of frame pfr
@@ -476,11 +415,6 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
   // wavefront 0 of strip 0 holds the packed column (lanes 0..TPT-1) and
   // forms its product (uniform per wavefront)
   const bool pwave = strip == 0 && threadIdx.x < 64;
-  // the first product spreads the packed column over the wavefront; the
-  // two-adjoint pass forms its second one on the column's own lanes (spread
-  // twice, its registers spill)
-  constexpr bool SPREAD1 = true;
-  constexpr bool SPREAD2 = false;
   // a wavefront whose columns all lie past the last bin skips its transforms
   const bool wact = strip * CS + (int)(threadIdx.x >> 6) * (64 / TPT) < NB - 1;
   // group and row offset of this patch in shared row transforms
@@ -494,8 +428,12 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
   constexpr bool XC = XS && OP == COL_ADJ2;
   float2* sl = sm + cc * SL;
 
-  Twiddles<TH> T;
-  twiddles_init<TH, true>(T, t, tw);
+  using Lds = ColsLds<TH, OP, WGC>;
+  std::conditional_t<Lds::twl, TwiddlesLds<TH>, Twiddles<TH>> T;
+  if constexpr (Lds::twl)
+    T.p = sm + Lds::work;
+  else
+    twiddles_init<TH, true>(T, t, tw);
 
   float2 A[16];
   // operands of at most 3*TPT stored rows (PSF rows) take a transform whose
@@ -512,6 +450,10 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
     if (wact) fft<TH, -1, 12>(A, sl, t, T);
   } else {
     col_load<TH, 16, XA>(A, a, p, c, NB, t, grp, row0, cx);
+    if constexpr (Lds::twl) {  // (in flight with the operand; this pass takes no other path)
+      TwiddlesLds<TH>::fill(sm + Lds::work, tw);
+      __syncthreads();
+    }
     if (wact) fft<TH, -1>(A, sl, t, T);
   }
   if constexpr (OP == COL_SPEC) {
@@ -537,10 +479,7 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
       col_load<TH, 16, XB>(B, b, p, c, NB, t, grp, row0, cx);
       if (wact) fft<TH, -1>(B, sl, t, T);
     }
-    {
-      constexpr bool SPREAD = SPREAD1;
-      VMBD_COL_PRODUCT(OP != COL_FWD, A, B);
-    }
+    VMBD_COL_PRODUCT(OP != COL_FWD, A, B);
     if (OP == COL_ADJ1 && o1.nrows <= 3 * TPT) {
       if (wact) fft<TH, +1>(B, sl, t, T);
       col_store_rows<TH, CS, true, 3, WGC>(B, sm, o1, p, strip, NB, g.NBP, cc, t);
@@ -556,10 +495,7 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
         col_load<TH, 16, XC>(B, c3, p, c, NB, t, grp, row0, cx);
         if (wact) fft<TH, -1>(B, sl, t, T);
       }
-      {
-        constexpr bool SPREAD = SPREAD2;
-        VMBD_COL_PRODUCT(true, A, B);
-      }
+      VMBD_COL_PRODUCT(true, A, B);
       if (wact) fft<TH, +1>(B, sl, t, T);
       if (PRUNE && o2.nrows <= 3 * TPT)
         col_store_rows<TH, CS, true, 3, WGC>(B, sm, o2, p, strip, NB, g.NBP, cc, t);
@@ -671,20 +607,27 @@ struct C2r {
 // zeros, so every lane issues the same loads without a per-lane test.
 __device__ const float4 c2r_zero_bins[512 / 4] = {};
 
-// global loads of both rows' chunks (all issued before any is used)
+// global loads of both rows' chunks (all issued before any is used).  The
+// pointers are kept in the global address space: selected between a buffer
+// and the zero row they would be generic, and generic loads count as LDS
+// operations too, so that every LDS wait would wait for them.
+typedef float float4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+typedef const __attribute__((address_space(1))) float4_a8* gchunk_t;
 template <int TW>
 __device__ __forceinline__ void c2r_fetch(float4 (&A)[4], float4 (&B)[4], const float2* ra, const float2* rb,
                                           bool hasa, bool hasb, int t) {
   static_assert(C2r<TW>::NCH <= 512 / 4, "zero row shorter than a row's chunks");
-  const float2* pa = hasa ? ra : (const float2*)c2r_zero_bins;
-  const float2* pb = hasb ? rb : (const float2*)c2r_zero_bins;
+  const gchunk_t zero = (gchunk_t)c2r_zero_bins;
+  const gchunk_t pa = hasa ? (gchunk_t)ra : zero;
+  const gchunk_t pb = hasb ? (gchunk_t)rb : zero;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int k = t + C2r<TW>::TPT * i;
     A[i] = B[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (k < C2r<TW>::NCH) {
-      __builtin_memcpy(&A[i], pa + 2 * k, 16);
-      __builtin_memcpy(&B[i], pb + 2 * k, 16);
+      const float4_a8 a = pa[k], b = pb[k];
+      A[i] = make_float4(a.x, a.y, a.z, a.w);
+      B[i] = make_float4(b.x, b.y, b.z, b.w);
     }
   }
 }
@@ -1042,6 +985,26 @@ __host__ __device__ inline int ola_sum_wcol_offset_floats(const Geo& g, const Ol
   return ((fl > rb ? fl : rb) + 3) & ~3;
 }
 
+// Operands of the final store of output columns j0 + e*WG of row i: the fused
+// solver terms, and (WGT) the column normalisers of the row's type (zr: every
+// covering window of the row is at the floor).
+struct OlaEpi {
+  float sub[4], mul[4], axz[4], cw[4];
+};
+template <bool WGT>
+__device__ __forceinline__ void ola_epi_load(OlaEpi& E, const OlaDst& d, int i, int fr, int j0, bool zr) {
+  const size_t orow = ((size_t)fr * d.O0 + i) * d.O1;
+  const float* cw = WGT ? d.colw + (zr ? d.O1 : 0) : nullptr;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int j = min(j0 + e * WG, d.O1 - 1);
+    if (d.sub) E.sub[e] = d.sub[orow + j];
+    if (d.mul) E.mul[e] = d.mul[orow + j];
+    if (d.axz) E.axz[e] = d.axz[orow + j];
+    if constexpr (WGT) E.cw[e] = cw[j];
+  }
+}
+
 template <int TW, bool WGT>
 __device__ __forceinline__ void c2r_sum_body(Geo g, OlaDst d, int i0, int fr, float2* dyn,
                                              const float2* __restrict__ tw) {
@@ -1054,7 +1017,7 @@ __device__ __forceinline__ void c2r_sum_body(Geo g, OlaDst d, int i0, int fr, fl
   float* rowbuf = (float*)dyn;  // class rows alias the FFT slices
   const int tr = threadIdx.x / TPT;
   const int t = threadIdx.x - tr * TPT;
-  const int ri = tr / NP2;
+  const int ri = div_by(tr, g.dNP2);
   const int jp = tr - ri * NP2;
   const int i = i0 + ri;
   const bool act = ri < R && i < d.O0;
@@ -1062,9 +1025,9 @@ __device__ __forceinline__ void c2r_sum_body(Geo g, OlaDst d, int i0, int fr, fl
   // covering patch rows m: m*hop0 <= u < m*hop0 + ext0
   int mlo = 0, mhi = -1;
   if (act && u >= 0) {
-    mhi = min(g.csf0 - 1, u / g.hop0);
+    mhi = min(g.csf0 - 1, div_by(u, g.dhop0));
     const int lo = u - d.ext0 + 1;
-    mlo = lo <= 0 ? 0 : (lo + g.hop0 - 1) / g.hop0;
+    mlo = lo <= 0 ? 0 : div_by(lo + g.hop0 - 1, g.dhop0);
   }
   const int na = 2 * jp, nb = na + 1;
   const bool hasb = nb < g.csf1;
@@ -1075,14 +1038,12 @@ __device__ __forceinline__ void c2r_sum_body(Geo g, OlaDst d, int i0, int fr, fl
   const int MW = ola_win_mw(g);
   float* wcs = (float*)dyn + ola_sum_wcol_offset_floats(g, d);
   if constexpr (WGT) {
-    for (int e = threadIdx.x; e < TPT * MW; e += WG) {
-      const int tt = e / MW;
-      const int c = tt + TPT * (e - tt * MW);
-      wcs[e] = c < g.sw1 ? d.wcol[c] : 0.f;
-    }
+    for (int c = threadIdx.x; c < TPT * MW; c += WG)
+      wcs[(c % TPT) * MW + c / TPT] = c < g.sw1 ? d.wcol[c] : 0.f;
   }
   // unit weights on a row whose covering windows are all at the floor
   const bool zr = WGT && act && d.zrow[i];
+  const bool zr0 = WGT && d.zrow[i0];  // (the first row, uniform)
   // a wavefront whose transforms all lie past the workgroup's rows skips them
   const int trw = (int)(threadIdx.x >> 6) * (64 / TPT);
   const bool wact = trw < R * NP2 && i0 + trw / NP2 < d.O0;
@@ -1103,7 +1064,9 @@ __device__ __forceinline__ void c2r_sum_body(Geo g, OlaDst d, int i0, int fr, fl
       const float2* ra = ok ? d.src + ((size_t)(kf + m * g.csf1 + na) * d.srow + r) * g.NBP : d.src;
       c2r_fetch<TW>(a, b, ra, ra + (size_t)d.srow * g.NBP, ok, ok && hasb, t);
       nok += ok;
-      return ok ? ((WGT && !zr) ? d.wrow[r] : 1.f) : 0.f;
+      // (the factor is loaded whatever the row's type, so that no load waits for it)
+      const float w = WGT ? d.wrow[ok ? r : 0] : 1.f;
+      return ok ? ((WGT && !zr) ? w : 1.f) : 0.f;
     };
     auto add = [&](float4(&A)[4], float4(&B)[4], const float4(&a)[4], const float4(&b)[4], float w) {
 #pragma unroll
@@ -1173,6 +1136,11 @@ __device__ __forceinline__ void c2r_sum_body(Geo g, OlaDst d, int i0, int fr, fl
     c2r_stage<TW>(v, A, B, sl, t);
     fft<TW, +1>(v, sl, t, T);
   }
+  // the epilogue's operands of the first output columns, in flight with the
+  // overlap-add below
+  const bool epi = WGT || d.sub || d.mul || d.axz;
+  OlaEpi E;
+  if (epi) ola_epi_load<WGT>(E, d, i0, fr, (int)threadIdx.x, zr0);
   __syncthreads();  // the slices become class rows; column weights staged
   {
     float4* z4 = (float4*)rowbuf;
@@ -1209,13 +1177,12 @@ __device__ __forceinline__ void c2r_sum_body(Geo g, OlaDst d, int i0, int fr, fl
   // together
   for (int rr = 0; rr < R && i0 + rr < d.O0; ++rr) {
     const float* cr = rowbuf + rr * NC * RLc;
-    const int irow = i0 + rr;
-    const size_t orow = ((size_t)fr * d.O0 + irow) * d.O1;
+    const size_t orow = ((size_t)fr * d.O0 + i0 + rr) * d.O1;
     // floor columns of a row with real weights: the left one from its slot,
     // others evaluated apart below
-    const bool fix = WGT && !d.zrow[irow];
-    const float* cw = WGT ? d.colw + (fix ? 0 : d.O1) : nullptr;
+    const bool fix = WGT && !(rr ? d.zrow[i0 + rr] != 0 : zr0);
     for (int j0 = threadIdx.x; j0 < d.O1; j0 += 4 * WG) {
+      if (epi && (rr || j0 != (int)threadIdx.x)) ola_epi_load<WGT>(E, d, i0 + rr, fr, j0, !fix);
       float acc[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -1232,19 +1199,18 @@ __device__ __forceinline__ void c2r_sum_body(Geo g, OlaDst d, int i0, int fr, fl
         const int eb = vcol == d.bcol[0] ? 0 : vcol == d.bcol[1] ? 1 : -1;
         const int bce = eb == 0 ? d.bc[0] : d.bc[1];
         if (j < d.O1 && !(fix && eb >= 0 && bce != 0)) {
-          const size_t o = orow + j;
           float a;
           if (WGT && fix && eb >= 0)
             a = wcs[TPT * MW + rr] * d.scale;  // left floor column: mean of the covering patches
           else if constexpr (WGT)
-            a = acc[e] * d.scale * cw[j];
+            a = acc[e] * d.scale * E.cw[e];
           else
             a = acc[e] * d.scale;
-          if (d.sub) a -= d.sub[o];
-          if (d.mul) a *= d.mul[o];
-          if (d.axz) a += d.beta * d.axz[o];
+          if (d.sub) a -= E.sub[e];
+          if (d.mul) a *= E.mul[e];
+          if (d.axz) a += d.beta * E.axz[e];
           if (d.clip_lo) a = fmaxf(a, d.lo);
-          d.out[o] = a;
+          d.out[orow + j] = a;
         }
       }
     }
@@ -1597,13 +1563,9 @@ __global__ __launch_bounds__(WG) void k_batch_rows(const BatchGroup* __restrict_
   const int gi = batch_find(L, (int)blockIdx.x);
   const int lb = (int)blockIdx.x - L.start[gi];
   const BatchGroup& B = G[L.gidx[gi]];
-  const Geo& g = res == 1 ? B.gres : res == 2 ? B.gx : B.g;
   const RowJobs& jobs = res == 1 ? B.rows_res : res == 2 ? B.rows_x : B.rows_fwd;
-  if (lb >= g.P * jobs.blk_end[jobs.n - 1]) return;
-  int pu, ji, q0;
-  rows_unit<TW>(g, jobs, lb, pu, ji, q0);
-  const RowSrc s = jobs.s[ji];
-  rows_r2c_body<TW>(g, s, jobs.out[ji], pu, q0, sm, B.tw);
+  if (jobs.n == 0 || lb >= jobs.u[jobs.n - 1].send * NXCD) return;
+  rows_r2c_unit<TW>(B.g, jobs, lb, sm, B.tw);
 }
 
 template <int TH, int OP>
@@ -1688,9 +1650,9 @@ int batch_tile(const BatchGroup& G, int pass) {
 int batch_blocks(const BatchGroup& G, int pass) {
   const int TPW = WG / (G.g.Tw / 16);
   switch (pass) {
-    case BP_ROWS_FWD: return G.g.P * G.rows_fwd.blk_end[G.rows_fwd.n - 1];
-    case BP_ROWS_RES: return G.gres.P * G.rows_res.blk_end[G.rows_res.n - 1];
-    case BP_ROWS_X: return G.rows_x.n ? G.gx.P * G.rows_x.blk_end[G.rows_x.n - 1] : 0;
+    case BP_ROWS_FWD: return row_blocks(G.rows_fwd);
+    case BP_ROWS_RES: return row_blocks(G.rows_res);
+    case BP_ROWS_X: return row_blocks(G.rows_x);
     case BP_COLS_FWD:
     case BP_COLS_ADJ: {
       const int CS = WG / (G.g.Th / 16);
