@@ -109,6 +109,9 @@ def kernel_models(plan, B):
                                  flops=B * (H * half(plan.csf[1]) if plan.separable else P * sw0 / 2) * rf),
         'rows_c2r_stack': dict(bytes=B * (P * sf0 * NB * 8 + P * sf0 * sf1 * 4), flops=B * P * half(sf0) * rf),
     }
+    # the x-adjoint's overlap-add and the f-adjoint's stack in one launch
+    win, stk = m['rows_c2r_ola_win'], m['rows_c2r_stack']
+    m['rows_c2r_ola_win_stack'] = {k: win[k] + stk[k] for k in win}
     return m
 
 

@@ -345,6 +345,11 @@ OlaDst dst_adjoint_x(const vmbd_plan* p, float* xbar) {
 
 // row transforms of x and f: one launch over both (one geometry, or, with
 // the image rows shared per patch column, a geometry per job)
+// the PSF-shaped results of a call's column pass
+StackDst dst_stack(const vmbd_plan* p, const Geo& g, float* out, const float* axz = nullptr, float beta = 0.f) {
+  return StackDst{p->Y2, g.sf0, out, g.sf0, g.sf1, inv_scale(g), axz, beta, fast_div(g.P)};
+}
+
 // One launch of the row transforms of up to four operands, each over the
 // patches of its own geometry
 struct RowOp {
@@ -835,7 +840,7 @@ int vmbd_ola_adjoint_f(vmbd_plan* p, int32_t nframes, const float* gres, const f
   ColOut o1{p->Y2, g.sf0}, o2{nullptr, 0};
   ColIn none{};
   VMBD_LAUNCH(launch_cols(g, COL_ADJ1, shared_in(p->wsG, sr), xr.in, none, o1, o2, nullptr, p->tw, st, p->tune.col_threads));
-  VMBD_LAUNCH(launch_rows_c2r_stack(g, p->Y2, g.sf0, fbar, g.sf0, g.sf1, inv_scale(g), p->tw, st));
+  VMBD_LAUNCH(launch_rows_c2r_stack(g, dst_stack(p, g, fbar), p->tw, st));
   return VMBD_OK;
 }
 
@@ -863,8 +868,8 @@ int vmbd_ola_adjoint_xf(vmbd_plan* p, int32_t nframes, const float* gres, const 
   ColOut o1{p->Y1, g.sw0}, o2{p->Y2, g.sf0};
   VMBD_LAUNCH(launch_cols(g, COL_ADJ2, shared_in(p->wsG, sr), raw_in(p->wsF, sf), xr.in, o1, o2, nullptr, p->tw, st,
                           p->tune.col_threads));
-  VMBD_LAUNCH(launch_rows_c2r_ola(g, dst_adjoint_x(p, xbar), p->tw, st, p->tune.ola_threads));
-  VMBD_LAUNCH(launch_rows_c2r_stack(g, p->Y2, g.sf0, fbar, g.sf0, g.sf1, inv_scale(g), p->tw, st));
+  VMBD_LAUNCH(launch_rows_c2r_ola_stack(g, dst_adjoint_x(p, xbar), dst_stack(p, g, fbar), p->tw, st,
+                                        p->tune.ola_threads));
   return VMBD_OK;
 }
 
@@ -983,7 +988,7 @@ int vmbd_ola_adjoint_cached_ex(vmbd_plan* p, int32_t nframes, int32_t kind, cons
   } else {
     ColOut o1{p->Y2, g.sf0};
     VMBD_LAUNCH(launch_cols(g, COL_ADJ1, shared_in(p->wsG, sr), spec_in(spec, g.Th), none, o1, o2, nullptr, p->tw, st, p->tune.col_threads));
-    VMBD_LAUNCH(launch_rows_c2r_stack(g, p->Y2, g.sf0, out, g.sf0, g.sf1, inv_scale(g), p->tw, st, z, beta));
+    VMBD_LAUNCH(launch_rows_c2r_stack(g, dst_stack(p, g, out, z, beta), p->tw, st));
   }
   return VMBD_OK;
 }
@@ -1093,7 +1098,7 @@ int vmbd_deconv_direct(vmbd_plan* p, int32_t kind, const void* spec, const float
     VMBD_LAUNCH(launch_rows_c2r_ola(g, dst_patches(p, out, false), p->tw, st));
   } else {
     VMBD_LAUNCH(launch_cols_div(g, DIV_X, in, 2, prm, ColOut{p->Y2, g.sf0}, nullptr, p->tw, st));
-    VMBD_LAUNCH(launch_rows_c2r_stack(g, p->Y2, g.sf0, out, g.sf0, g.sf1, inv_scale(g), p->tw, st));
+    VMBD_LAUNCH(launch_rows_c2r_stack(g, dst_stack(p, g, out), p->tw, st));
   }
   return VMBD_OK;
 }
@@ -1118,7 +1123,7 @@ int vmbd_deconv_gdirect(vmbd_plan* p, const float* xx, const float* xy, const fl
                        raw_in(outs[3], srcs[3])};
   VMBD_LAUNCH(launch_cols_div(g, DIV_G, in, 4, DivParams{alpha, beta, 0.f}, ColOut{p->Y2, g.sf0}, nullptr, p->tw,
                               st));
-  VMBD_LAUNCH(launch_rows_c2r_stack(g, p->Y2, g.sf0, fout, g.sf0, g.sf1, inv_scale(g), p->tw, st));
+  VMBD_LAUNCH(launch_rows_c2r_stack(g, dst_stack(p, g, fout), p->tw, st));
   return VMBD_OK;
 }
 
@@ -1229,12 +1234,7 @@ bool batch_group(BatchGroup& B, vmbd_plan* p, int nframes, const float* x, const
   B.ola_adj = dst_adjoint_x(p, xbar);
   ola_fit_rows(B.ola_adj, (long long)B.ola_adj.O0 * nframes);
   // the grouped OLA launch runs WG threads per workgroup for every group
-  B.st_src = p->Y2;
-  B.st_srow = g.sf0;
-  B.st_nrows = g.sf0;
-  B.st_ncols = g.sf1;
-  B.st_out = fbar;
-  B.st_scale = inv_scale(g);
+  B.stack = dst_stack(p, g, fbar);
   return ok;
 }
 

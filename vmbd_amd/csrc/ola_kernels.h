@@ -85,12 +85,16 @@ struct RowUnits {
   int nfull, Tl;  // tiles of TP patches, patches of the last, shorter one
   FastDiv dTile, dTP, dTl, dPf;  // division by TP*nb, TP, Tl, Pf
 };
-struct RowJobs {
-  RowSrc s[ROW_JOBS_MAX];
-  float2* out[ROW_JOBS_MAX];
-  RowUnits u[ROW_JOBS_MAX];
+// (NJ: room for that many jobs; a launch passes no more than it needs as
+// kernel arguments)
+template <int NJ>
+struct RowJobsN {
   int n;
+  RowUnits u[NJ];
+  float2* out[NJ];
+  RowSrc s[NJ];
 };
+using RowJobs = RowJobsN<ROW_JOBS_MAX>;
 
 // Row-pass output: [P][NB][row_pitch(nr)] holding tile rows [rlo, rlo+nr);
 // the pitch rounds nr up to 16 rows so every bin column starts on a 128-byte
@@ -227,6 +231,23 @@ hipError_t launch_cols(const Geo& g, int op, const ColIn& a, const ColIn& b, con
 // wgs: threads per OLA workgroup (128, 192 or 256; 0 = ola_wg's choice);
 // 128 and 192 need every output row in one round (ola_fits)
 hipError_t launch_rows_c2r_ola(const Geo& g, const OlaDst& d, const float2* tw, hipStream_t st, int wgs = 0);
+// out = scale * the inverse row transforms of the first nrows x ncols of every
+// patch's tile (+ beta * axz when axz != null)
+struct StackDst {
+  const float2* src;
+  int srow;
+  float* out;
+  int nrows, ncols;
+  float scale;
+  const float* axz;
+  float beta;
+  FastDiv dP;  // division by the patches of the launch
+};
+hipError_t launch_rows_c2r_stack(const Geo& g, const StackDst& k, const float2* tw, hipStream_t st);
+// The overlap-add and the stack of one two-adjoint call, in one launch where
+// the overlap-add takes its weighted summed form
+hipError_t launch_rows_c2r_ola_stack(const Geo& g, const OlaDst& d, const StackDst& k, const float2* tw,
+                                     hipStream_t st, int wgs);
 // a single-round launch of wgs threads holds every output row's transforms
 int ola_fits(const Geo& g, const OlaDst& d, int wgs);
 // Column pass of a Fourier division (deconv_kernels.hip): operands a[0..na)
@@ -235,9 +256,6 @@ int ola_fits(const Geo& g, const OlaDst& d, int wgs);
 // [0, o.nrows) to o, or (SPROD) the spectrum to spec_out.
 hipError_t launch_cols_div(const Geo& g, int op, const ColIn* a, int na, DivParams prm, const ColOut& o,
                            float2* spec_out, const float2* tw, hipStream_t st);
-// out = scale * inverse row transforms (+ beta * axz when axz != null)
-hipError_t launch_rows_c2r_stack(const Geo& g, const float2* src, int srow, float* out, int nrows, int ncols,
-                                 float scale, const float2* tw, hipStream_t st, const float* axz = nullptr, float beta = 0.f);
 // Batches of several plans (frames of different geometry) whose passes run
 // as single launches over a table of groups (one group = one plan's frames):
 // everything the seven passes of a step (forward + both exact adjoints) need
@@ -252,10 +270,7 @@ struct BatchGroup {
   ColIn ca_a, ca_b, ca_c;
   ColOut ca_o1, ca_o2;
   OlaDst ola_fwd, ola_adj;
-  const float2* st_src;
-  int st_srow, st_nrows, st_ncols;
-  float* st_out;
-  float st_scale;
+  StackDst stack;
   const float2* tw;
 };
 enum BatchPass { BP_ROWS_FWD = 0, BP_ROWS_X, BP_COLS_FWD, BP_OLA_FWD, BP_ROWS_RES, BP_COLS_ADJ, BP_OLA_ADJ, BP_STACK, BP_N };

@@ -221,14 +221,14 @@ __device__ __forceinline__ void rows_r2c_body(Geo g, RowSrc s, float2* __restric
 // the same pixels, run on one XCD at the same time and share its L2.  The map
 // id -> (job, patch, row block) is a bijection whatever the hardware
 // placement, apart from ids past an XCD's share, which have no unit.
-template <int TW>
-__device__ __forceinline__ void rows_r2c_unit(const Geo& g, const RowJobs& jobs, int blk, float2* sm,
+template <int TW, int NJ>
+__device__ __forceinline__ void rows_r2c_unit(const Geo& g, const RowJobsN<NJ>& jobs, int blk, float2* sm,
                                               const float2* __restrict__ tw) {
   constexpr int TPW = WG / (TW / 16);
   const int xcd = blk % NXCD;
   int ji = 0, slot = blk / NXCD, s0 = 0;
 #pragma unroll
-  for (int jj = 0; jj < ROW_JOBS_MAX - 1; ++jj)
+  for (int jj = 0; jj < NJ - 1; ++jj)
     if (jobs.n > jj + 1 && slot >= jobs.u[jj].send) {
       ji = jj + 1;
       s0 = jobs.u[jj].send;
@@ -245,8 +245,8 @@ __device__ __forceinline__ void rows_r2c_unit(const Geo& g, const RowJobs& jobs,
   rows_r2c_body<TW>(g, jobs.s[ji], jobs.out[ji], p, fr, p - fr * U.Pf, by * TPW, sm, tw);
 }
 
-template <int TW>
-__global__ __launch_bounds__(WG) void k_rows_r2c(Geo g, RowJobs jobs, const float2* __restrict__ tw) {
+template <int TW, int NJ>
+__global__ __launch_bounds__(WG) void k_rows_r2c(Geo g, RowJobsN<NJ> jobs, const float2* __restrict__ tw) {
   __shared__ float2 sm[RowsLds<TW>::v];
   rows_r2c_unit<TW>(g, jobs, (int)blockIdx.x, sm, tw);
 }
@@ -281,7 +281,22 @@ int row_blocks(const RowJobs& jobs) { return jobs.n ? jobs.u[jobs.n - 1].send * 
 template <int TW>
 static hipError_t rows_r2c_t(const Geo& g, const RowJobs& jobs, const float2* tw, hipStream_t st, const char* name) {
   ProfScope ps(name, st);
-  hipLaunchKernelGGL(k_rows_r2c<TW>, dim3((unsigned)row_blocks(jobs)), dim3(WG), 0, st, g, jobs, tw);
+  auto go = [&](auto few) {
+    constexpr int NJ = sizeof(few.u) / sizeof(RowUnits);
+    few.n = jobs.n;
+    for (int i = 0; i < jobs.n; ++i) {
+      few.u[i] = jobs.u[i];
+      few.out[i] = jobs.out[i];
+      few.s[i] = jobs.s[i];
+    }
+    hipLaunchKernelGGL((k_rows_r2c<TW, NJ>), dim3((unsigned)row_blocks(jobs)), dim3(WG), 0, st, g, few, tw);
+  };
+  if (jobs.n == 1)
+    go(RowJobsN<1>{});
+  else if (jobs.n == 2)
+    go(RowJobsN<2>{});
+  else
+    go(RowJobs(jobs));
   return hipGetLastError();
 }
 
@@ -1466,10 +1481,13 @@ struct StackLds {
 // One workgroup of the stack pass: row block by of patch p (fl:
 // StackLds<TW>::v float2 of LDS).
 template <int TW>
-__device__ __forceinline__ void c2r_stack_body(Geo g, const float2* __restrict__ src, int srow,
-                                               float* __restrict__ out, int nrows, int ncols, float scale,
-                                               const float2* __restrict__ tw, const float* __restrict__ axz, float beta,
-                                               int p, int by, float2* fl) {
+__device__ __forceinline__ void c2r_stack_body(Geo g, const StackDst& k, const float2* __restrict__ tw, int p, int by,
+                                               float2* fl) {
+  const float2* __restrict__ src = k.src;
+  float* __restrict__ out = k.out;
+  const float* __restrict__ axz = k.axz;
+  const int srow = k.srow, nrows = k.nrows, ncols = k.ncols;
+  const float scale = k.scale, beta = k.beta;
   constexpr int TPT = TW / 16;
   constexpr int TPW = WG / TPT;
   constexpr int SL = FftLds<TW>::floats2;
@@ -1508,36 +1526,90 @@ __device__ __forceinline__ void c2r_stack_body(Geo g, const float2* __restrict__
 }
 
 template <int TW>
-__global__ __launch_bounds__(WG) void k_rows_c2r_stack(Geo g, const float2* __restrict__ src, int srow,
-                                                       float* __restrict__ out, int nrows, int ncols, float scale,
-                                                       const float2* __restrict__ tw, const float* __restrict__ axz,
-                                                       float beta) {
+__global__ __launch_bounds__(WG) void k_rows_c2r_stack(Geo g, StackDst k, const float2* __restrict__ tw) {
   __shared__ float2 fl[StackLds<TW>::v];
-  c2r_stack_body<TW>(g, src, srow, out, nrows, ncols, scale, tw, axz, beta, blockIdx.x, blockIdx.y, fl);
+  c2r_stack_body<TW>(g, k, tw, blockIdx.x, blockIdx.y, fl);
 }
 
 template <int TW>
-static hipError_t c2r_stack_t(const Geo& g, const float2* src, int srow, float* out, int nrows, int ncols,
-                              float scale, const float2* tw, hipStream_t st, const float* axz, float beta) {
+static int stack_blocks(const StackDst& k) {  // row blocks per patch
   constexpr int TPW = WG / (TW / 16);
-  const int blocks = ((nrows + 1) / 2 + TPW - 1) / TPW;
+  return ((k.nrows + 1) / 2 + TPW - 1) / TPW;
+}
+
+template <int TW>
+static hipError_t c2r_stack_t(const Geo& g, const StackDst& k, const float2* tw, hipStream_t st) {
+  const int blocks = stack_blocks<TW>(k);
   if (blocks <= 0 || g.P <= 0) return hipSuccess;
   ProfScope ps("rows_c2r_stack", st);
-  hipLaunchKernelGGL(k_rows_c2r_stack<TW>, dim3((unsigned)g.P, (unsigned)blocks), dim3(WG), 0, st, g, src, srow,
-                     out, nrows, ncols, scale, tw, axz, beta);
+  hipLaunchKernelGGL(k_rows_c2r_stack<TW>, dim3((unsigned)g.P, (unsigned)blocks), dim3(WG), 0, st, g, k, tw);
   return hipGetLastError();
 }
 
-hipError_t launch_rows_c2r_stack(const Geo& g, const float2* src, int srow, float* out, int nrows, int ncols,
-                                 float scale, const float2* tw, hipStream_t st, const float* axz, float beta) {
+hipError_t launch_rows_c2r_stack(const Geo& g, const StackDst& k, const float2* tw, hipStream_t st) {
   if (g.NBP < g.Tw / 2 + 2) return hipErrorInvalidValue;  // two-bin loads need a padding bin per row
   switch (g.Tw) {
-    case 16: return c2r_stack_t<16>(g, src, srow, out, nrows, ncols, scale, tw, st, axz, beta);
-    case 32: return c2r_stack_t<32>(g, src, srow, out, nrows, ncols, scale, tw, st, axz, beta);
-    case 64: return c2r_stack_t<64>(g, src, srow, out, nrows, ncols, scale, tw, st, axz, beta);
-    case 128: return c2r_stack_t<128>(g, src, srow, out, nrows, ncols, scale, tw, st, axz, beta);
-    case 256: return c2r_stack_t<256>(g, src, srow, out, nrows, ncols, scale, tw, st, axz, beta);
-    case 512: return c2r_stack_t<512>(g, src, srow, out, nrows, ncols, scale, tw, st, axz, beta);
+    case 16: return c2r_stack_t<16>(g, k, tw, st);
+    case 32: return c2r_stack_t<32>(g, k, tw, st);
+    case 64: return c2r_stack_t<64>(g, k, tw, st);
+    case 128: return c2r_stack_t<128>(g, k, tw, st);
+    case 256: return c2r_stack_t<256>(g, k, tw, st);
+    case 512: return c2r_stack_t<512>(g, k, tw, st);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// The x-adjoint's overlap-add (weighted summed form, blocks [0, nsum)) and the
+// f-adjoint's stack (the blocks after it) of one call in one launch: both read
+// only the column pass's results, and the stack's short rows fill the tail of
+// the overlap-add.  One 1024^2 frame: 11.8 + 4.4 us in two launches, 14.1 in
+// one.
+template <int TW>
+__global__ __launch_bounds__(WG, (TW >= 512 ? 3 : TW >= 64 ? 4 : 1)) void k_rows_c2r_sum_stack(
+    Geo g, OlaDst d, StackDst k, int nsum, FastDiv drows, const float2* __restrict__ tw) {
+  extern __shared__ float2 dyn[];
+  const int b = (int)blockIdx.x;
+  if (b < nsum) {
+    const int nbr = (d.O0 + d.sumr - 1) / d.sumr;
+    const int fr = div_by(b, drows);
+    c2r_sum_body<TW, true>(g, d, (b - fr * nbr) * d.sumr, fr, dyn, tw);
+  } else {
+    const int by = div_by(b - nsum, k.dP);
+    c2r_stack_body<TW>(g, k, tw, b - nsum - by * g.P, by, dyn);
+  }
+}
+
+template <int TW>
+static hipError_t c2r_ola_stack_t(const Geo& g, const OlaDst& d0, const StackDst& k, const float2* tw, hipStream_t st,
+                                  int wgs) {
+  const int frames = g.P / g.Pf;
+  OlaDst d = d0;
+  ola_fit_rows(d, (long long)d.O0 * frames);
+  const int nst = stack_blocks<TW>(k);
+  const long long nbr = d.sumr ? (d.O0 + d.sumr - 1) / d.sumr : 0;
+  const long long nsum = nbr * frames, n = nsum + (long long)g.P * nst;
+  if (!d.sumr || !d.wrow || nst <= 0 || d.O0 <= 0 || d.O1 <= 0 || n > INT_MAX) {
+    const hipError_t e = launch_rows_c2r_ola(g, d0, tw, st, wgs);
+    return e != hipSuccess ? e : launch_rows_c2r_stack(g, k, tw, st);
+  }
+  const size_t shm = std::max(ola_shared_bytes(g, d), StackLds<TW>::v * sizeof(float2));
+  ProfScope ps("rows_c2r_ola_win_stack", st);
+  hipLaunchKernelGGL(k_rows_c2r_sum_stack<TW>, dim3((unsigned)n), dim3(WG), shm, st, g, d, k, (int)nsum,
+                     fast_div((int)nbr), tw);
+  return hipGetLastError();
+}
+
+hipError_t launch_rows_c2r_ola_stack(const Geo& g, const OlaDst& d, const StackDst& k, const float2* tw,
+                                     hipStream_t st, int wgs) {
+  if (g.NBP < g.Tw / 2 + 2) return hipErrorInvalidValue;  // two-bin loads need a padding bin per row
+  if (wgs != 0 && wgs != 128 && wgs != 192 && wgs != WG) return hipErrorInvalidValue;
+  switch (g.Tw) {
+    case 16: return c2r_ola_stack_t<16>(g, d, k, tw, st, wgs);
+    case 32: return c2r_ola_stack_t<32>(g, d, k, tw, st, wgs);
+    case 64: return c2r_ola_stack_t<64>(g, d, k, tw, st, wgs);
+    case 128: return c2r_ola_stack_t<128>(g, d, k, tw, st, wgs);
+    case 256: return c2r_ola_stack_t<256>(g, d, k, tw, st, wgs);
+    case 512: return c2r_ola_stack_t<512>(g, d, k, tw, st, wgs);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1638,9 +1710,8 @@ __global__ __launch_bounds__(WG) void k_batch_stack(const BatchGroup* __restrict
   const int lb = (int)blockIdx.x - L.start[gi];
   const BatchGroup& B = G[L.gidx[gi]];
   const int by = lb / B.g.P;
-  if (by * TPW >= (B.st_nrows + 1) / 2) return;
-  c2r_stack_body<TW>(B.g, B.st_src, B.st_srow, B.st_out, B.st_nrows, B.st_ncols, B.st_scale, B.tw, nullptr, 0.f,
-                     lb - by * B.g.P, by, fl);
+  if (by * TPW >= (B.stack.nrows + 1) / 2) return;
+  c2r_stack_body<TW>(B.g, B.stack, B.tw, lb - by * B.g.P, by, fl);
 }
 
 int batch_tile(const BatchGroup& G, int pass) {
@@ -1664,7 +1735,7 @@ int batch_blocks(const BatchGroup& G, int pass) {
     case BP_OLA_ADJ:
       return (G.ola_adj.sumr ? (G.ola_adj.O0 + G.ola_adj.sumr - 1) / G.ola_adj.sumr : G.ola_adj.O0) *
              (G.g.P / G.g.Pf);
-    case BP_STACK: return G.g.P * (((G.st_nrows + 1) / 2 + TPW - 1) / TPW);
+    case BP_STACK: return G.g.P * (((G.stack.nrows + 1) / 2 + TPW - 1) / TPW);
     default: return 0;
   }
 }
