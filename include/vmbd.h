@@ -181,6 +181,17 @@ int vmbd_ola_adjoint_f(vmbd_plan* plan, int32_t nframes, const float* g, const f
 int vmbd_ola_adjoint_xf(vmbd_plan* plan, int32_t nframes, const float* g, const float* x, const float* f,
                         float* xbar, float* fbar, int32_t exact, int32_t flags, vmbd_stream_t stream);
 
+/* vmbd_ola_forward with `sub` (shaped like y, NULL for none) subtracted in
+ * the final store: y = B(x, f) - sub, the residual of a data term. */
+int vmbd_ola_forward_ex(vmbd_plan* plan, int32_t nframes, const float* x, const float* f, const float* sub,
+                        float* y, vmbd_stream_t stream);
+
+/* vmbd_ola_adjoint_xf with both results multiplied by the device scalar
+ * gscale[0] (NULL for 1), the upstream gradient of a loss. */
+int vmbd_ola_adjoint_xf_ex(vmbd_plan* plan, int32_t nframes, const float* g, const float* x, const float* f,
+                           const float* gscale, float* xbar, float* fbar, int32_t exact, int32_t flags,
+                           vmbd_stream_t stream);
+
 /* Cached spectra, the OlaGPU constructor (olaGPU.py:142-157):
  * kind VMBD_CACHE_PSF  : z = f stack  -> spec = FFT(pad_stack(f))
  * kind VMBD_CACHE_IMAGE: z = image x  -> spec = FFT(chop_mod_pad(x, ws))

@@ -111,6 +111,13 @@ int vmbd_tv(const float* x, int32_t K, int32_t H, int32_t W, float eps, double* 
 int vmbd_tv_grad(float* grad, const float* x, int32_t K, int32_t H, int32_t W, float eps, const float* scale,
                  float weight, int32_t accumulate, vmbd_stream_t stream);
 
+/* value_out[0] = sum r^2 / 2 + lam * TV(x): the loss of a residual r (nr
+ * values) and K images H x W, summed in double and rounded once.  lam = 0
+ * leaves x out (it may be NULL).  partials: 2 * vmbd_reduce_blocks(max(nr,
+ * K*H*W)) doubles. */
+int vmbd_loss(const float* r, int64_t nr, const float* x, int32_t K, int32_t H, int32_t W, float eps, float lam,
+              double* partials, float* value_out, vmbd_stream_t stream);
+
 /* Multiplicative latent-image step (vmbd_chimney.py:143-147):
  * x *= max(num / (den + tol), tol); then x = min(x, max of x over rows
  * [border0, H - border0) and columns [border1, W - border1)).  partial_max:

@@ -122,3 +122,54 @@ def test_adam_decreases_loss(cuda, setup):
         opt.step()
         first = loss.item() if first is None else first
     assert crit(xt, ft, yt).item() < 0.9 * first
+
+
+@pytest.mark.parametrize('shape', [(1, 1, 1), (2, 1, 7), (1, 5, 1), (1, 3, 257), (3, 9, 1030), (1, 70, 64)])
+def test_loss_and_tv_kernels_edges(cuda, shape):
+    # one row, one column, widths around the tiles of 64 and the 1024 columns
+    # a block takes per step; residual lengths that leave a remainder of 4.
+    # Sums are in double: 1e-6 covers the rounding of n (2^-23) and of the sum
+    import torch
+    from vmbd_amd import _lib
+    from vmbd_amd.autograd import tv
+    print(f'case loss kernels {shape}', flush=True)
+    K, H, W = shape
+    rng = np.random.default_rng(K + H + W)
+    x, r = _f32(rng.random(shape)), _f32(rng.standard_normal(H * W + 3))
+    xt, rt = _t(x, cuda, True), _t(r, cuda)
+    part = torch.empty(2 * _lib.lib().vmbd_reduce_blocks(max(r.size, x.size)), dtype=torch.float64, device=cuda)
+    for lam in (0.0, 0.3):
+        val = torch.empty(1, device=cuda)
+        _lib.call('vmbd_loss', _lib.ptr(rt), r.size, _lib.ptr(xt), K, H, W, 0.05, lam, _lib.ptr(part), _lib.ptr(val),
+                  _lib.stream_ptr())
+        ref = 0.5 * float(r @ r) + lam * L.tv(x, 0.05)
+        assert abs(val.item() - ref) < 1e-6 * ref
+    v = tv(xt, 0.05)
+    v.backward()
+    assert abs(v.item() - L.tv(x, 0.05)) < 1e-6 * L.tv(x, 0.05)
+    assert np.abs(_n(xt.grad) - L.tv_grad(x, 0.05)).max() < 1e-5
+
+
+def test_loss_forms_agree(cuda, setup):
+    # the one-function form (constant y) against the sum of its terms (y that
+    # takes a gradient), upstream gradient 2.5, each gradient alone as well:
+    # the same operator, three roundings more or less (1e-6)
+    import torch
+    from vmbd_amd.autograd import OlaLoss
+    print('case loss forms', flush=True)
+    plan, owa, x, f, y = setup
+    crit = OlaLoss(plan, 1e-3, 1e-2)
+    up = torch.tensor(2.5, device=cuda)
+    a, b, c = _t(x, cuda, True), _t(f, cuda, True), _t(y, cuda, True)
+    general = crit(a, b, c)
+    general.backward(up)
+    assert c.grad is not None
+    for need in ((True, True), (True, False), (False, True)):
+        p, q = _t(x, cuda, need[0]), _t(f, cuda, need[1])
+        v = crit(p, q, _t(y, cuda))
+        v.backward(up)
+        assert abs(v.item() - general.item()) < 1e-6 * abs(general.item())
+        assert not need[0] or rel_l2(_n(p.grad), _n(a.grad)) < 1e-6
+        assert not need[1] or rel_l2(_n(q.grad), _n(b.grad)) < 1e-6
+    with torch.no_grad():
+        assert abs(crit(a, b, _t(y, cuda)).item() - general.item()) < 1e-6 * abs(general.item())

@@ -55,6 +55,8 @@ SIGNATURES = {
     'vmbd_ola_adjoint_x': (ctypes.c_int, [_P, _I, _F, _F, _F, _I, _P]),
     'vmbd_ola_adjoint_f': (ctypes.c_int, [_P, _I, _F, _F, _F, _I, _P]),
     'vmbd_ola_adjoint_xf': (ctypes.c_int, [_P, _I, _F, _F, _F, _F, _F, _I, _I, _P]),
+    'vmbd_ola_forward_ex': (ctypes.c_int, [_P, _I, _F, _F, _F, _F, _P]),
+    'vmbd_ola_adjoint_xf_ex': (ctypes.c_int, [_P, _I, _F, _F, _F, _P, _F, _F, _I, _I, _P]),
     'vmbd_spectra': (ctypes.c_int, [_P, _I, _I, _F, _P, _P]),
     'vmbd_cache_psf_spectra': (ctypes.c_int, [_P, _I, _F, _P, _P]),
     'vmbd_cache_image_spectra': (ctypes.c_int, [_P, _I, _F, _P, _P]),
@@ -104,6 +106,7 @@ SIGNATURES = {
     'vmbd_pbb_step_noalloc': (ctypes.c_int, [_F, _F, _F, _F, _F, ctypes.c_int64, _I, _I, _F, _P]),
     'vmbd_tv': (ctypes.c_int, [_F, _I, _I, _I, ctypes.c_float, _P, _P, _P]),
     'vmbd_tv_grad': (ctypes.c_int, [_F, _F, _I, _I, _I, ctypes.c_float, _P, ctypes.c_float, _I, _P]),
+    'vmbd_loss': (ctypes.c_int, [_F, ctypes.c_int64, _F, _I, _I, _I, ctypes.c_float, ctypes.c_float, _P, _F, _P]),
     'vmbd_rl_update': (ctypes.c_int, [_F, _F, _F, _I, _I, ctypes.c_float, _I, _I, _F, _F, _P]),
     # filters, include/vmbd_filters.h
     'vmbd_shock_step': (ctypes.c_int, [_F, _F, _I, _I, ctypes.c_float, ctypes.c_float, _P]),

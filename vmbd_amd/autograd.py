@@ -85,6 +85,46 @@ def tv(x, eps=1e-3):
     return _TvFunction.apply(x, eps)
 
 
+class _LossFunction(torch.autograd.Function):
+    """1/2 |B(x, f) - y|^2 + lam TV(x) for a constant y: the residual is formed
+    in the operator's final store and kept for the backward, which is linear in
+    it; the upstream scalar is applied in the adjoints' final stores."""
+
+    @staticmethod
+    def forward(ctx, x, f, y, plan, lam, eps, exact):
+        r = plan.forward(x, f, sub=y)
+        xc = x.contiguous()
+        H, W = int(xc.shape[-2]), int(xc.shape[-1])
+        K = xc.numel() // (H * W)
+        nb = _lib.lib().vmbd_reduce_blocks(max(r.numel(), xc.numel()))
+        part = torch.empty(2 * nb, dtype=torch.float64, device=xc.device)
+        val = torch.empty((), dtype=torch.float32, device=xc.device)
+        _lib.call('vmbd_loss', _lib.ptr(r), r.numel(), _lib.ptr(xc), K, H, W, eps, lam, _lib.ptr(part), _lib.ptr(val),
+                  _lib.stream_ptr())
+        ctx.plan, ctx.lam, ctx.eps, ctx.exact = plan, lam, eps, exact
+        ctx.save_for_backward(x, f, r)
+        return val
+
+    @staticmethod
+    def backward(ctx, g):
+        x, f, r = ctx.saved_tensors
+        plan = ctx.plan
+        gx = gf = None
+        g = g.contiguous()
+        if ctx.needs_input_grad[0] and ctx.needs_input_grad[1]:
+            gx, gf = plan.adjoint_xf(r, x, f, exact=ctx.exact, scale=g)
+        elif ctx.needs_input_grad[0]:
+            gx = plan.adjoint_x(r * g, f, exact=ctx.exact)
+        elif ctx.needs_input_grad[1]:
+            gf = plan.adjoint_f(r * g, x, exact=ctx.exact)
+        if gx is not None and ctx.lam:
+            xc = x.contiguous()
+            H, W = int(xc.shape[-2]), int(xc.shape[-1])
+            _lib.call('vmbd_tv_grad', _lib.ptr(gx), _lib.ptr(xc), xc.numel() // (H * W), H, W, ctx.eps, _lib.ptr(g),
+                      ctx.lam, 1, _lib.stream_ptr())
+        return gx, gf, None, None, None, None, None
+
+
 class OlaLoss(torch.nn.Module):
     """L(x, f) = 1/2 |B(x, f) - y|^2 + lam TV(x)."""
 
@@ -95,7 +135,18 @@ class OlaLoss(torch.nn.Module):
         self.eps = float(eps)
         self.exact = bool(exact)
 
+    def _fused(self, x, f, y):
+        """The operands the one-function form takes: float32 tensors on the
+        plan's device, y constant and shaped like the result."""
+        p = self.plan
+        if not all(isinstance(t, torch.Tensor) and t.dtype == torch.float32 and t.device == p.device
+                   for t in (x, f, y)):
+            return False
+        return not y.requires_grad and x.dim() in (2, 3) and tuple(y.shape) == tuple(x.shape[:-2]) + p.sy
+
     def forward(self, x, f, y):
+        if self._fused(x, f, y):
+            return _LossFunction.apply(x, f, y, self.plan, self.lam, self.eps, self.exact)
         r = ola(x, f, self.plan, self.exact) - y
         out = 0.5 * (r * r).sum()
         if self.lam:

@@ -347,7 +347,7 @@ OlaDst dst_adjoint_x(const vmbd_plan* p, float* xbar) {
 // the image rows shared per patch column, a geometry per job)
 // the PSF-shaped results of a call's column pass
 StackDst dst_stack(const vmbd_plan* p, const Geo& g, float* out, const float* axz = nullptr, float beta = 0.f) {
-  return StackDst{p->Y2, g.sf0, out, g.sf0, g.sf1, inv_scale(g), axz, beta, fast_div(g.P)};
+  return StackDst{p->Y2, g.sf0, out, g.sf0, g.sf1, inv_scale(g), axz, beta, fast_div(g.P), nullptr};
 }
 
 // One launch of the row transforms of up to four operands, each over the
@@ -789,6 +789,11 @@ size_t vmbd_plan_spectrum_elems(const vmbd_plan* plan) {
 
 int vmbd_ola_forward(vmbd_plan* p, int32_t nframes, const float* x, const float* f, float* y,
                      vmbd_stream_t stream) {
+  return vmbd_ola_forward_ex(p, nframes, x, f, nullptr, y, stream);
+}
+
+int vmbd_ola_forward_ex(vmbd_plan* p, int32_t nframes, const float* x, const float* f, const float* sub, float* y,
+                        vmbd_stream_t stream) {
   vmbd_clear_error();
   if (int r = check_plan(p, nframes)) return r;
   if (!x || !f || !y) return vmbd_fail(VMBD_E_ARG, "vmbd_ola_forward: null pointer");
@@ -802,7 +807,9 @@ int vmbd_ola_forward(vmbd_plan* p, int32_t nframes, const float* x, const float*
   ColIn none{nullptr, 0, 0, 0};
   VMBD_LAUNCH(launch_cols(g, COL_FWD, xr.in, raw_in(p->wsF, sf), none, o1, o2, nullptr, p->tw, st,
                           p->tune.col_threads));
-  VMBD_LAUNCH(launch_rows_c2r_ola(g, dst_forward(p, y), p->tw, st, p->tune.ola_threads));
+  OlaDst d = dst_forward(p, y);
+  d.sub = sub;
+  VMBD_LAUNCH(launch_rows_c2r_ola(g, d, p->tw, st, p->tune.ola_threads));
   p->rows_frames = nframes;
   return VMBD_OK;
 }
@@ -846,6 +853,12 @@ int vmbd_ola_adjoint_f(vmbd_plan* p, int32_t nframes, const float* gres, const f
 
 int vmbd_ola_adjoint_xf(vmbd_plan* p, int32_t nframes, const float* gres, const float* x, const float* f,
                         float* xbar, float* fbar, int32_t exact, int32_t flags, vmbd_stream_t stream) {
+  return vmbd_ola_adjoint_xf_ex(p, nframes, gres, x, f, nullptr, xbar, fbar, exact, flags, stream);
+}
+
+int vmbd_ola_adjoint_xf_ex(vmbd_plan* p, int32_t nframes, const float* gres, const float* x, const float* f,
+                           const float* gscale, float* xbar, float* fbar, int32_t exact, int32_t flags,
+                           vmbd_stream_t stream) {
   vmbd_clear_error();
   if (int r = check_plan(p, nframes)) return r;
   if (!gres || !xbar || !fbar) return vmbd_fail(VMBD_E_ARG, "vmbd_ola_adjoint_xf: null pointer");
@@ -868,8 +881,10 @@ int vmbd_ola_adjoint_xf(vmbd_plan* p, int32_t nframes, const float* gres, const 
   ColOut o1{p->Y1, g.sw0}, o2{p->Y2, g.sf0};
   VMBD_LAUNCH(launch_cols(g, COL_ADJ2, shared_in(p->wsG, sr), raw_in(p->wsF, sf), xr.in, o1, o2, nullptr, p->tw, st,
                           p->tune.col_threads));
-  VMBD_LAUNCH(launch_rows_c2r_ola_stack(g, dst_adjoint_x(p, xbar), dst_stack(p, g, fbar), p->tw, st,
-                                        p->tune.ola_threads));
+  OlaDst dx = dst_adjoint_x(p, xbar);
+  StackDst df = dst_stack(p, g, fbar);
+  dx.gs = df.gs = gscale;
+  VMBD_LAUNCH(launch_rows_c2r_ola_stack(g, dx, df, p->tw, st, p->tune.ola_threads));
   return VMBD_OK;
 }
 

@@ -184,8 +184,10 @@ struct OlaDst {
   const float* colw;
   const int* zrow;
   int bcol[2], bn[2], bc[2];
-  // 1/(Th*Tw) of the unnormalised transforms, applied to the overlap-add sum
+  // 1/(Th*Tw) of the unnormalised transforms, applied to the overlap-add sum,
+  // times the device scalar gs[0] (null: 1)
   float scale;
+  const float* gs;
   // fused solver arithmetic on the stored value v = scale * sum (each optional):
   // v = ((v - sub[o]) * mul[o]) + beta * axz[o], o = output index
   const float* sub;
@@ -242,6 +244,7 @@ struct StackDst {
   const float* axz;
   float beta;
   FastDiv dP;  // division by the patches of the launch
+  const float* gs;  // device factor of scale (null: 1)
 };
 hipError_t launch_rows_c2r_stack(const Geo& g, const StackDst& k, const float2* tw, hipStream_t st);
 // The overlap-add and the stack of one two-adjoint call, in one launch where

@@ -763,6 +763,7 @@ constexpr int OLA_KJ = 8;  // output columns per thread of streamed launches (O1
 template <int TW, bool STREAM, bool WIN, int WGS>
 __device__ __forceinline__ void c2r_ola_body(Geo g, OlaDst d, int i, int fr, float2* dyn,
                                              const float2* __restrict__ tw) {
+  if (d.gs) d.scale *= d.gs[0];
   constexpr int TPT = TW / 16;
   constexpr int wgs = WGS;
   constexpr int TPW = WGS / TPT;
@@ -1023,6 +1024,7 @@ __device__ __forceinline__ void ola_epi_load(OlaEpi& E, const OlaDst& d, int i, 
 template <int TW, bool WGT>
 __device__ __forceinline__ void c2r_sum_body(Geo g, OlaDst d, int i0, int fr, float2* dyn,
                                              const float2* __restrict__ tw) {
+  if (d.gs) d.scale *= d.gs[0];
   constexpr int TPT = TW / 16;
   constexpr int SL = FftLds<TW>::floats2;
   const int R = d.sumr;
@@ -1487,7 +1489,7 @@ __device__ __forceinline__ void c2r_stack_body(Geo g, const StackDst& k, const f
   float* __restrict__ out = k.out;
   const float* __restrict__ axz = k.axz;
   const int srow = k.srow, nrows = k.nrows, ncols = k.ncols;
-  const float scale = k.scale, beta = k.beta;
+  const float scale = k.gs ? k.scale * k.gs[0] : k.scale, beta = k.beta;
   constexpr int TPT = TW / 16;
   constexpr int TPW = WG / TPT;
   constexpr int SL = FftLds<TW>::floats2;

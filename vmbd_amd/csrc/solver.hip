@@ -8,6 +8,7 @@
 // shuffles (DPP/permute through __shfl_xor) and one LDS exchange per wave.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <initializer_list>
 #include <mutex>
@@ -324,45 +325,101 @@ __device__ __forceinline__ float tv_norm(const float* s, int H, int W, int i, in
   return sqrtf(a * a + b * b + eps2);
 }
 
-__global__ __launch_bounds__(TB) void k_tv_value(const float* x, long long n, int H, int W, float eps2,
-                                                 double* partials) {
-  double v[1] = {0.0};
-  const long long HW = (long long)H * W;
-  for (long long e = (long long)blockIdx.x * TB + threadIdx.x; e < n; e += (long long)gridDim.x * TB) {
-    const long long k = e / HW;
-    const int r = (int)(e - k * HW);
-    const int i = r / W, j = r - (r / W) * W;
-    float a, b;
-    v[0] += (double)tv_norm(x + k * HW, H, W, i, j, eps2, &a, &b);
+// This block's share of the TV sum: whole image rows, blocks taking every
+// gridDim-th, so that a row's images and index divisions are once per row
+// (one per pixel, they and 64-bit addresses were most of the kernel) and four
+// pixels per thread are in flight.
+__device__ __forceinline__ double tv_rows(const float* __restrict__ x, long long rows, int H, int W, float eps2) {
+  double v = 0.0;
+  for (long long rho = blockIdx.x; rho < rows; rho += gridDim.x) {
+    const int i = (int)(rho % H);
+    const float* s = x + rho * W;
+    const bool down = i + 1 < H;
+    for (int j0 = threadIdx.x; j0 < W; j0 += 4 * TB) {
+      float c[4], r[4], d[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int j = min(j0 + e * TB, W - 1);
+        c[e] = s[j];
+        r[e] = s[min(j + 1, W - 1)];
+        d[e] = down ? s[j + W] : c[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float a = r[e] - c[e], b = d[e] - c[e];
+        if (j0 + e * TB < W) v += (double)sqrtf(a * a + b * b + eps2);
+      }
+    }
   }
+  return v;
+}
+
+__global__ __launch_bounds__(TB) void k_tv_value(const float* x, long long rows, int H, int W, float eps2,
+                                                 double* partials) {
+  double v[1] = {tv_rows(x, rows, H, W, eps2)};
   block_sum<1>(v);
   if (threadIdx.x == 0) partials[blockIdx.x] = v[0];
 }
 
+// partials of sum r^2 and (rows > 0) of the TV sum, one launch for both
+__global__ __launch_bounds__(TB) void k_loss_partials(const float* __restrict__ r, long long n, long long n4,
+                                                      const float* x, long long rows, int H, int W, float eps2,
+                                                      double* partials) {
+  double v[2] = {0.0, 0.0};
+  const long long stride = (long long)gridDim.x * TB;
+  const long long tid = (long long)blockIdx.x * TB + threadIdx.x;
+  const float4* r4 = (const float4*)r;
+  for (long long e = tid; e < n4; e += 2 * stride) {
+    const float4 a = r4[e];
+    const float4 b = e + stride < n4 ? r4[e + stride] : make_float4(0.f, 0.f, 0.f, 0.f);
+    v[0] += (double)a.x * a.x + (double)a.y * a.y + (double)a.z * a.z + (double)a.w * a.w;
+    v[0] += (double)b.x * b.x + (double)b.y * b.y + (double)b.z * b.z + (double)b.w * b.w;
+  }
+  for (long long e = 4 * n4 + tid; e < n; e += stride) v[0] += (double)r[e] * r[e];
+  if (rows) v[1] = tv_rows(x, rows, H, W, eps2);
+  block_sum<2>(v);
+  if (threadIdx.x == 0) {
+    partials[blockIdx.x] = v[0];
+    partials[gridDim.x + blockIdx.x] = v[1];
+  }
+}
+
+__global__ __launch_bounds__(TB) void k_loss_out(const double* partials, int nb, double lam, float* out) {
+  double s[2];
+  reduce_partials<2>(partials, nb, s);
+  if (threadIdx.x == 0) *out = (float)(0.5 * s[0] + (lam != 0.0 ? lam * s[1] : 0.0));
+}
+
 // grad (+)= weight * scale[0] * dTV/dx:
 //   dTV/dx_ij = -(dx_ij + dy_ij)/n_ij + dx_{i,j-1}/n_{i,j-1} + dy_{i-1,j}/n_{i-1,j}
-__global__ __launch_bounds__(TB) void k_tv_grad(float* grad, const float* x, long long n, int H, int W, float eps2,
+// One pixel per thread in 64 x 4 tiles, its seven neighbours through the L1:
+// the kernel is bound by its three square roots and divisions per pixel once
+// enough wavefronts are in flight (a grid of 512 blocks with the pixel's
+// position from two divisions took 16 us for 1024^2, this 8).
+__global__ __launch_bounds__(TB) void k_tv_grad(float* grad, const float* x, int K, int H, int W, float eps2,
                                                 const float* scale, float weight, int accumulate) {
   const float w = weight * (scale ? scale[0] : 1.f);
-  const long long HW = (long long)H * W;
-  for (long long e = (long long)blockIdx.x * TB + threadIdx.x; e < n; e += (long long)gridDim.x * TB) {
-    const long long k = e / HW;
-    const int r = (int)(e - k * HW);
-    const int i = r / W, j = r - (r / W) * W;
-    const float* s = x + k * HW;
-    float a, b;
-    const float nc = tv_norm(s, H, W, i, j, eps2, &a, &b);
-    float gv = -(a + b) / nc;
-    if (j > 0) {
-      const float nl = tv_norm(s, H, W, i, j - 1, eps2, &a, &b);
-      gv += a / nl;
+  const int j = blockIdx.x * 64 + (threadIdx.x & 63);
+  if (j >= W) return;
+  for (int k = blockIdx.z; k < K; k += gridDim.z) {
+    const float* s = x + (long long)k * H * W;
+    float* gr = grad + (long long)k * H * W;
+    for (int i = blockIdx.y * 4 + (threadIdx.x >> 6); i < H; i += gridDim.y * 4) {
+      float a, b;
+      const float nc = tv_norm(s, H, W, i, j, eps2, &a, &b);
+      float gv = -(a + b) / nc;
+      if (j > 0) {
+        const float nl = tv_norm(s, H, W, i, j - 1, eps2, &a, &b);
+        gv += a / nl;
+      }
+      if (i > 0) {
+        const float nu = tv_norm(s, H, W, i - 1, j, eps2, &a, &b);
+        gv += b / nu;
+      }
+      gv *= w;
+      const long long e = (long long)i * W + j;
+      gr[e] = accumulate ? gr[e] + gv : gv;
     }
-    if (i > 0) {
-      const float nu = tv_norm(s, H, W, i - 1, j, eps2, &a, &b);
-      gv += b / nu;
-    }
-    gv *= w;
-    grad[e] = accumulate ? grad[e] + gv : gv;
   }
 }
 
@@ -566,7 +623,7 @@ int vmbd_tv(const float* x, int32_t K, int32_t H, int32_t W, float eps, double* 
   const long long n = (long long)K * H * W;
   const int nb = grid_for(n);
   ProfScope ps("tv", st);
-  hipLaunchKernelGGL(k_tv_value, dim3(nb), dim3(TB), 0, st, x, n, H, W, eps * eps, partials);
+  hipLaunchKernelGGL(k_tv_value, dim3(nb), dim3(TB), 0, st, x, (long long)K * H, H, W, eps * eps, partials);
   hipLaunchKernelGGL(k_reduce_out, dim3(1), dim3(TB), 0, st, partials, nb, 1, value_out);
   SOLVER_DONE("vmbd_tv");
 }
@@ -576,11 +633,26 @@ int vmbd_tv_grad(float* grad, const float* x, int32_t K, int32_t H, int32_t W, f
   vmbd_clear_error();
   if (!grad || !x || K <= 0 || H <= 0 || W <= 0) return vmbd_fail(VMBD_E_ARG, "vmbd_tv_grad: bad argument");
   hipStream_t st = (hipStream_t)stream;
-  const long long n = (long long)K * H * W;
+  const dim3 grid((unsigned)((W + 63) / 64), (unsigned)std::min((H + 3) / 4, 65535), (unsigned)std::min(K, 65535));
   ProfScope ps("tv_grad", st);
-  hipLaunchKernelGGL(k_tv_grad, dim3(grid_for(n)), dim3(TB), 0, st, grad, x, n, H, W, eps * eps, scale, weight,
-                     accumulate);
+  hipLaunchKernelGGL(k_tv_grad, grid, dim3(TB), 0, st, grad, x, K, H, W, eps * eps, scale, weight, accumulate);
   SOLVER_DONE("vmbd_tv_grad");
+}
+
+int vmbd_loss(const float* r, int64_t nr, const float* x, int32_t K, int32_t H, int32_t W, float eps, float lam,
+              double* partials, float* value_out, vmbd_stream_t stream) {
+  vmbd_clear_error();
+  const bool tv = lam != 0.f;
+  if (!r || nr <= 0 || !partials || !value_out || (tv && (!x || K <= 0 || H <= 0 || W <= 0)))
+    return vmbd_fail(VMBD_E_ARG, "vmbd_loss: bad argument");
+  hipStream_t st = (hipStream_t)stream;
+  const long long n = tv ? (long long)K * H * W : 0;
+  const int nb = grid_for(std::max<long long>(nr, n));
+  ProfScope ps("loss", st);
+  hipLaunchKernelGGL(k_loss_partials, dim3(nb), dim3(TB), 0, st, r, (long long)nr, vec4_chunks(nr, {r}), x,
+                     tv ? (long long)K * H : 0LL, H, W, eps * eps, partials);
+  hipLaunchKernelGGL(k_loss_out, dim3(1), dim3(TB), 0, st, partials, nb, (double)lam, value_out);
+  SOLVER_DONE("vmbd_loss");
 }
 
 int vmbd_rl_update(float* x, const float* num, const float* den, int32_t H, int32_t W, float tol, int32_t border0,

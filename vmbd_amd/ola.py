@@ -201,13 +201,17 @@ class OlaPlan:
                 and kst == torch.cuda.current_stream().cuda_stream)
 
     # -- operators ----------------------------------------------------------
-    def forward(self, x, f, out=None):
+    def forward(self, x, f, out=None, sub=None):
+        """B(x, f); with `sub` (shaped like the result) B(x, f) - sub, formed
+        in the operator's final store."""
         (x, nx, bx), (f, nfr, bf) = self._x(x), self._f(f)
         nf, bat = self._same((nx, bx), (nfr, bf))
-        y = self._empty(self._lead(nf, bat) + self.sy, out)
+        shape = self._lead(nf, bat) + self.sy
+        sub = self._like(sub, shape, 'sub')
+        y = self._empty(shape, out)
         self._rows_key = None
-        _lib.check(_lib.lib().vmbd_ola_forward(self._h, nf, _lib.ptr(x), _lib.ptr(f), _lib.ptr(y),
-                                               _lib.stream_ptr()), 'forward')
+        _lib.check(_lib.lib().vmbd_ola_forward_ex(self._h, nf, _lib.ptr(x), _lib.ptr(f), _lib.ptr(sub), _lib.ptr(y),
+                                                  _lib.stream_ptr()), 'forward')
         self._rows_key = self._key(x, f, nf)
         return y
 
@@ -229,11 +233,17 @@ class OlaPlan:
                                                  int(bool(exact)), _lib.stream_ptr()), 'adjoint_f')
         return fb
 
-    def adjoint_xf(self, g, x, f, exact=True, out_x=None, out_f=None, reuse='auto'):
+    def adjoint_xf(self, g, x, f, exact=True, out_x=None, out_f=None, reuse='auto', scale=None):
+        """Both transposes of g; with `scale` (a one-element device tensor)
+        both are multiplied by it in their final stores."""
         (g, ng, bg), (x, nx, bx), (f, nfr, bf) = self._g(g), self._x(x), self._f(f)
         nf, bat = self._same((ng, bg), (nx, bx), (nfr, bf))
         xb = self._empty(self._lead(nf, bat) + self.sx, out_x)
         fb = self._empty(self._lead(nf, bat) + (self.P,) + self.sf, out_f)
+        if scale is not None:
+            scale = _as_dev(scale, self.device, 'scale')
+            if scale.numel() != 1:
+                raise ValueError('scale must have one element')
         flags = 0
         if reuse == 'auto':
             reuse = self._key_matches(x, f, nf)
@@ -241,9 +251,9 @@ class OlaPlan:
             flags |= _lib.REUSE_ROWS
         if not reuse:
             self._rows_key = None
-        _lib.check(_lib.lib().vmbd_ola_adjoint_xf(self._h, nf, _lib.ptr(g), _lib.ptr(x), _lib.ptr(f), _lib.ptr(xb),
-                                                  _lib.ptr(fb), int(bool(exact)), flags, _lib.stream_ptr()),
-                   'adjoint_xf')
+        _lib.check(_lib.lib().vmbd_ola_adjoint_xf_ex(self._h, nf, _lib.ptr(g), _lib.ptr(x), _lib.ptr(f),
+                                                     _lib.ptr(scale), _lib.ptr(xb), _lib.ptr(fb), int(bool(exact)),
+                                                     flags, _lib.stream_ptr()), 'adjoint_xf')
         # the workspaces now hold the row transforms of this x and f
         self._rows_key = self._key(x, f, nf)
         return xb, fb
