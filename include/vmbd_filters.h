@@ -59,6 +59,18 @@ int vmbd_shrink_alpha(float* y, int64_t n, float beta, float alpha, vmbd_stream_
 int vmbd_edgetaper(float* im, int32_t H, int32_t W, const float* wx, int32_t hx, const float* wy, int32_t hy,
                    vmbd_stream_t stream);
 
+/* vmbd_edgetaper with the tables of a PSF of s0 x s1 (gputools.py:651-659),
+ * computed on the host and passed as kernel arguments (no device tables, no
+ * copies).  VMBD_E_UNSUP when more than 128 rows or columns are tapered. */
+int vmbd_edgetaper_psf(float* im, int32_t H, int32_t W, int32_t s0, int32_t s1, vmbd_stream_t stream);
+
+/* The end of 'direct' (olaGPU.py:531-546) on images H x W: max(num, 0) over
+ * den tapered as by vmbd_edgetaper_psf and clipped to [0.01, 10]; of the
+ * result rows [o0, o0+m) and columns [o1, o1+n), replicated outwards to H x W
+ * with floor((H-m)/2) rows above and floor((W-n)/2) columns before them. */
+int vmbd_direct_ratio(float* out, const float* num, const float* den, int32_t H, int32_t W, int32_t s0, int32_t s1,
+                      int32_t o0, int32_t o1, int32_t m, int32_t n, vmbd_stream_t stream);
+
 /* Bilinear resampling of K slices H x W to OH x OW at normalised coordinates
  * (j/OW, i/OH), texel centres at +0.5, clamped addressing.  Replaces resize
  * (resize.cu:5-15, gputools.py:1205-1266). */

@@ -118,6 +118,8 @@ SIGNATURES = {
     'vmbd_shrink_alpha23': (ctypes.c_int, [_F, ctypes.c_int64, ctypes.c_float, _P]),
     'vmbd_shrink_alpha': (ctypes.c_int, [_F, ctypes.c_int64, ctypes.c_float, ctypes.c_float, _P]),
     'vmbd_edgetaper': (ctypes.c_int, [_F, _I, _I, _F, _I, _F, _I, _P]),
+    'vmbd_edgetaper_psf': (ctypes.c_int, [_F, _I, _I, _I, _I, _P]),
+    'vmbd_direct_ratio': (ctypes.c_int, [_F, _F, _F, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     'vmbd_resize': (ctypes.c_int, [_F, _I, _I, _F, _I, _I, _I, _P]),
     'vmbd_prof_enable': (ctypes.c_int, [_I]),
     'vmbd_prof_reset': (ctypes.c_int, []),

@@ -26,22 +26,53 @@ namespace {
 
 constexpr float SQRT1_2 = 0.70710678118654752440f;
 
-// 4 sin^2(pi q / T) = 2 - 2 cos(2 pi q / T), without the cancellation near 0
-__device__ __forceinline__ float four_sin2(int q, int T) {
-  const float s = sinpif((float)q / (float)T);
-  return 4.f * s * s;
+// Half the angle of a frequency q of T: sin and cos of pi q / T, 0 <= q <= T.
+// Everything the divisions need of a frequency follows from them:
+//   4 sin^2 (the filter energy 2 - 2 cos(2 pi q / T), without its cancellation
+//   near 0), (1 + 2 cos(2 pi q / T))^2 = (3 - 4 sin^2)^2, and the transform
+//   r (e^{-2 pi i q / T} - 1) = -2 r sin (sin + i cos) of the difference
+//   filter r [-1 1] at the tile origin, r = sqrt(2)/2.
+struct Half {
+  float s, c;
+};
+__device__ __forceinline__ Half half_tab(int q, int T, const float2* __restrict__ tw) {
+  const float2 w = tw[(q * (TW_LEN / 2 / T)) & (TW_LEN - 1)];
+  return Half{-w.y, w.x};
 }
-// (1 + 2 cos(2 pi q / T))^2
-__device__ __forceinline__ float one_2cos_sq(int q, int T) {
-  const float c = 1.f + 2.f * cospif(2.f * (float)q / (float)T);
+// The half angles of a thread's 16 frequencies k = t + TPT*m from two table
+// entries, by the sum of angles: pi k / T = pi t / T + pi m / 16 in the lower
+// half, and from the other end, pi (T - k) / T, in the upper (so that the
+// small sines of both ends come from small angles).  Sines and cosines per
+// frequency took half of the kernel.
+template <int TH>
+struct Halves {
+  Half lo, hi;
+  __device__ __forceinline__ Halves(int t, const float2* __restrict__ tw)
+      : lo(half_tab(t, TH, tw)), hi(half_tab(TH / 16 - t, TH, tw)) {}
+  __device__ __forceinline__ Half at(int m) const {
+    // sin and cos of pi j / 16
+    constexpr float S[8] = {0.f, 0.19509032201612826785f, 0.38268343236508977173f, 0.55557023301960222474f,
+                            0.70710678118654752440f, 0.83146961230254523708f, 0.92387953251128675613f,
+                            0.98078528040323044913f};
+    constexpr float C[8] = {1.f, 0.98078528040323044913f, 0.92387953251128675613f, 0.83146961230254523708f,
+                            0.70710678118654752440f, 0.55557023301960222474f, 0.38268343236508977173f,
+                            0.19509032201612826785f};
+    const bool up = m >= 8;
+    const int j = up ? 15 - m : m;
+    const Half b = up ? hi : lo;
+    if (j == 0) return Half{b.s, up ? -b.c : b.c};
+    const float s = fmaf(b.s, C[j], b.c * S[j]), c = fmaf(b.c, C[j], -(b.s * S[j]));
+    return Half{s, up ? -c : c};
+  }
+};
+__device__ __forceinline__ float four_sin2(Half h) { return 4.f * h.s * h.s; }
+__device__ __forceinline__ float one_2cos_sq(Half h) {
+  const float c = 3.f - four_sin2(h);
   return c * c;
 }
-// r (e^{-2 pi i q / T} - 1), r = sqrt(2)/2: the transform of the
-// difference filter r [-1 1] placed at the tile origin
-__device__ __forceinline__ float2 diff_filter(int q, int T) {
-  float s, c;
-  sincospif(2.f * (float)q / (float)T, &s, &c);
-  return make_float2(SQRT1_2 * (c - 1.f), -SQRT1_2 * s);
+__device__ __forceinline__ float2 diff_filter(Half h) {
+  const float a = -2.f * SQRT1_2 * h.s;
+  return make_float2(a * h.s, a * h.c);
 }
 
 __device__ __forceinline__ float cabs2(float2 a) { return fmaf(a.x, a.x, a.y * a.y); }
@@ -55,20 +86,20 @@ __device__ __forceinline__ void split(float2 p, float2 q, float2& d, float2& n) 
 __device__ __forceinline__ float2 join(float2 d, float2 n) { return make_float2(d.x - n.y, d.y + n.x); }
 
 // the division of one (row bin, column frequency) from its operand values
-// (order as in DivOp); cx = row bin, k = column frequency
+// (order as in DivOp); hx: row bin, hy: column frequency
 template <int OP>
-__device__ __forceinline__ float2 div_value(const float2 (&o)[4], int cx, int k, int Tw, int Th, DivParams p) {
+__device__ __forceinline__ float2 div_value(const float2 (&o)[4], Half hx, Half hy, DivParams p) {
   if constexpr (OP == DIV_X) {
-    const float L = four_sin2(cx, Tw) + four_sin2(k, Th);
+    const float L = four_sin2(hx) + four_sin2(hy);
     return cdivr(cmulc(o[0], o[1]), cabs2(o[1]) + p.alpha * L + p.beta);
   } else if constexpr (OP == DIV_G) {
-    const float L = one_2cos_sq(k, Th) * four_sin2(cx, Tw) + four_sin2(k, Th) * one_2cos_sq(cx, Tw);
+    const float L = one_2cos_sq(hy) * four_sin2(hx) + four_sin2(hy) * one_2cos_sq(hx);
     const float2 num = cadd(cmulc(o[1], o[0]), cmulc(o[3], o[2]));
     return cdivr(num, cabs2(o[0]) + cabs2(o[2]) + p.alpha * L + p.beta);
   } else if constexpr (OP == DIV_SPROD) {
     return cmulc(o[0], o[1]);
   } else {
-    const float2 gx = diff_filter(cx, Tw), gy = diff_filter(k, Th);
+    const float2 gx = diff_filter(hx), gy = diff_filter(hy);
     const float ab = p.alpha * p.beta;
     const float2 num = cadd(cadd(cmulc(o[0], gx), cmulc(o[1], gy)), cdivr(o[2], ab));
     return cdivr(num, cabs2(o[3]) / ab + cabs2(gx) + cabs2(gy) + p.gamma);
@@ -114,6 +145,8 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
   Twiddles<TH> T;
   twiddles_init<TH, true>(T, t, tw);
 
+  const Halves<TH> hy(t, tw);
+  const Half hx = half_tab(min(c, NB - 2), g.Tw, tw);
   const ColIn ins[4] = {a0, a1, a2, a3};
   // Operands are consumed one at a time: transformed (row-pass outputs) or
   // loaded (spectra), staged when the column is the packed one, and folded
@@ -141,9 +174,8 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
       const float ab = prm.alpha * prm.beta;
 #pragma unroll
       for (int m = 0; m < 16; ++m) {
-        const int k = t + TPT * m;
-        if (j == 0) num[m] = cmulc(v[m], diff_filter(c, g.Tw));
-        if (j == 1) num[m] = cadd(num[m], cmulc(v[m], diff_filter(k, g.Th)));
+        if (j == 0) num[m] = cmulc(v[m], diff_filter(hx));
+        if (j == 1) num[m] = cadd(num[m], cmulc(v[m], diff_filter(hy.at(m))));
         if (j == 2) num[m] = cadd(num[m], cdivr(v[m], ab));
         if (j == 3) acc[m] = make_float2(cabs2(v[m]) / ab, 0.f);
       }
@@ -166,7 +198,7 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
 #pragma unroll
         for (int m = 0; m < 16; ++m) {
           float2 ov[4] = {prev[m], v[m], make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
-          num[m] = div_value<OP>(ov, c, t + TPT * m, g.Tw, g.Th, prm);
+          num[m] = div_value<OP>(ov, hx, hy.at(m), prm);
         }
       }
     }
@@ -174,12 +206,12 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
   float2 Z[16];
 #pragma unroll
   for (int m = 0; m < 16; ++m) {
-    const int k = t + TPT * m;
     if constexpr (OP == DIV_S) {
-      const float2 gx = diff_filter(c, g.Tw), gy = diff_filter(k, g.Th);
+      const float2 gx = diff_filter(hx), gy = diff_filter(hy.at(m));
       Z[m] = cdivr(num[m], acc[m].x + cabs2(gx) + cabs2(gy) + prm.gamma);
     } else if constexpr (OP == DIV_G) {
-      const float L = one_2cos_sq(k, g.Th) * four_sin2(c, g.Tw) + four_sin2(k, g.Th) * one_2cos_sq(c, g.Tw);
+      const Half hk = hy.at(m);
+      const float L = one_2cos_sq(hk) * four_sin2(hx) + four_sin2(hk) * one_2cos_sq(hx);
       Z[m] = cdivr(num[m], acc[m].x + prm.alpha * L + prm.beta);
     } else {
       Z[m] = num[m];
@@ -199,7 +231,8 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
         od[j] = on[j] = make_float2(0.f, 0.f);
         if (j < NA) split(pk[j * SL + lds_pad(k)], pk[j * SL + lds_pad(kr)], od[j], on[j]);
       }
-      Z[m] = join(div_value<OP>(od, 0, k, g.Tw, g.Th, prm), div_value<OP>(on, g.Tw / 2, k, g.Tw, g.Th, prm));
+      // row bins 0 and Tw/2: half angles 0 and pi/2
+      Z[m] = join(div_value<OP>(od, Half{0.f, 1.f}, hy.at(m), prm), div_value<OP>(on, Half{1.f, 0.f}, hy.at(m), prm));
     }
   }
   if constexpr (OP == DIV_SPROD) {

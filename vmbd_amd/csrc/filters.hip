@@ -12,6 +12,9 @@
 // halo in LDS (121 taps per pixel).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
+
 #include "../../include/vmbd_filters.h"
 #include "capi_util.h"
 #include "prof.h"
@@ -242,6 +245,70 @@ __global__ __launch_bounds__(BX* BY) void k_edgetaper(float* im, int H, int W, c
   im[(long long)i * W + j] = v;
 }
 
+// The same taper with its tables as kernel arguments (tables computed per
+// call on the host need no copy to the device, which would wait for the
+// stream's earlier work).
+constexpr int TAPER_MAX = 128;
+struct TaperTab {
+  int hx, hy;
+  float wx[TAPER_MAX], wy[TAPER_MAX];
+};
+__device__ __forceinline__ float taper_at(const TaperTab& t, float v, int i, int j, int H, int W) {
+  if (i < t.hy) v *= t.wy[i];
+  else if (i > H - 1 - t.hy) v *= t.wy[H - 1 - i];
+  if (j < t.hx) v *= t.wx[j];
+  else if (j > W - 1 - t.hx) v *= t.wx[W - 1 - j];
+  return v;
+}
+__global__ __launch_bounds__(BX* BY) void k_edgetaper_tab(float* im, int H, int W, TaperTab t) {
+  const int i = blockIdx.y * BY + threadIdx.y, j = blockIdx.x * BX + threadIdx.x;
+  if (i >= H || j >= W) return;
+  if (!(i < t.hy || i > H - 1 - t.hy || j < t.hx || j > W - 1 - t.hx)) return;
+  im[(long long)i * W + j] = taper_at(t, im[(long long)i * W + j], i, j, H, W);
+}
+
+// The end of 'direct' (olaGPU.py:531-546) in one pass: max(num, 0) over the
+// tapered den clipped to [0.01, 10], its inner rows [o0, o0 + m) and columns
+// [o1, o1 + n) replicated outwards to H x W (p0, p1: first inner row and
+// column of the result).  As six passes it read and wrote the image eleven
+// times.
+__global__ __launch_bounds__(BX* BY) void k_direct_ratio(float* out, const float* num, const float* den, int H, int W,
+                                                         int o0, int o1, int m, int n, int p0, int p1, TaperTab t) {
+  const int i = blockIdx.y * BY + threadIdx.y, j = blockIdx.x * BX + threadIdx.x;
+  if (i >= H || j >= W) return;
+  const int si = o0 + min(max(i - p0, 0), m - 1), sj = o1 + min(max(j - p1, 0), n - 1);
+  float a = num[(long long)si * W + sj];
+  a = a < 0.f ? 0.f : a;
+  float d = taper_at(t, den[(long long)si * W + sj], si, sj, H, W);
+  d = d < 0.01f ? 0.01f : d;
+  d = d > 10.f ? 10.f : d;
+  out[(long long)i * W + j] = a / d;
+}
+
+// Taper tables of a PSF size (edgetaper_windows in gputools.py): the sizes
+// made odd, the rising halves of two Bartlett-Hann windows over the product
+// of their maxima.  False when they do not fit the kernel arguments.
+bool taper_tab(TaperTab& t, int s0, int s1) {
+  const int n1 = s1 + 1 - s1 % 2, n0 = s0 + 1 - s0 % 2;
+  t.hx = n1 / 2;
+  t.hy = n0 / 2;
+  if (s0 <= 0 || s1 <= 0 || t.hx > TAPER_MAX || t.hy > TAPER_MAX) return false;
+  auto win = [](int k, int n) {
+    if (n <= 1) return 1.0;
+    const double fac = std::fabs((double)k / (double)n - 0.5);
+    return 0.62 - 0.48 * fac + 0.38 * std::cos(2.0 * M_PI * fac);
+  };
+  auto top = [&](int n) {
+    double m = 0.0;
+    for (int k = 0; k < n; ++k) m = std::max(m, win(k, n));
+    return m;
+  };
+  const double mx = top(n1) * top(n0);
+  for (int k = 0; k < t.hx; ++k) t.wx[k] = (float)(win(k, n1) / mx);
+  for (int k = 0; k < t.hy; ++k) t.wy[k] = (float)(win(k, n0) / mx);
+  return true;
+}
+
 // resize.cu:5-15: sample at normalised (j/OW, i/OH) with bilinear filtering
 // and clamp addressing (texel centres at +0.5), per slice
 __global__ __launch_bounds__(BX* BY) void k_resize(float* out, int OH, int OW, const float* in, int H, int W) {
@@ -370,6 +437,34 @@ int vmbd_edgetaper(float* im, int32_t H, int32_t W, const float* wx, int32_t hx,
   ProfScope ps("edgetaper", st);
   hipLaunchKernelGGL(k_edgetaper, grid2(H, W), dim3(BX, BY), 0, st, im, H, W, wx, hx, wy, hy);
   FILT_DONE("vmbd_edgetaper");
+}
+
+int vmbd_edgetaper_psf(float* im, int32_t H, int32_t W, int32_t s0, int32_t s1, vmbd_stream_t stream) {
+  vmbd_clear_error();
+  TaperTab t;
+  if (!im || H <= 0 || W <= 0 || s0 <= 0 || s1 <= 0) return vmbd_fail(VMBD_E_ARG, "vmbd_edgetaper_psf: bad argument");
+  if (!taper_tab(t, s0, s1))
+    return vmbd_fail(VMBD_E_UNSUP, "vmbd_edgetaper_psf: %d x %d tapers more than %d rows or columns", s0, s1, TAPER_MAX);
+  hipStream_t st = (hipStream_t)stream;
+  ProfScope ps("edgetaper", st);
+  hipLaunchKernelGGL(k_edgetaper_tab, grid2(H, W), dim3(BX, BY), 0, st, im, H, W, t);
+  FILT_DONE("vmbd_edgetaper_psf");
+}
+
+int vmbd_direct_ratio(float* out, const float* num, const float* den, int32_t H, int32_t W, int32_t s0, int32_t s1,
+                      int32_t o0, int32_t o1, int32_t m, int32_t n, vmbd_stream_t stream) {
+  vmbd_clear_error();
+  TaperTab t;
+  if (!out || !num || !den || H <= 0 || W <= 0 || s0 <= 0 || s1 <= 0 || o0 < 0 || o1 < 0 || m <= 0 || n <= 0 ||
+      o0 + m > H || o1 + n > W)
+    return vmbd_fail(VMBD_E_ARG, "vmbd_direct_ratio: bad argument");
+  if (!taper_tab(t, s0, s1))
+    return vmbd_fail(VMBD_E_UNSUP, "vmbd_direct_ratio: %d x %d tapers more than %d rows or columns", s0, s1, TAPER_MAX);
+  hipStream_t st = (hipStream_t)stream;
+  ProfScope ps("direct_ratio", st);
+  hipLaunchKernelGGL(k_direct_ratio, grid2(H, W), dim3(BX, BY), 0, st, out, num, den, H, W, o0, o1, m, n, (H - m) / 2,
+                     (W - n) / 2, t);
+  FILT_DONE("vmbd_direct_ratio");
 }
 
 int vmbd_resize(float* out, int32_t OH, int32_t OW, const float* in, int32_t K, int32_t H, int32_t W,

@@ -325,9 +325,16 @@ def edgetaper_windows(shape, sf, win='barthann'):
     return (wx[:hsf[1]] / maxw).astype(np.float32), (wy[:hsf[0]] / maxw).astype(np.float32)
 
 
+TAPER_PSF_MAX = 256  # sizes whose tables the library passes as kernel arguments
+
+
 def edgetaper_gpu(y_gpu, sf, win='barthann'):
     """gputools.py:643-673: in-place border taper of width floor(sf/2)."""
     _inplace(y_gpu, 'edgetaper_gpu')
+    s0, s1 = _pair(sf)
+    if win == 'barthann' and 0 < s0 <= TAPER_PSF_MAX and 0 < s1 <= TAPER_PSF_MAX:
+        _lib.call('vmbd_edgetaper_psf', _p(y_gpu), y_gpu.shape[0], y_gpu.shape[1], s0, s1, _st())
+        return
     wx, wy = edgetaper_windows(y_gpu.shape, sf, win)
     dwx = torch.as_tensor(wx, device=y_gpu.device) if wx.size else None
     dwy = torch.as_tensor(wy, device=y_gpu.device) if wy.size else None

@@ -165,7 +165,10 @@ class OlaGPU:
         """olaGPU.py:315-736."""
         if not np.all(np.array(y.shape) == self.sy):
             raise IOError('Sizes incompatible. Expected blurred image!')
-        y_gpu = gputools._dev(y).clone()
+        # (the fused forms of these two only read it)
+        y_gpu = gputools._dev(y)
+        if not (self.fused and mode in ('xdirect', 'direct')):
+            y_gpu = y_gpu.clone()
         if mode == 'lbfgsb':
             return self._deconv_lbfgsb(y_gpu, z0, maxfun, alpha, beta, verbose, m)
         if mode == 'gdirect':
@@ -277,6 +280,8 @@ class OlaGPU:
         image, border re-padded."""
         const = torch.ones_like(y_gpu)
         yd = self.deconv(y_gpu, mode='xdirect', alpha=alpha, beta=beta, edgetapering=edgetapering)
+        if self.fused and yd.dim() == 2 and factor >= 1 and max(2 * self.sf) <= gputools.TAPER_PSF_MAX:
+            return self._direct_ratio(yd, const, alpha, beta, edgetapering, factor)
         gputools.cliplower_GPU(yd, 0)
         if edgetapering == 1:
             gputools.edgetaper_gpu(const, 2 * self.sf, 'barthann')
@@ -287,6 +292,21 @@ class OlaGPU:
         sz = np.array(yd.shape)
         yd = gputools.crop_gpu2cpu(yd, sz - factor * self.sf - 1, offset=np.floor((factor * self.sf - 1) / 2.))
         return gputools.impad_gpu(yd, tuple(sz - np.array(yd.shape)))
+
+    def _direct_ratio(self, yd, const, alpha, beta, edgetapering, factor):
+        """The rest of 'direct' for an image: the constant's deconvolution,
+        then the clipped ratio and its re-padded border in one pass."""
+        if edgetapering == 1:
+            gputools.edgetaper_gpu(const, 2 * self.sf, 'barthann')
+        const = self.deconv(const, mode='xdirect', alpha=alpha, beta=beta, edgetapering=edgetapering)
+        H, W = (int(v) for v in yd.shape)
+        m, n = (int(v) for v in np.array(yd.shape) - factor * self.sf - 1)
+        o0, o1 = (int(v) for v in np.floor((factor * self.sf - 1) / 2.))
+        s0, s1 = (int(v) for v in 2 * self.sf)
+        out = torch.empty_like(yd)
+        _lib.call('vmbd_direct_ratio', _lib.ptr(out), _lib.ptr(yd), _lib.ptr(const), H, W, s0, s1, o0, o1, m, n,
+                  _lib.stream_ptr())
+        return out
 
     def _deconv_xdirect(self, y, y_gpu, alpha, beta, edgetapering):
         """olaGPU.py:550-609: one Fourier division per patch.  As in the
