@@ -192,8 +192,14 @@ def ptr(t):
 
 
 def stream_ptr(stream=None):
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    return ctypes.c_void_p(raw_stream() if stream is None else stream.cuda_stream)
+
+
+def raw_stream():
+    """The current stream of the current device as an integer (what
+    torch.cuda.current_stream().cuda_stream gives, without building a Stream
+    object: 0.3 us instead of 2.6, once per library call)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def prof_enable(on=True):

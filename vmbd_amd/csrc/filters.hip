@@ -91,42 +91,72 @@ __global__ __launch_bounds__(BX* BY) void k_bfilter(float* out, const float* a, 
 }
 
 // The same filter for a half size WR known at compile time (the MFBD prior's
-// w = 5): loops unrolled, the spatial factor folded into one exponent,
-// exp(-t) evaluated as the hardware 2^(-t log2 e), and the in-image test
-// only in workgroups whose window crosses the image border.  Same sums in
-// the same order as k_bfilter.
-template <int WR>
-__global__ __launch_bounds__(BX* BY) void k_bfilter_w(float* out, const float* a, int H, int W, float sd, float sr) {
-  extern __shared__ float tile[];
-  constexpr int TW = BX + 2 * WR, TH = BY + 2 * WR;
-  const int i0 = blockIdx.y * BY - WR, j0 = blockIdx.x * BX - WR;
-  for (int idx = threadIdx.y * BX + threadIdx.x; idx < TW * TH; idx += BX * BY) {
+// w = 5), R pixels of one column per thread, 64 columns x 4R rows per
+// workgroup: a column of 2 WR + R values is read from LDS once for its R
+// pixels, the spatial factor is folded into one exponent, exp(-t) evaluated as
+// the hardware 2^(-t log2 e).  Bound by VALU issue: five instructions and one
+// quarter-rate exponential per tap.  The in-image test is made only in
+// workgroups whose window crosses the image border, in code of its own: inside
+// one unrolled loop it was a branch per tap, 121 blocks that overlapped nothing
+// and 242 registers (two wavefronts per SIMD); 2048^2 took 229 us, this
+// 104.  Same sums in the same order as k_bfilter.
+constexpr int BFX = 64;
+template <int WR, int R, bool EDGE>
+__device__ __forceinline__ void bfilter_taps(const float* tc, int i0, int j, int H, int W, float kr, float kd,
+                                             float (&sw)[R], float (&acc)[R]) {
+  constexpr int TW = BFX + 2 * WR;
+  float c[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    c[q] = tc[q * TW];
+    sw[q] = acc[q] = 0.f;
+  }
+#pragma unroll 1
+  for (int x = -WR; x <= WR; ++x) {
+    if (EDGE && (j + x < 0 || j + x >= W)) continue;
+    float v[R + 2 * WR];
+#pragma unroll
+    for (int r = 0; r < R + 2 * WR; ++r) v[r] = tc[(r - WR) * TW + x];
+#pragma unroll
+    for (int y = -WR; y <= WR; ++y) {
+      const float sp = (float)(x * x + y * y) * kd;
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const float dv = v[q + y + WR] - c[q];
+        float wt = __builtin_amdgcn_exp2f(fmaf(dv * dv, kr, sp));
+        if (EDGE) wt = (i0 + q + y >= 0 && i0 + q + y < H) ? wt : 0.f;
+        sw[q] += wt;
+        acc[q] += wt * v[q + y + WR];
+      }
+    }
+  }
+}
+
+template <int WR, int R>
+__global__ __launch_bounds__(256) void k_bfilter_w(float* out, const float* a, int H, int W, float sd, float sr) {
+  constexpr int TW = BFX + 2 * WR, TH = 4 * R + 2 * WR;
+  __shared__ float tile[TW * TH];
+  const int ti0 = blockIdx.y * 4 * R - WR, tj0 = blockIdx.x * BFX - WR;
+  for (int idx = threadIdx.x; idx < TW * TH; idx += 256) {
     const int ti = idx / TW, tj = idx - (idx / TW) * TW;
-    const int ii = i0 + ti, jj = j0 + tj;
+    const int ii = ti0 + ti, jj = tj0 + tj;
     tile[idx] = (ii >= 0 && ii < H && jj >= 0 && jj < W) ? a[(long long)ii * W + jj] : 0.f;
   }
   __syncthreads();
-  const int i = blockIdx.y * BY + threadIdx.y, j = blockIdx.x * BX + threadIdx.x;
-  if (i >= H || j >= W) return;
-  const bool inner = i0 >= 0 && j0 >= 0 && i0 + TH <= H && j0 + TW <= W;  // uniform per workgroup
-  const float* tc = tile + (threadIdx.y + WR) * TW + threadIdx.x + WR;
-  const float c = tc[0];
+  const int lj = threadIdx.x & (BFX - 1), li = (int)(threadIdx.x / BFX) * R;
+  const int i0 = blockIdx.y * 4 * R + li, j = blockIdx.x * BFX + lj;
+  if (i0 >= H || j >= W) return;
+  const float* tc = tile + (li + WR) * TW + lj + WR;
   constexpr float LOG2E = 1.44269504088896340736f;
   const float kr = -LOG2E / (2.f * sr * sr), kd = -LOG2E / (2.f * sd * sd);
-  float sw = 0.f, acc = 0.f;
+  float sw[R], acc[R];
+  if (ti0 >= 0 && tj0 >= 0 && ti0 + TH <= H && tj0 + TW <= W)  // uniform per workgroup
+    bfilter_taps<WR, R, false>(tc, i0, j, H, W, kr, kd, sw, acc);
+  else
+    bfilter_taps<WR, R, true>(tc, i0, j, H, W, kr, kd, sw, acc);
 #pragma unroll
-  for (int x = -WR; x <= WR; ++x) {
-#pragma unroll
-    for (int y = -WR; y <= WR; ++y) {
-      const float v = tc[y * TW + x];
-      const float dv = v - c;
-      float wt = __builtin_amdgcn_exp2f(fmaf(dv * dv, kr, (float)(x * x + y * y) * kd));
-      if (!inner && !(i + y >= 0 && i + y < H && j + x >= 0 && j + x < W)) wt = 0.f;
-      sw += wt;
-      acc += wt * v;
-    }
-  }
-  out[(long long)i * W + j] = acc / sw;
+  for (int q = 0; q < R; ++q)
+    if (i0 + q < H) out[(long long)(i0 + q) * W + j] = acc[q] / sw[q];
 }
 
 #define SQRT2H 0.70710678118654752440f
@@ -359,8 +389,13 @@ int vmbd_bilateral(float* out, const float* in, int32_t H, int32_t W, int32_t w,
   hipStream_t st = (hipStream_t)stream;
   const size_t shm = (size_t)(BX + 2 * w) * (BY + 2 * w) * sizeof(float);
   ProfScope ps("bilateral", st);
-  if (w == 5)
-    hipLaunchKernelGGL(k_bfilter_w<5>, grid2(H, W), dim3(BX, BY), shm, st, out, in, H, W, sigma_d, sigma_r);
+  // four pixels per thread from two workgroups per CU on (at 512 x 1024 and
+  // above), one where that would leave CUs without work
+  const dim3 g4((W + BFX - 1) / BFX, (H + 15) / 16), g1((W + BFX - 1) / BFX, (H + 3) / 4);
+  if (w == 5 && (long long)g4.x * g4.y >= 512)
+    hipLaunchKernelGGL((k_bfilter_w<5, 4>), g4, dim3(256), 0, st, out, in, H, W, sigma_d, sigma_r);
+  else if (w == 5 && g1.y <= 65535)
+    hipLaunchKernelGGL((k_bfilter_w<5, 1>), g1, dim3(256), 0, st, out, in, H, W, sigma_d, sigma_r);
   else
     hipLaunchKernelGGL(k_bfilter, grid2(H, W), dim3(BX, BY), shm, st, out, in, H, W, w, sigma_d, sigma_r);
   FILT_DONE("vmbd_bilateral");

@@ -190,7 +190,7 @@ class OlaPlan:
         # tensors carry no version counter and are never reused
         if x.is_inference() or f.is_inference():
             return None
-        return (x, x._version, f, f._version, nf, torch.cuda.current_stream().cuda_stream)
+        return (x, x._version, f, f._version, nf, _lib.raw_stream())
 
     def _key_matches(self, x, f, nf):
         k = self._rows_key
@@ -198,7 +198,7 @@ class OlaPlan:
             return False
         kx, vx, kf, vf, knf, kst = k
         return (kx is x and kf is f and vx == x._version and vf == f._version and knf == nf
-                and kst == torch.cuda.current_stream().cuda_stream)
+                and kst == _lib.raw_stream())
 
     # -- operators ----------------------------------------------------------
     def forward(self, x, f, out=None, sub=None):
