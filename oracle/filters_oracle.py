@@ -69,6 +69,8 @@ def bilateral(a, w=5, sigma_d=3.0, sigma_r=0.1):
             sh = np.full((H, W), np.nan)
             i0, i1 = max(0, -dy), min(H, H - dy)
             j0, j1 = max(0, -dx), min(W, W - dx)
+            if i0 >= i1 or j0 >= j1:  # the neighbour lies outside for every pixel
+                continue
             sh[i0:i1, j0:j1] = a[i0 + dy:i1 + dy, j0 + dx:j1 + dx]
             ok = ~np.isnan(sh)
             v = np.where(ok, sh, 0.0)
