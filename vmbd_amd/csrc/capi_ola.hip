@@ -1236,7 +1236,7 @@ bool batch_group(BatchGroup& B, vmbd_plan* p, int nframes, const float* x, const
   bool ok = row_job(xr.shared ? B.rows_x : B.rows_fwd, xr.g, xr.s, p->wsX) && row_job(B.rows_fwd, g, sf, p->wsF);
   B.cf_a = xr.in;
   B.cf_b = raw_in(p->wsF, sf);
-  B.cf_o = ColOut{p->Y1, g.ext0};
+  B.cf_o = col_out_policy(g, ColOut{p->Y1, g.ext0});
   B.ola_fwd = dst_forward(p, y);
   ola_fit_rows(B.ola_fwd, (long long)B.ola_fwd.O0 * nframes);
   const SharedRows sr = residual_rows(p, g, gres, exact);
@@ -1244,8 +1244,8 @@ bool batch_group(BatchGroup& B, vmbd_plan* p, int nframes, const float* x, const
   B.ca_a = shared_in(p->wsG, sr);
   B.ca_b = raw_in(p->wsF, sf);
   B.ca_c = xr.in;
-  B.ca_o1 = ColOut{p->Y1, g.sw0};
-  B.ca_o2 = ColOut{p->Y2, g.sf0};
+  B.ca_o1 = col_out_policy(g, ColOut{p->Y1, g.sw0});
+  B.ca_o2 = col_out_policy(g, ColOut{p->Y2, g.sf0});
   B.ola_adj = dst_adjoint_x(p, xbar);
   ola_fit_rows(B.ola_adj, (long long)B.ola_adj.O0 * nframes);
   // the grouped OLA launch runs WG threads per workgroup for every group

@@ -4,6 +4,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "fft_core.h"
 #include "ola_kernels.h"
 
@@ -11,6 +13,17 @@ namespace vmbd {
 
 constexpr int WG = 256;
 constexpr int NXCD = 8;  // XCDs of an MI355X; workgroups are dealt to them round-robin
+
+// NT: a store for data that passes through memory once between two launches;
+// it leaves the L2 to the operands that are read again.
+typedef float float2_nt __attribute__((ext_vector_type(2)));
+template <bool NT>
+__device__ __forceinline__ void store_f2(float2* p, float2 v) {
+  if constexpr (NT)
+    __builtin_nontemporal_store((float2_nt){v.x, v.y}, (float2_nt*)p);
+  else
+    *p = v;
+}
 
 template <int A, int B>
 struct cmax {
@@ -158,22 +171,28 @@ __device__ __forceinline__ void col_store_rows(const float2 (&v)[16], float2* st
     const unsigned vo = (unsigned)(r0 * NBP + ci);
     const float2* sr = st + r0 * (CS + 1) + ci;
     const size_t step = (size_t)RS * NBP;
-    int k = 0;
-    // four steps of whole rows at a time, their LDS reads together
-    for (; k + 4 * RS <= nrows; k += 4 * RS) {
-      float2 x[4];
+    auto rows = [&](auto nt) {
+      int k = 0;
+      // four steps of whole rows at a time, their LDS reads together
+      for (; k + 4 * RS <= nrows; k += 4 * RS) {
+        float2 x[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = sr[i * RS * (CS + 1)];
+        for (int i = 0; i < 4; ++i) x[i] = sr[i * RS * (CS + 1)];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) (dst + i * step)[vo] = x[i];
-      dst += 4 * step;
-      sr += 4 * RS * (CS + 1);
-    }
-    for (; k < nrows; k += RS) {
-      if (k + r0 < nrows) dst[vo] = sr[0];
-      dst += step;
-      sr += RS * (CS + 1);
-    }
+        for (int i = 0; i < 4; ++i) store_f2<decltype(nt)::value>(dst + i * step + vo, x[i]);
+        dst += 4 * step;
+        sr += 4 * RS * (CS + 1);
+      }
+      for (; k < nrows; k += RS) {
+        if (k + r0 < nrows) store_f2<decltype(nt)::value>(dst + vo, sr[0]);
+        dst += step;
+        sr += RS * (CS + 1);
+      }
+    };
+    if (o.nt)
+      rows(std::true_type{});
+    else
+      rows(std::false_type{});
   }
   if (!LAST) __syncthreads();  // staging drained before the slices are reused
 }

@@ -260,21 +260,22 @@ hipError_t cols_div_t(const Geo& g, int op, const ColIn* a, DivParams prm, const
   const dim3 grid((unsigned)strips, (unsigned)g.Pf, (unsigned)(g.P / g.Pf));
   static const char* names[4] = {"cols_div_x", "cols_div_g", "cols_sprod", "cols_div_s"};
   ProfScope ps(names[op & 3], st);
+  const ColOut po = col_out_policy(g, o);
   switch (op) {
     case DIV_X:
-      hipLaunchKernelGGL((k_cols_div<TH, DIV_X>), grid, dim3(WG), 0, st, g, a[0], a[1], a[2], a[3], prm, o,
+      hipLaunchKernelGGL((k_cols_div<TH, DIV_X>), grid, dim3(WG), 0, st, g, a[0], a[1], a[2], a[3], prm, po,
                          spec_out, tw);
       break;
     case DIV_G:
-      hipLaunchKernelGGL((k_cols_div<TH, DIV_G>), grid, dim3(WG), 0, st, g, a[0], a[1], a[2], a[3], prm, o,
+      hipLaunchKernelGGL((k_cols_div<TH, DIV_G>), grid, dim3(WG), 0, st, g, a[0], a[1], a[2], a[3], prm, po,
                          spec_out, tw);
       break;
     case DIV_SPROD:
-      hipLaunchKernelGGL((k_cols_div<TH, DIV_SPROD>), grid, dim3(WG), 0, st, g, a[0], a[1], a[2], a[3], prm, o,
+      hipLaunchKernelGGL((k_cols_div<TH, DIV_SPROD>), grid, dim3(WG), 0, st, g, a[0], a[1], a[2], a[3], prm, po,
                          spec_out, tw);
       break;
     case DIV_S:
-      hipLaunchKernelGGL((k_cols_div<TH, DIV_S>), grid, dim3(WG), 0, st, g, a[0], a[1], a[2], a[3], prm, o,
+      hipLaunchKernelGGL((k_cols_div<TH, DIV_S>), grid, dim3(WG), 0, st, g, a[0], a[1], a[2], a[3], prm, po,
                          spec_out, tw);
       break;
     default:

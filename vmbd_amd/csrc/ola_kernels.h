@@ -136,7 +136,21 @@ struct ColCtx {
 struct ColOut {
   float2* p;
   int nrows;
+  bool nt = false;  // set by col_out_policy
 };
+
+// Outputs of 4 MB and more (one die's L2) are stored nontemporally: the next
+// launch reads them once, and the write-back then does not push the operand
+// rows out.  Below, the next launch finds the rows in the caches and the
+// stores stay plain.  Measured, plain / nontemporal: 1024^2, 10 x 10 patches,
+// 41^2 PSFs, 32 frames (816 MB) 1360 / 1326 us for the whole step, the PSF
+// gradient of one such frame 53.1 / 52.0 us, 2048^2 with 63^2 PSFs 350 / 343
+// us; 256^2 frames of 0.2 to 1 MB 18.4 / 18.7 and 32.2 / 32.8 us.
+constexpr size_t COL_NT_BYTES = (size_t)4 << 20;
+inline ColOut col_out_policy(const Geo& g, ColOut o) {
+  o.nt = (size_t)g.P * o.nrows * g.NBP * sizeof(float2) >= COL_NT_BYTES;
+  return o;
+}
 
 // Inverse row transform + overlap-add gather + crop into an output image.
 // Output pixel (i, j) sums, over every patch k whose local extent covers the
