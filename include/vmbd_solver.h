@@ -81,6 +81,15 @@ int vmbd_pbb_step_noalloc(float* xnew, const float* x, const float* oldx, const 
 int vmbd_pbb_select(float* x, float* oldx, float* g, float* oldg, int64_t n, const double* dots, double beta,
                     vmbd_stream_t stream);
 
+/* The start of PBB from the points' residuals: vmbd_pbb_start forms the second
+ * point, y = (u - x) - 0.5; vmbd_pbb_choose takes the four squared norms as
+ * vmbd_dot sums them (r, oldr: the m residuals at x and oldx) and then does
+ * what vmbd_pbb_select does.  partials: 4 * vmbd_reduce_blocks(max(n, m))
+ * doubles of scratch. */
+int vmbd_pbb_start(float* y, const float* u, const float* x, int64_t n, vmbd_stream_t stream);
+int vmbd_pbb_choose(float* x, float* oldx, float* g, float* oldg, int64_t n, const float* r, const float* oldr,
+                    int64_t m, double beta, double* partials, vmbd_stream_t stream);
+
 /* out = a*s + b*t (b may be NULL). */
 int vmbd_axpby(float* out, const float* a, float s, const float* b, float t, int64_t n, vmbd_stream_t stream);
 /* Elementwise family: out = a*b, a/b, s/a, a-b, a + s*b or s*a (op

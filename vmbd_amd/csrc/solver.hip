@@ -33,7 +33,7 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-// block sum of up to 3 values (double accumulation), result valid in thread 0
+// block sum of K values (double accumulation), result valid in thread 0
 template <int K>
 __device__ __forceinline__ void block_sum(double (&v)[K]) {
   __shared__ double sh[K][TB / 64];
@@ -228,6 +228,60 @@ __global__ __launch_bounds__(TB) void k_pbb_select(float* x, float* oldx, float*
   const double fx = 0.5 * dots[0] + 0.5 * beta * dots[1];
   const double fy = 0.5 * dots[2] + 0.5 * beta * dots[3];
   if (fx < fy) return;
+  for (long long e = (long long)blockIdx.x * TB + threadIdx.x; e < n; e += (long long)gridDim.x * TB) {
+    const float a = x[e], b = g[e];
+    x[e] = oldx[e];
+    oldx[e] = a;
+    g[e] = oldg[e];
+    oldg[e] = b;
+  }
+}
+
+// The second start point of PBB: y = u - (x + 0.5) as (u - x) - 0.5.
+__global__ __launch_bounds__(TB) void k_pbb_start(float* y, const float* u, const float* x, long long n) {
+  for (long long e = (long long)blockIdx.x * TB + threadIdx.x; e < n; e += (long long)gridDim.x * TB)
+    y[e] = u[e] - x[e] - 0.5f;
+}
+
+// PBB start in two launches, each bound by its latency (4 to 5 us): the four
+// squared norms' partials side by side (blockIdx.y), then the selection, where
+// every block adds up the partials in one order (same decision everywhere).
+// An online frame of 512^2 with 64 31^2 PSFs, four iterations of each solver,
+// took 684 us with four dots of two launches each and k_pbb_select, 648 so.
+// The sums and their order are those of vmbd_dot.
+struct PbbDots {
+  const float* v[4];  // r and z at the first point, then at the second
+  long long n[4];
+  int nb[4];          // blocks, and partials, of each
+};
+__global__ __launch_bounds__(TB) void k_pbb_dots(PbbDots d, double* partials, int pitch) {
+  const int k = blockIdx.y;
+  const int nb = d.nb[k];
+  if ((int)blockIdx.x >= nb) return;
+  const float* a = d.v[k];
+  const long long n = d.n[k];
+  double v[1] = {0.0};
+  for (long long e = (long long)blockIdx.x * TB + threadIdx.x; e < n; e += (long long)nb * TB)
+    v[0] += (double)a[e] * (double)a[e];
+  block_sum<1>(v);
+  if (threadIdx.x == 0) partials[(long long)k * pitch + blockIdx.x] = v[0];
+}
+
+__global__ __launch_bounds__(TB) void k_pbb_choose(float* x, float* oldx, float* g, float* oldg, long long n,
+                                                   const double* partials, int pitch, int nbr, int nbz, double beta) {
+  double dots[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int nb = k & 1 ? nbz : nbr;
+    dots[k] = 0.0;
+    for (int i = threadIdx.x; i < nb; i += TB) dots[k] += partials[(long long)k * pitch + i];
+  }
+  block_sum<4>(dots);
+  __shared__ int keep;
+  if (threadIdx.x == 0)
+    keep = 0.5 * dots[0] + 0.5 * beta * dots[1] < 0.5 * dots[2] + 0.5 * beta * dots[3];
+  __syncthreads();
+  if (keep) return;
   for (long long e = (long long)blockIdx.x * TB + threadIdx.x; e < n; e += (long long)gridDim.x * TB) {
     const float a = x[e], b = g[e];
     x[e] = oldx[e];
@@ -581,6 +635,30 @@ int vmbd_pbb_select(float* x, float* oldx, float* g, float* oldg, int64_t n, con
   ProfScope ps("pbb_select", st);
   hipLaunchKernelGGL(k_pbb_select, dim3(grid_for(n)), dim3(TB), 0, st, x, oldx, g, oldg, (long long)n, dots, beta);
   SOLVER_DONE("vmbd_pbb_select");
+}
+
+int vmbd_pbb_start(float* y, const float* u, const float* x, int64_t n, vmbd_stream_t stream) {
+  vmbd_clear_error();
+  if (!y || !u || !x || n <= 0) return vmbd_fail(VMBD_E_ARG, "vmbd_pbb_start: bad argument");
+  hipStream_t st = (hipStream_t)stream;
+  ProfScope ps("pbb_start", st);
+  hipLaunchKernelGGL(k_pbb_start, dim3(grid_for(n)), dim3(TB), 0, st, y, u, x, (long long)n);
+  SOLVER_DONE("vmbd_pbb_start");
+}
+
+int vmbd_pbb_choose(float* x, float* oldx, float* g, float* oldg, int64_t n, const float* r, const float* oldr,
+                    int64_t m, double beta, double* partials, vmbd_stream_t stream) {
+  vmbd_clear_error();
+  if (!x || !oldx || !g || !oldg || !r || !oldr || !partials || n <= 0 || m <= 0)
+    return vmbd_fail(VMBD_E_ARG, "vmbd_pbb_choose: bad argument");
+  hipStream_t st = (hipStream_t)stream;
+  const int nbr = grid_for(m), nbz = grid_for(n), pitch = nbr > nbz ? nbr : nbz;
+  const PbbDots d{{r, x, oldr, oldx}, {m, n, m, n}, {nbr, nbz, nbr, nbz}};
+  ProfScope ps("pbb_choose", st);
+  hipLaunchKernelGGL(k_pbb_dots, dim3(pitch, 4), dim3(TB), 0, st, d, partials, pitch);
+  hipLaunchKernelGGL(k_pbb_choose, dim3(grid_pbb(n)), dim3(TB), 0, st, x, oldx, g, oldg, (long long)n, partials, pitch,
+                     nbr, nbz, beta);
+  SOLVER_DONE("vmbd_pbb_choose");
 }
 
 int vmbd_axpby(float* out, const float* a, float s, const float* b, float t, int64_t n, vmbd_stream_t stream) {

@@ -32,7 +32,6 @@ synchronisation; ``capture=True`` records it once in a HIP graph and replays
 it for every frame (the random second start points are drawn before each
 replay).  The latent image and the PSFs stay on the device between frames.
 """
-import ctypes
 
 import numpy as np
 import torch
@@ -125,15 +124,16 @@ class OnlineMFBD:
         self.y = torch.zeros(self.sy, dtype=f32, device=d)
         self.mask = torch.zeros(self.sy, dtype=f32, device=d)
         self.ym = torch.zeros(self.sy, dtype=f32, device=d)
+        # residuals: the last gradient's, and the start pair's second
         self.r = torch.zeros(self.sy, dtype=f32, device=d)
+        self.r2 = torch.zeros(self.sy, dtype=f32, device=d)
         self.specX = torch.zeros(spec_shape, dtype=torch.complex64, device=d)
         self.specF = torch.zeros(spec_shape, dtype=torch.complex64, device=d)
-        self.dots = torch.zeros(4, dtype=torch.float64, device=d)
         nf = int(np.prod(fshape))
         nx = self.sx[0] * self.sx[1]
         self.sc_f = _Scratch(nf, d)
         self.sc_x = _Scratch(nx, d)
-        self.dot_part = torch.zeros(3 * _lib.lib().vmbd_reduce_blocks(max(nf, nx, self.sy[0] * self.sy[1])),
+        self.dot_part = torch.zeros(4 * _lib.lib().vmbd_reduce_blocks(max(nf, nx, self.sy[0] * self.sy[1])),
                                     dtype=torch.float64, device=d)
         self.fz = [torch.zeros(fshape, dtype=f32, device=d) for _ in range(4)]     # z, oldz, g, oldg
         self.fu = torch.zeros(fshape, dtype=f32, device=d)
@@ -152,44 +152,35 @@ class OnlineMFBD:
         _lib.call('vmbd_ew', _lib.ptr(out), _lib.ptr(a), _lib.ptr(b), float(s), a.numel(), int(op),
                   _lib.stream_ptr())
 
-    def _dot(self, a, b, slot):
-        out = ctypes.c_void_p(self.dots.data_ptr() + slot * self.dots.element_size())
-        _lib.call('vmbd_dot', _lib.ptr(a), _lib.ptr(b), a.numel(), _lib.ptr(self.dot_part), out, _lib.stream_ptr())
-
-    def _grad_f(self, z, out, dots_at=None):
-        """out = X'(X z - y) + beta z (X: cached image spectra); the residual
-        and the Tikhonov term are formed in the operators' final stores."""
+    def _grad_f(self, z, out, r):
+        """r = X z - y, out = X'r + beta z (X: cached image spectra); the
+        residual and the Tikhonov term are formed in the operators' final
+        stores."""
         p = self.plan
-        p.forward_cached('X', self.specX, z, out=self.r, sub=self.y)
-        p.adjoint_cached('X', self.specX, self.r, exact=self.exact, out=out,
+        p.forward_cached('X', self.specX, z, out=r, sub=self.y)
+        p.adjoint_cached('X', self.specX, r, exact=self.exact, out=out,
                          z=z if self.f_beta != 0. else None, beta=self.f_beta)
-        if dots_at is not None:
-            self._dot(self.r, self.r, dots_at)
-            self._dot(z, z, dots_at + 1)
 
-    def _grad_x(self, z, out, dots_at=None):
-        """out = F'(mask (F z - y)) (F: cached PSF spectra)."""
+    def _grad_x(self, z, out, r):
+        """r = mask (F z - y), out = F'r (F: cached PSF spectra)."""
         p = self.plan
-        p.forward_cached('F', self.specF, z, out=self.r, sub=self.y, mul=self.mask)
-        p.adjoint_cached('F', self.specF, self.r, exact=self.exact, out=out)
-        if dots_at is not None:
-            self._dot(self.r, self.r, dots_at)
-            self._dot(z, z, dots_at + 1)
+        p.forward_cached('F', self.specF, z, out=r, sub=self.y, mul=self.mask)
+        p.adjoint_cached('F', self.specF, r, exact=self.exact, out=out)
 
     def _pbb(self, grad, z, oldz, g, oldg, u, iters, beta, sc):
         """optGPU.PBB with a fixed iteration count: start pair (z, u - (z + 0.5)),
         the better one becomes the iterate (on the device), then `iters`
         projected BB steps.  Returns the buffer holding the final iterate."""
-        self._ew(gputools.EW_SUB, oldz, u, z)
-        self._ew(gputools.EW_ADDS, oldz, oldz, None, -0.5)
-        grad(z, g, dots_at=0)
-        grad(oldz, oldg, dots_at=2)
-        _lib.call('vmbd_pbb_select', _lib.ptr(z), _lib.ptr(oldz), _lib.ptr(g), _lib.ptr(oldg), z.numel(),
-                  _lib.ptr(self.dots), float(beta), _lib.stream_ptr())
+        st = _lib.stream_ptr()
+        _lib.call('vmbd_pbb_start', _lib.ptr(oldz), _lib.ptr(u), _lib.ptr(z), z.numel(), st)
+        grad(z, g, self.r)
+        grad(oldz, oldg, self.r2)
+        _lib.call('vmbd_pbb_choose', _lib.ptr(z), _lib.ptr(oldz), _lib.ptr(g), _lib.ptr(oldg), z.numel(),
+                  _lib.ptr(self.r), _lib.ptr(self.r2), self.r.numel(), float(beta), _lib.ptr(self.dot_part), st)
         for it in range(1, iters + 1):
             pbb_step(z, oldz, g, oldg, it, oldz, sc)      # new iterate overwrites oldz
             z, oldz = oldz, z
-            grad(z, oldg)                                # new gradient overwrites oldg
+            grad(z, oldg, self.r)                        # new gradient overwrites oldg
             g, oldg = oldg, g
         return z
 
@@ -244,7 +235,8 @@ class OnlineMFBD:
     def _frame_body(self):
         # vmbd_chimney.py:117-118: mask = 1. * (y < 1)
         self._ew(gputools.EW_LT, self.mask, self.y, None, 1.0)
-        self._ew(gputools.EW_MUL, self.ym, self.mask, self.y)
+        if self.x_solver == 'rl':
+            self._ew(gputools.EW_MUL, self.ym, self.mask, self.y)
         if self.f_solver == 'pbb':
             self._f_step_device()
         else:
