@@ -20,7 +20,8 @@ launch forms:
   Groups whose image rows are shared per patch column (separable windows,
   the default, at launches that fill the GPU) transform them in a row pass
   of their own.
-* ``grouped=False``: the groups' own launches, seven per group; with
+* ``grouped=False``: the groups' own launches, seven passes per group (the
+  overlap-add of the x-adjoint and the stack in one launch); with
   ``streams=k > 1`` (default 3) ``capture()`` forks the groups over k
   streams inside the graph (largest groups first, each to the stream with
   the fewest pixels so far) so that one group's launches fill the tail of
@@ -135,7 +136,7 @@ class MixedBatch:
 
     @property
     def launches(self):
-        """Kernel launches per step."""
+        """Kernel launches per step (passes, without grouping)."""
         if self.grouped:
             return sum(int(_lib.lib().vmbd_batch_launches(vb)) for vb in self._batches().values())
         return 7 * len(self.groups)
