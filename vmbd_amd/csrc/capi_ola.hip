@@ -531,7 +531,7 @@ vmbd_plan* vmbd_plan_create(const vmbd_geom* gm, const float* win_table, int32_t
   }
   size_t tot = 0;
   const size_t P = (size_t)g.Pf * p->max_frames, NB = g.NB, NBP = g.NBP;
-  bool ok = dev_alloc(&p->tw, TW_LEN, tot) && dev_alloc(&p->win, (size_t)n_win * g.sw0 * g.sw1, tot) &&
+  bool ok = dev_alloc(&p->tw, TW_PLAN, tot) && dev_alloc(&p->win, (size_t)n_win * g.sw0 * g.sw1, tot) &&
             dev_alloc(&p->win_idx, g.Pf, tot) && dev_alloc(&p->wsG, (size_t)p->max_frames * g.csf1 * NB * row_pitch(residual_virtual_rows(g, g.ext0)), tot) &&
             dev_alloc(&p->wsX, P * NB * row_pitch(g.sw0), tot) && dev_alloc(&p->wsF, P * NB * row_pitch(g.sf0), tot) &&
             dev_alloc(&p->Y1, P * NBP * g.ext0, tot) && dev_alloc(&p->Y2, P * NBP * g.sf0, tot) &&
@@ -542,12 +542,9 @@ vmbd_plan* vmbd_plan_create(const vmbd_geom* gm, const float* win_table, int32_t
     return nullptr;
   }
   p->bytes = tot;
-  std::vector<float2> tw(TW_LEN);
-  for (int m = 0; m < TW_LEN; ++m) {
-    const double a = -2.0 * M_PI * (double)m / (double)TW_LEN;
-    tw[m] = make_float2((float)std::cos(a), (float)std::sin(a));
-  }
-  hipError_t e = hipMemcpy(p->tw, tw.data(), TW_LEN * sizeof(float2), hipMemcpyHostToDevice);
+  std::vector<float2> tw(TW_PLAN);
+  twiddle_table(tw.data());
+  hipError_t e = hipMemcpy(p->tw, tw.data(), tw.size() * sizeof(float2), hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMemcpy(p->win, win_table, (size_t)n_win * g.sw0 * g.sw1 * sizeof(float), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(p->win_idx, win_idx, (size_t)g.Pf * sizeof(int), hipMemcpyHostToDevice);

@@ -143,7 +143,7 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
   float2* sl = sm + cc * SL;
 
   Twiddles<TH> T;
-  twiddles_init<TH, true>(T, t, tw);
+  twiddles_init<TH>(T, t, tw);
 
   const Halves<TH> hy(t, tw);
   const Half hx = half_tab(min(c, NB - 2), g.Tw, tw);

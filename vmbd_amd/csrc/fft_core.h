@@ -20,10 +20,19 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 namespace vmbd {
 
 // Twiddle table length.  tw[m] = exp(-2 pi i m / TW_LEN), rounded from FP64.
 constexpr int TW_LEN = 1024;
+// A plan's table goes on with the twiddles of the passes after the first as the
+// butterflies take them (Twiddles), each array 16 entries apart so that the
+// lanes of a transform read consecutive ones: the second passes of radix 2, 4,
+// 8 and 16, then the third pass of 512 points.
+constexpr int TW_P2 = TW_LEN;
+constexpr int TW_P3 = TW_P2 + 240;
+constexpr int TW_PLAN = TW_P3 + 128;
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
@@ -54,8 +63,8 @@ __device__ __forceinline__ void wave_sync() {
 // and an FMA takes the issue slot of an addition, so both passes are written
 // to put their multiplications into FMAs.  Per 256-point transform and thread
 // (16 points): first pass 144 (from 160: constant twiddles factored out of
-// the sums), second pass 192 (from 160 + 60 for the separate products), 336
-// instead of 380 slots, with 8 twiddle registers pairs instead of 15.
+// the sums), second pass 208 (from 160 + 60 for the separate products), 352
+// instead of 380 slots, with 8 twiddle register pairs instead of 15.
 #define VMBD_R2H 0.70710678118654752440f
 #define VMBD_C8 0.92387953251128675613f  // cos(pi/8)
 #define VMBD_S8 0.38268343236508977173f  // sin(pi/8)
@@ -171,21 +180,38 @@ __device__ __forceinline__ void dft16(float2 (&v)[16]) {
   for (int i = 0; i < 16; ++i) v[i] = o[i];
 }
 
-// Radix-2 butterfly with its twiddle in the sums, six FMAs:
-// a' = a + W b, b' = a - W b = 2a - a'.  w: forward twiddle (conjugated for
-// S = +1); ROT: W = S i w.
+// Radix-2 butterflies hi = a + W b, lo = a - W b.  w: forward twiddle
+// (conjugated for S = +1); ROT: W = S i w.
+// bfly_tan: w as (cos, tan) of its angle, |angle| < pi/2; W b = cos (b + i tan b)
+// and both outputs are FMAs of a and that, six in all (Linzer and Feig,
+// "Implementation of efficient FFT algorithms on fused multiply-add
+// architectures", 1993).  bfly_exp: w as (cos, sin), any angle, eight FMAs (as a
+// product and two sums it has the same eight slots, but the scheduler then keeps
+// 30 registers more: the two-adjoint pass spilled 33 instead of 5).
+// Each output is rounded from its own sum: lo taken as 2a - hi needs no product
+// of its own either, but carries hi's rounding into a difference that may be
+// small (256 points of smooth input 1.04e-7 rms against 64 bits, 512 points
+// 1.11e-7, where these give 0.90e-7 and 0.95e-7).
 template <int S, bool ROT>
-__device__ __forceinline__ void bfly(float2 a, float2 b, float2 w, float2& hi, float2& lo) {
+__device__ __forceinline__ void bfly_tan(float2 a, float2 b, float2 w, float2& hi, float2& lo) {
   if constexpr (ROT) b = mul_si<S>(b);
-  const float wy = -(float)S * w.y;
-  const float2 t = make_float2(fmaf(-wy, b.y, fmaf(w.x, b.x, a.x)), fmaf(wy, b.x, fmaf(w.x, b.y, a.y)));
-  lo = make_float2(fmaf(2.f, a.x, -t.x), fmaf(2.f, a.y, -t.y));
-  hi = t;
+  const float t = -(float)S * w.y;
+  const float2 u = make_float2(fmaf(-t, b.y, b.x), fmaf(t, b.x, b.y));
+  hi = cfma(w.x, u, a);
+  lo = cfma(-w.x, u, a);
+}
+template <int S>
+__device__ __forceinline__ void bfly_exp(float2 a, float2 b, float2 w, float2& hi, float2& lo) {
+  const float y = -(float)S * w.y;
+  hi = make_float2(fmaf(-y, b.y, fmaf(w.x, b.x, a.x)), fmaf(y, b.x, fmaf(w.x, b.y, a.y)));
+  lo = make_float2(fmaf(y, b.y, fmaf(-w.x, b.x, a.x)), fmaf(-y, b.x, fmaf(-w.x, b.y, a.y)));
 }
 
 // Twiddles of an R-point DFT of w^r x_r: level R (spans R/2) uses w e_R^k,
 // k < R/2, of which the second half is S i times the first; then level R/2
-// with w^2, and so on.  Kept per level: R/4 (one at R = 2), R/2 in all.
+// with w^2, and so on.  Kept per level: R/4 (one at R = 2), R/2 in all.  Above
+// level 2 the kept angles stay below a quarter turn and are held as (cos, tan);
+// the last spans a half turn and is held as (cos, sin).
 template <int R>
 struct TwCount {
   static constexpr int top = R > 2 ? R / 4 : 1;
@@ -201,7 +227,7 @@ template <int R, int S>
 __device__ __forceinline__ void dft_tw(float2* x, const float2* w) {
   if constexpr (R == 2) {
     const float2 a = x[0], b = x[1];
-    bfly<S, false>(a, b, w[0], x[0], x[1]);
+    bfly_exp<S>(a, b, w[0], x[0], x[1]);
   } else {
     constexpr int H = R / 2;
     float2 e[H], o[H];
@@ -214,8 +240,8 @@ __device__ __forceinline__ void dft_tw(float2* x, const float2* w) {
     dft_tw<H, S>(o, w + TwCount<R>::top);
 #pragma unroll
     for (int k = 0; k < H / 2; ++k) {
-      bfly<S, false>(e[k], o[k], w[k], x[k], x[k + H]);
-      bfly<S, true>(e[k + H / 2], o[k + H / 2], w[k], x[k + H / 2], x[k + H / 2 + H]);
+      bfly_tan<S, false>(e[k], o[k], w[k], x[k], x[k + H]);
+      bfly_tan<S, true>(e[k + H / 2], o[k + H / 2], w[k], x[k + H / 2], x[k + H / 2 + H]);
     }
   }
 }
@@ -260,107 +286,73 @@ struct Twiddles {
   }
 };
 
-// twiddle array of an R-point DFT from w = tw[i] (table index i)
+// (cos, tan) of w
+__host__ __device__ __forceinline__ float2 tw_tan(float2 w) { return make_float2(w.x, w.y / w.x); }
+
+// twiddle array of an R-point DFT whose w has table index i
 template <int R>
 __device__ __forceinline__ void tw_load(float2* w, int i, const float2* __restrict__ tw) {
-  constexpr int top = TwCount<R>::top;
-#pragma unroll
-  for (int k = 0; k < top; ++k) w[k] = tw[(i + k * (TW_LEN / R)) & (TW_LEN - 1)];
-  if constexpr (R > 2) tw_load<R / 2>(w + top, 2 * i, tw);
-}
-// the same from w and w^4 by products
-template <int R>
-__device__ __forceinline__ void tw_powers(float2* w, float2 w1, float2 w4) {
-  const float2 e8 = make_float2(VMBD_R2H, -VMBD_R2H);
   if constexpr (R == 2) {
-    w[0] = w1;
-  } else if constexpr (R == 4) {
-    w[0] = w1;
-    w[1] = cmul(w1, w1);
-  } else if constexpr (R == 8) {
-    w[0] = w1;
-    w[1] = cmul(w1, e8);
-    w[2] = cmul(w1, w1);
-    w[3] = w4;
+    w[0] = tw[i];
   } else {
-    w[0] = w1;
-    w[1] = cmul(w1, make_float2(VMBD_C8, -VMBD_S8));
-    w[2] = cmul(w1, e8);
-    w[3] = cmul(w1, make_float2(VMBD_S8, -VMBD_C8));
-    w[4] = cmul(w1, w1);
-    w[5] = cmul(w[4], e8);
-    w[6] = w4;
-    w[7] = cmul(w4, w4);
+    constexpr int top = TwCount<R>::top;
+#pragma unroll
+    for (int k = 0; k < top; ++k) w[k] = tw_tan(tw[i + k * (TW_LEN / R)]);
+    tw_load<R / 2>(w + top, 2 * i, tw);
   }
 }
 
-// table index of the second pass's w for butterfly b, of the third pass's w
-template <int N>
-__device__ __forceinline__ int tw_index1(int t, int b) {
-  return ((t + b * (N / 16)) & 15) * (TW_LEN / (16 * Plan<N>::R1));
-}
-template <int N>
-__device__ __forceinline__ int tw_index2(int t, int b) {
-  return (t + b * (N / 16)) * (TW_LEN / (256 * Plan<N>::R2));
-}
-
-// The twiddles in two steps: twiddles_seed issues the table loads (w and w^4
-// of each second-pass butterfly, w of the third pass's), twiddles_from_seed
-// forms the others, so the loads can be in flight with other work while only
-// the seeds hold registers.
-template <int N>
-struct TwSeed {
-  static constexpr int NB1 = Twiddles<N>::NB1;
-  float2 w1[NB1], w4[NB1], w3[4];
-};
-template <int N>
-__device__ __forceinline__ void twiddles_seed(TwSeed<N>& S, int t, const float2* __restrict__ tw) {
-  if constexpr (Plan<N>::R1 > 1) {
-#pragma unroll
-    for (int b = 0; b < TwSeed<N>::NB1; ++b) {
-      S.w1[b] = tw[tw_index1<N>(t, b)];
-      if constexpr (Plan<N>::R1 > 4) S.w4[b] = tw[4 * tw_index1<N>(t, b) & (TW_LEN - 1)];
-    }
-  }
-  if constexpr (Plan<N>::R2 > 1) {
-#pragma unroll
-    for (int b = 0; b < 4; ++b) S.w3[b] = tw[tw_index2<N>(t, b)];
-  }
-}
-template <int N>
-__device__ __forceinline__ void twiddles_from_seed(Twiddles<N>& T, const TwSeed<N>& S) {
+// PLAN: every twiddle from a plan's table, as many instructions as forming
+// them from w and w^4 takes and without the products' rounding (256 points 15 %
+// rms); otherwise from the exponentials alone.
+template <int N, bool PLAN = true>
+__device__ __forceinline__ void twiddles_init(Twiddles<N>& T, int t, const float2* __restrict__ tw) {
   constexpr int R1 = Plan<N>::R1, R2 = Plan<N>::R2;
+  static_assert(!PLAN || R2 <= 2, "a plan's tiles are at most 512 points");
   if constexpr (R1 > 1) {
 #pragma unroll
-    for (int b = 0; b < TwSeed<N>::NB1; ++b) tw_powers<R1>(T.w + b * Twiddles<N>::C1, S.w1[b], S.w4[b]);
+    for (int b = 0; b < Twiddles<N>::NB1; ++b) {
+      const int k = (t + b * (N / 16)) & 15;
+      float2* w = T.w + b * Twiddles<N>::C1;
+      if constexpr (PLAN) {
+#pragma unroll
+        for (int i = 0; i < Twiddles<N>::C1; ++i) w[i] = (tw + TW_P2 + 16 * (R1 / 2 - 1 + i))[k];
+      } else {
+        tw_load<R1>(w, k * (TW_LEN / (16 * R1)), tw);
+      }
+    }
   }
   if constexpr (R2 > 1) {
 #pragma unroll
-    for (int b = 0; b < 4; ++b) tw_powers<R2>(T.w3 + b * Twiddles<N>::C2, S.w3[b], S.w3[b]);
+    for (int b = 0; b < 4; ++b) {
+      const int j = t + b * (N / 16);
+      if constexpr (PLAN)
+        T.w3[b] = (tw + TW_P3)[j];
+      else if constexpr (R2 == 2)
+        T.w3[b] = tw_tan(tw[2 * j]);
+      else
+        tw_load<R2>(T.w3 + b * Twiddles<N>::C2, j, tw);
+    }
   }
 }
 
-// LOAD=true reads every twiddle from the table (best when a thread performs
-// several transforms); LOAD=false reads the seeds and builds the others
-// (fewer memory instructions for one transform per thread).
-template <int N, bool LOAD = false>
-__device__ __forceinline__ void twiddles_init(Twiddles<N>& T, int t, const float2* __restrict__ tw) {
-  if constexpr (LOAD) {
-    if constexpr (Plan<N>::R1 > 1) {
-#pragma unroll
-      for (int b = 0; b < Twiddles<N>::NB1; ++b)
-        tw_load<(Plan<N>::R1 > 1 ? Plan<N>::R1 : 2)>(T.w + b * Twiddles<N>::C1, tw_index1<N>(t, b), tw);
+// A plan's table on the host (TW_PLAN entries).  Exponentials are rounded from
+// FP64; a tangent is the FP64 sine over the rounded cosine, so that their
+// product is the sine to one rounding.
+inline void twiddle_table(float2* tw) {
+  auto sine = [](int i) { return std::sin(-2.0 * M_PI * (double)i / (double)TW_LEN); };
+  for (int m = 0; m < TW_LEN; ++m)
+    tw[m] = make_float2((float)std::cos(-2.0 * M_PI * (double)m / (double)TW_LEN), (float)sine(m));
+  auto tan_entry = [&](int i) { return make_float2(tw[i].x, (float)(sine(i) / (double)tw[i].x)); };
+  for (int R1 = 2; R1 <= 16; R1 *= 2)
+    for (int k = 0; k < 16; ++k) {
+      float2* o = tw + TW_P2 + 16 * (R1 / 2 - 1) + k;
+      int i = k * (TW_LEN / (16 * R1));
+      for (int R = R1; R > 2; R /= 2, i *= 2)  // the levels in the order of TwCount
+        for (int q = 0; q < R / 4; ++q, o += 16) *o = tan_entry(i + q * (TW_LEN / R));
+      *o = tw[i];
     }
-    if constexpr (Plan<N>::R2 > 1) {
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-        tw_load<(Plan<N>::R2 > 1 ? Plan<N>::R2 : 2)>(T.w3 + b * Twiddles<N>::C2, tw_index2<N>(t, b), tw);
-    }
-  } else {
-    TwSeed<N> S;
-    twiddles_seed<N>(S, t, tw);
-    twiddles_from_seed<N>(T, S);
-  }
+  for (int j = 0; j < 128; ++j) tw[TW_P3 + j] = tan_entry(2 * j);
 }
 
 // The same twiddles in LDS, shared by the transforms of a workgroup and read
@@ -376,7 +368,7 @@ struct TwiddlesLds {
   static __device__ __forceinline__ void fill(float2* p, const float2* __restrict__ tw) {
     if ((int)threadIdx.x < TPT) {
       T r;
-      twiddles_init<N, true>(r, threadIdx.x, tw);
+      twiddles_init<N>(r, threadIdx.x, tw);
 #pragma unroll
       for (int i = 0; i < T::N2; ++i) p[i * TPT + threadIdx.x] = r.w[i];
       if constexpr (T::R2 > 1) {
@@ -425,9 +417,9 @@ __device__ __forceinline__ void stockham_pass(float2 (&v)[16], float2* sl, int t
       // third pass of 512 points: butterfly b + 4 on a quarter turn from b
       const float2 x = q[0], y = q[1];
       if (b < 4)
-        bfly<S, false>(x, y, w[b & 3], q[0], q[1]);
+        bfly_tan<S, false>(x, y, w[b & 3], q[0], q[1]);
       else
-        bfly<S, true>(x, y, w[b & 3], q[0], q[1]);
+        bfly_tan<S, true>(x, y, w[b & 3], q[0], q[1]);
     } else {
       dft_tw<R, S>(q, w + b * TwCount<R>::n);
     }

@@ -448,7 +448,7 @@ __device__ __forceinline__ void cols_body(Geo g, ColIn a, ColIn b, ColIn c3, Col
   if constexpr (Lds::twl)
     T.p = sm + Lds::work;
   else
-    twiddles_init<TH, true>(T, t, tw);
+    twiddles_init<TH>(T, t, tw);
 
   float2 A[16];
   // operands of at most 3*TPT stored rows (PSF rows) take a transform whose
@@ -1070,8 +1070,6 @@ __device__ __forceinline__ void c2r_sum_body(Geo g, OlaDst d, int i0, int fr, fl
   float s0 = 0.f;
   bool f0a = false;
   if (wact) {
-    TwSeed<TW> S;  // twiddle loads in flight with the row fetches
-    twiddles_seed<TW>(S, t, tw);
     // the first three covering patch rows (all of them at 50 % overlap) are
     // fetched together, any further ones one at a time; added in ascending
     // patch-row order, absent rows as zeros.  Returns the row's weight.
@@ -1149,8 +1147,8 @@ __device__ __forceinline__ void c2r_sum_body(Geo g, OlaDst d, int i0, int fr, fl
         s0 = nok ? s0 / (float)nok : 0.f;
       }
     }
-    Twiddles<TW> T;
-    twiddles_from_seed<TW>(T, S);
+    Twiddles<TW> T;  // in flight with the staging and the first pass
+    twiddles_init<TW>(T, t, tw);
     c2r_stage<TW>(v, A, B, sl, t);
     fft<TW, +1>(v, sl, t, T);
   }

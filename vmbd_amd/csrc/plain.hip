@@ -127,7 +127,7 @@ __global__ __launch_bounds__(TB) void k_fft_rows(float2* data, long long rows, f
   const bool act = row < rows;
   float2* rp = data + (act ? row : 0) * N;
   Twiddles<N> T;
-  twiddles_init<N>(T, t, tw);
+  twiddles_init<N, false>(T, t, tw);  // (a caller's table: exponentials only)
   float2 v[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) v[r] = act ? rp[t + TPT * r] : make_float2(0.f, 0.f);
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(TB) void k_fft_cols(float2* data, int Tw, int strip
   for (int r = 0; r < 16; ++r) v[r] = sm[(t + TPT * r) * (CS + 1) + cc];
   __syncthreads();
   Twiddles<N> T;
-  twiddles_init<N>(T, t, tw);
+  twiddles_init<N, false>(T, t, tw);  // (a caller's table: exponentials only)
   fft<N, S>(v, sm + cc * SL, t, T);
   __syncthreads();
 #pragma unroll
