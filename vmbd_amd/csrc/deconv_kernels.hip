@@ -16,6 +16,7 @@
 // D(k) = (P(k) + conj P(-k))/2, N(k) = (P(k) - conj P(-k))/(2i) are formed from
 // it; the quotients of both parts (Hermitian again) are put back as D' + iN'.
 #include "col_device.h"
+#include "div_terms.h"
 #include "fft_core.h"
 #include "ola_kernels.h"
 #include "prof.h"
@@ -24,55 +25,10 @@ namespace vmbd {
 
 namespace {
 
-constexpr float SQRT1_2 = 0.70710678118654752440f;
-
-// Half the angle of a frequency q of T: sin and cos of pi q / T, 0 <= q <= T.
-// Everything the divisions need of a frequency follows from them:
-//   4 sin^2 (the filter energy 2 - 2 cos(2 pi q / T), without its cancellation
-//   near 0), (1 + 2 cos(2 pi q / T))^2 = (3 - 4 sin^2)^2, and the transform
-//   r (e^{-2 pi i q / T} - 1) = -2 r sin (sin + i cos) of the difference
-//   filter r [-1 1] at the tile origin, r = sqrt(2)/2.
-struct Half {
-  float s, c;
-};
-__device__ __forceinline__ Half half_tab(int q, int T, const float2* __restrict__ tw) {
-  const float2 w = tw[(q * (TW_LEN / 2 / T)) & (TW_LEN - 1)];
-  return Half{-w.y, w.x};
-}
-// The half angles of a thread's 16 frequencies k = t + TPT*m from two table
-// entries, by the sum of angles: pi k / T = pi t / T + pi m / 16 in the lower
-// half, and from the other end, pi (T - k) / T, in the upper (so that the
-// small sines of both ends come from small angles).  Sines and cosines per
-// frequency took half of the kernel.
-template <int TH>
-struct Halves {
-  Half lo, hi;
-  __device__ __forceinline__ Halves(int t, const float2* __restrict__ tw)
-      : lo(half_tab(t, TH, tw)), hi(half_tab(TH / 16 - t, TH, tw)) {}
-  __device__ __forceinline__ Half at(int m) const {
-    // sin and cos of pi j / 16
-    constexpr float S[8] = {0.f, 0.19509032201612826785f, 0.38268343236508977173f, 0.55557023301960222474f,
-                            0.70710678118654752440f, 0.83146961230254523708f, 0.92387953251128675613f,
-                            0.98078528040323044913f};
-    constexpr float C[8] = {1.f, 0.98078528040323044913f, 0.92387953251128675613f, 0.83146961230254523708f,
-                            0.70710678118654752440f, 0.55557023301960222474f, 0.38268343236508977173f,
-                            0.19509032201612826785f};
-    const bool up = m >= 8;
-    const int j = up ? 15 - m : m;
-    const Half b = up ? hi : lo;
-    if (j == 0) return Half{b.s, up ? -b.c : b.c};
-    const float s = fmaf(b.s, C[j], b.c * S[j]), c = fmaf(b.c, C[j], -(b.s * S[j]));
-    return Half{s, up ? -c : c};
-  }
-};
-__device__ __forceinline__ float four_sin2(Half h) { return 4.f * h.s * h.s; }
-__device__ __forceinline__ float one_2cos_sq(Half h) {
-  const float c = 3.f - four_sin2(h);
-  return c * c;
-}
-__device__ __forceinline__ float2 diff_filter(Half h) {
-  const float a = -2.f * SQRT1_2 * h.s;
-  return make_float2(a * h.s, a * h.c);
+// the angle a division works with: full for the difference filters of DIV_S
+template <int OP>
+__device__ __forceinline__ Freq div_freq(int q, int T, const float2* __restrict__ tw) {
+  return OP == DIV_S ? full_freq(q, T, tw) : half_freq(q, T, tw);
 }
 
 __device__ __forceinline__ float cabs2(float2 a) { return fmaf(a.x, a.x, a.y * a.y); }
@@ -88,7 +44,7 @@ __device__ __forceinline__ float2 join(float2 d, float2 n) { return make_float2(
 // the division of one (row bin, column frequency) from its operand values
 // (order as in DivOp); hx: row bin, hy: column frequency
 template <int OP>
-__device__ __forceinline__ float2 div_value(const float2 (&o)[4], Half hx, Half hy, DivParams p) {
+__device__ __forceinline__ float2 div_value(const float2 (&o)[4], Freq hx, Freq hy, DivParams p) {
   if constexpr (OP == DIV_X) {
     const float L = four_sin2(hx) + four_sin2(hy);
     return cdivr(cmulc(o[0], o[1]), cabs2(o[1]) + p.alpha * L + p.beta);
@@ -114,7 +70,7 @@ struct DivArity {
 };
 
 template <int TH, int OP>
-__global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, ColIn a2, ColIn a3, DivParams prm,
+__global__ __launch_bounds__(WG, 2) void k_cols_div(Geo g, ColIn a0, ColIn a1, ColIn a2, ColIn a3, DivParams prm,
                                                    ColOut o, float2* __restrict__ spec_out,
                                                    const float2* __restrict__ tw) {
   constexpr int TPT = TH / 16;
@@ -145,8 +101,19 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
   Twiddles<TH> T;
   twiddles_init<TH>(T, t, tw);
 
-  const Halves<TH> hy(t, tw);
-  const Half hx = half_tab(min(c, NB - 2), g.Tw, tw);
+  // the column's row bin; the thread's column frequencies, one table entry
+  // each, loaded ahead of the operands where that costs no wavefront (the one
+  // sine per frequency of DIV_X; loaded where they are used, they take 2 of the
+  // 20 us of a 1024^2 frame)
+  constexpr bool AHEAD = OP == DIV_X && TH <= 256;
+  const Freq hx = div_freq<OP>(min(c, NB - 2), g.Tw, tw);
+  Freq ahead[16];
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int m = 0; m < 16; ++m) ahead[m] = div_freq<OP>(t + TPT * m, TH, tw);
+  }
+  const float2* twf = tw;
+  auto hy = [&](int m) { return AHEAD ? ahead[m] : div_freq<OP>(t + TPT * m, TH, twf); };
   const ColIn ins[4] = {a0, a1, a2, a3};
   // Operands are consumed one at a time: transformed (row-pass outputs) or
   // loaded (spectra), staged when the column is the packed one, and folded
@@ -175,7 +142,7 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
 #pragma unroll
       for (int m = 0; m < 16; ++m) {
         if (j == 0) num[m] = cmulc(v[m], diff_filter(hx));
-        if (j == 1) num[m] = cadd(num[m], cmulc(v[m], diff_filter(hy.at(m))));
+        if (j == 1) num[m] = cadd(num[m], cmulc(v[m], diff_filter(hy(m))));
         if (j == 2) num[m] = cadd(num[m], cdivr(v[m], ab));
         if (j == 3) acc[m] = make_float2(cabs2(v[m]) / ab, 0.f);
       }
@@ -198,25 +165,29 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
 #pragma unroll
         for (int m = 0; m < 16; ++m) {
           float2 ov[4] = {prev[m], v[m], make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
-          num[m] = div_value<OP>(ov, hx, hy.at(m), prm);
+          num[m] = div_value<OP>(ov, hx, hy(m), prm);
         }
       }
     }
   }
+  // loads of their own here and below: kept from the operands' loop, the
+  // entries would cost a wavefront of DIV_S
+  if constexpr (!AHEAD) asm volatile("" : "+s"(twf));
   float2 Z[16];
 #pragma unroll
   for (int m = 0; m < 16; ++m) {
     if constexpr (OP == DIV_S) {
-      const float2 gx = diff_filter(hx), gy = diff_filter(hy.at(m));
+      const float2 gx = diff_filter(hx), gy = diff_filter(hy(m));
       Z[m] = cdivr(num[m], acc[m].x + cabs2(gx) + cabs2(gy) + prm.gamma);
     } else if constexpr (OP == DIV_G) {
-      const Half hk = hy.at(m);
+      const Freq hk = hy(m);
       const float L = one_2cos_sq(hk) * four_sin2(hx) + four_sin2(hk) * one_2cos_sq(hx);
       Z[m] = cdivr(num[m], acc[m].x + prm.alpha * L + prm.beta);
     } else {
       Z[m] = num[m];
     }
   }
+  if constexpr (!AHEAD) asm volatile("" : "+s"(twf));
   if (packed) {
     // both Hermitian parts of every staged operand, the division of each
     // part (row bins 0 and Tw/2), the quotient packed again
@@ -231,8 +202,9 @@ __global__ __launch_bounds__(WG, 1) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
         od[j] = on[j] = make_float2(0.f, 0.f);
         if (j < NA) split(pk[j * SL + lds_pad(k)], pk[j * SL + lds_pad(kr)], od[j], on[j]);
       }
-      // row bins 0 and Tw/2: half angles 0 and pi/2
-      Z[m] = join(div_value<OP>(od, Half{0.f, 1.f}, hy.at(m), prm), div_value<OP>(on, Half{1.f, 0.f}, hy.at(m), prm));
+      // row bins 0 and Tw/2: half angles 0 and pi/2, full 0 and pi
+      constexpr Freq h0{0.f, 1.f}, h1 = OP == DIV_S ? Freq{0.f, -1.f} : Freq{1.f, 0.f};
+      Z[m] = join(div_value<OP>(od, h0, hy(m), prm), div_value<OP>(on, h1, hy(m), prm));
     }
   }
   if constexpr (OP == DIV_SPROD) {
