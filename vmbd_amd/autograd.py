@@ -15,6 +15,7 @@ last row/column; its value and gradient are HIP kernels, and the gradient
 reads the upstream scalar from device memory (no host synchronisation).
 """
 import torch
+import torch.autograd.forward_ad as fwAD
 
 from . import _lib
 from .optGPU import _Scratch
@@ -137,12 +138,15 @@ class OlaLoss(torch.nn.Module):
 
     def _fused(self, x, f, y):
         """The operands the one-function form takes: float32 tensors on the
-        plan's device, y constant and shaped like the result."""
+        plan's device, y constant (no gradient, no forward-mode tangent) and
+        shaped like the result."""
         p = self.plan
         if not all(isinstance(t, torch.Tensor) and t.dtype == torch.float32 and t.device == p.device
                    for t in (x, f, y)):
             return False
-        return not y.requires_grad and x.dim() in (2, 3) and tuple(y.shape) == tuple(x.shape[:-2]) + p.sy
+        if y.requires_grad or fwAD.unpack_dual(y).tangent is not None:
+            return False
+        return x.dim() in (2, 3) and tuple(y.shape) == tuple(x.shape[:-2]) + p.sy
 
     def forward(self, x, f, y):
         if self._fused(x, f, y):
