@@ -280,7 +280,7 @@ class OlaGPU:
         image, border re-padded."""
         const = torch.ones_like(y_gpu)
         yd = self.deconv(y_gpu, mode='xdirect', alpha=alpha, beta=beta, edgetapering=edgetapering)
-        if self.fused and yd.dim() == 2 and factor >= 1 and max(2 * self.sf) <= gputools.TAPER_PSF_MAX:
+        if self.fused and yd.dim() == 2 and np.min(factor) >= 1 and max(2 * self.sf) <= gputools.TAPER_PSF_MAX:
             return self._direct_ratio(yd, const, alpha, beta, edgetapering, factor)
         gputools.cliplower_GPU(yd, 0)
         if edgetapering == 1:
