@@ -21,3 +21,4 @@ extern HostIndex threadIdx;
 void host_wave_sync();
 #define __builtin_amdgcn_fence(order, scope) ((void)0)
 #define __builtin_amdgcn_wave_barrier() host_wave_sync()
+#define __builtin_amdgcn_sched_barrier(mask) ((void)0)

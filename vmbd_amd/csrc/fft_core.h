@@ -27,9 +27,8 @@ namespace vmbd {
 // Twiddle table length.  tw[m] = exp(-2 pi i m / TW_LEN), rounded from FP64.
 constexpr int TW_LEN = 1024;
 // A plan's table goes on with the twiddles of the passes after the first as the
-// butterflies take them (Twiddles), each array 16 entries apart so that the
-// lanes of a transform read consecutive ones: the second passes of radix 2, 4,
-// 8 and 16, then the third pass of 512 points.
+// butterflies take them (Twiddles), the entries of one butterfly together: the
+// second passes of radix 2, 4, 8 and 16, then the third pass of 512 points.
 constexpr int TW_P2 = TW_LEN;
 constexpr int TW_P3 = TW_P2 + 240;
 constexpr int TW_PLAN = TW_P3 + 128;
@@ -237,7 +236,11 @@ __device__ __forceinline__ void dft_tw(float2* x, const float2* w) {
       o[j] = x[2 * j + 1];
     }
     dft_tw<H, S>(e, w + TwCount<R>::top);
+    // halves one after the other: interleaved, the 512-point two-adjoint pass
+    // spills 24 registers instead of 10
+    if constexpr (R == 16) __builtin_amdgcn_sched_barrier(0);
     dft_tw<H, S>(o, w + TwCount<R>::top);
+    if constexpr (R == 16) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int k = 0; k < H / 2; ++k) {
       bfly_tan<S, false>(e[k], o[k], w[k], x[k], x[k + H]);
@@ -316,7 +319,7 @@ __device__ __forceinline__ void twiddles_init(Twiddles<N>& T, int t, const float
       float2* w = T.w + b * Twiddles<N>::C1;
       if constexpr (PLAN) {
 #pragma unroll
-        for (int i = 0; i < Twiddles<N>::C1; ++i) w[i] = (tw + TW_P2 + 16 * (R1 / 2 - 1 + i))[k];
+        for (int i = 0; i < Twiddles<N>::C1; ++i) w[i] = (tw + TW_P2 + 16 * (R1 / 2 - 1))[k * Twiddles<N>::C1 + i];
       } else {
         tw_load<R1>(w, k * (TW_LEN / (16 * R1)), tw);
       }
@@ -346,10 +349,10 @@ inline void twiddle_table(float2* tw) {
   auto tan_entry = [&](int i) { return make_float2(tw[i].x, (float)(sine(i) / (double)tw[i].x)); };
   for (int R1 = 2; R1 <= 16; R1 *= 2)
     for (int k = 0; k < 16; ++k) {
-      float2* o = tw + TW_P2 + 16 * (R1 / 2 - 1) + k;
+      float2* o = tw + TW_P2 + 16 * (R1 / 2 - 1) + k * (R1 / 2);
       int i = k * (TW_LEN / (16 * R1));
       for (int R = R1; R > 2; R /= 2, i *= 2)  // the levels in the order of TwCount
-        for (int q = 0; q < R / 4; ++q, o += 16) *o = tan_entry(i + q * (TW_LEN / R));
+        for (int q = 0; q < R / 4; ++q) *o++ = tan_entry(i + q * (TW_LEN / R));
       *o = tw[i];
     }
   for (int j = 0; j < 128; ++j) tw[TW_P3 + j] = tan_entry(2 * j);
