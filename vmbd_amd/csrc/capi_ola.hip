@@ -1241,8 +1241,8 @@ bool batch_group(BatchGroup& B, vmbd_plan* p, int nframes, const float* x, const
   B.ca_a = shared_in(p->wsG, sr);
   B.ca_b = raw_in(p->wsF, sf);
   B.ca_c = xr.in;
-  B.ca_o1 = col_out_policy(g, ColOut{p->Y1, g.sw0});
-  B.ca_o2 = col_out_policy(g, ColOut{p->Y2, g.sf0});
+  B.ca_o1 = col_out_policy(g, ColOut{p->Y1, g.sw0}, COL_NT_BYTES_ADJ2);
+  B.ca_o2 = col_out_policy(g, ColOut{p->Y2, g.sf0}, COL_NT_BYTES_ADJ2);
   B.ola_adj = dst_adjoint_x(p, xbar);
   ola_fit_rows(B.ola_adj, (long long)B.ola_adj.O0 * nframes);
   // the grouped OLA launch runs WG threads per workgroup for every group

@@ -139,16 +139,20 @@ struct ColOut {
   bool nt = false;  // set by col_out_policy
 };
 
-// Outputs of 4 MB and more (one die's L2) are stored nontemporally: the next
-// launch reads them once, and the write-back then does not push the operand
-// rows out.  Below, the next launch finds the rows in the caches and the
-// stores stay plain.  Measured, plain / nontemporal: 1024^2, 10 x 10 patches,
-// 41^2 PSFs, 32 frames (816 MB) 1360 / 1326 us for the whole step, the PSF
-// gradient of one such frame 53.1 / 52.0 us, 2048^2 with 63^2 PSFs 350 / 343
-// us; 256^2 frames of 0.2 to 1 MB 18.4 / 18.7 and 32.2 / 32.8 us.
-constexpr size_t COL_NT_BYTES = (size_t)4 << 20;
-inline ColOut col_out_policy(const Geo& g, ColOut o) {
-  o.nt = (size_t)g.P * o.nrows * g.NBP * sizeof(float2) >= COL_NT_BYTES;
+// Large outputs are stored nontemporally: the next launch reads them once, and
+// the write-back then does not push the operand rows out of the L2.  Small ones
+// the next launch finds in the caches.  The line lies where both cost the same,
+// further up for the two-adjoint pass, whose second half reads its operands
+// beside the stores of the first.  us per call, plain / nontemporal, by the
+// bytes of the output:
+//   one output: 1.0 MB 19.0 / 19.5, 4.1 22.0 / 22.5, 4.7 25.7 / 25.8, 6.7
+//     24.3 / 23.6, 7.5 20.5 / 19.7, 10 21.8 / 20.9, 15 24.6 / 23.3, 25
+//     27.6 / 26.7, 50 44.1 / 43.2, 75 to 100 even, 200 164 / 151
+//   two adjoints: 8.0 MB 30.3 / 31.7, 12 45.6 / 47.6, 13 39.0 / 41.9, 21
+//     42.0 / 42.3, 41 67.8 / 68.9, 83 124 / 122, 165 213 / 212
+constexpr size_t COL_NT_BYTES = (size_t)6 << 20, COL_NT_BYTES_ADJ2 = (size_t)64 << 20;
+inline ColOut col_out_policy(const Geo& g, ColOut o, size_t line = COL_NT_BYTES) {
+  o.nt = (size_t)g.P * o.nrows * g.NBP * sizeof(float2) >= line;
   return o;
 }
 

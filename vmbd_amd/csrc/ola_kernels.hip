@@ -542,7 +542,8 @@ template <int TH, int OP, int WGC>
 static void cols_op(const Geo& g, const ColIn& a, const ColIn& b, const ColIn& c, const ColOut& o1, const ColOut& o2,
                     float2* spec_out, const float2* tw, hipStream_t st, const dim3& grid) {
   const bool xs = (OP == COL_ADJ1 ? b.rsc : OP == COL_ADJ2 ? c.rsc : a.rsc) != nullptr;
-  const ColOut p1 = col_out_policy(g, o1), p2 = col_out_policy(g, o2);
+  constexpr size_t line = OP == COL_ADJ2 ? COL_NT_BYTES_ADJ2 : COL_NT_BYTES;
+  const ColOut p1 = col_out_policy(g, o1, line), p2 = col_out_policy(g, o2, line);
   auto go = [&](auto k) { hipLaunchKernelGGL(k, grid, dim3(WGC), 0, st, g, a, b, c, p1, p2, spec_out, tw); };
   if constexpr (OP == COL_FWD) {
     if (b.spec)
