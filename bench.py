@@ -328,7 +328,7 @@ def mixed_rate(nframes, timed, steps):
             replay()
         ms = timed(replay, steps)
         out[name] = {'ms_per_step': round(ms, 3), 'frames_per_s': round(nframes / (ms * 1e-3), 1),
-                     'mpix_s': round(mb.pixels / (ms * 1e-3) / 1e6, 1), 'launches_per_step': mb.launches,
+                     'mpix_s': round(mb.pixels / (ms * 1e-3) / 1e6, 1), 'launches_per_step': mb.kernel_launches,
                      'groups': len(mb.groups)}
         outs[name] = [tuple(t.clone() for t in mb.outputs(i)) for i in range(nframes)]
         del mb

@@ -150,6 +150,12 @@ int vmbd_plan_set_window_factors(vmbd_plan* plan, const float* a, const float* b
  * image_rows is not 2.  No counterpart in the reference's API. */
 int vmbd_plan_image_rows_shared(const vmbd_plan* plan, int32_t nframes);
 
+/* Kernel launches of vmbd_ola_forward and vmbd_ola_adjoint_xf with
+ * VMBD_REUSE_ROWS on `nframes` frames: six where the x-adjoint's overlap-add
+ * takes the weighted summed form and shares a launch with the f-adjoint's
+ * stack, else seven.  No counterpart in the reference's API. */
+int vmbd_plan_step_launches(const vmbd_plan* plan, int32_t nframes);
+
 /* Device bytes held by the plan (workspaces, windows, twiddles). */
 size_t vmbd_plan_workspace_bytes(const vmbd_plan* plan);
 /* Output size of the forward operator for the plan's mode (olaGPU.py:127-136). */

@@ -136,10 +136,20 @@ class MixedBatch:
 
     @property
     def launches(self):
-        """Kernel launches per step (passes, without grouping)."""
+        """Passes per step: with grouping one launch each; the groups' own
+        launches run the last two passes together where they can (see
+        ``kernel_launches``)."""
         if self.grouped:
-            return sum(int(_lib.lib().vmbd_batch_launches(vb)) for vb in self._batches().values())
+            return self.kernel_launches
         return 7 * len(self.groups)
+
+    @property
+    def kernel_launches(self):
+        """Kernel launches per step."""
+        L = _lib.lib()
+        if self.grouped:
+            return sum(int(L.vmbd_batch_launches(vb)) for vb in self._batches().values())
+        return sum(int(L.vmbd_plan_step_launches(G['plan']._h, len(G['idx']))) for G in self.groups)
 
     def _batch_step(self, vb):
         _lib.check(_lib.lib().vmbd_batch_step(vb, _lib.stream_ptr()), 'vmbd_batch_step')

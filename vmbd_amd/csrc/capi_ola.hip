@@ -343,8 +343,6 @@ OlaDst dst_adjoint_x(const vmbd_plan* p, float* xbar) {
   return d;
 }
 
-// row transforms of x and f: one launch over both (one geometry, or, with
-// the image rows shared per patch column, a geometry per job)
 // the PSF-shaped results of a call's column pass
 StackDst dst_stack(const vmbd_plan* p, const Geo& g, float* out, const float* axz = nullptr, float beta = 0.f) {
   return StackDst{p->Y2, g.sf0, out, g.sf0, g.sf1, inv_scale(g), axz, beta, fast_div(g.P), nullptr};
@@ -365,6 +363,8 @@ hipError_t launch_rows(const vmbd_plan* p, const Geo& g, std::initializer_list<R
   return launch_rows_r2c(g, jobs, p->tw, st, name);
 }
 
+// row transforms of x and f: one launch over both (one geometry, or, with
+// the image rows shared per patch column, a geometry per job)
 hipError_t launch_xf_rows(const vmbd_plan* p, const Geo& g, const XRows& xr, const RowSrc& sf, hipStream_t st) {
   return launch_rows(p, g, {{xr.g, xr.s, p->wsX}, {g, sf, p->wsF}}, st,
                      xr.shared ? "rows_r2c_x_psf" : "rows_r2c_multi");
@@ -762,6 +762,15 @@ int vmbd_plan_image_rows_shared(const vmbd_plan* p, int32_t nframes) {
   if (nframes < 1 || nframes > p->max_frames)
     return vmbd_fail(VMBD_E_ARG, "nframes=%d outside [1, max_frames=%d]", nframes, p->max_frames);
   return shared_x(p, call_geo(p, nframes), false) ? 1 : 0;
+}
+
+int vmbd_plan_step_launches(const vmbd_plan* p, int32_t nframes) {
+  vmbd_clear_error();
+  if (!p) return vmbd_fail(VMBD_E_ARG, "vmbd_plan_step_launches: null plan");
+  if (nframes < 1 || nframes > p->max_frames)
+    return vmbd_fail(VMBD_E_ARG, "nframes=%d outside [1, max_frames=%d]", nframes, p->max_frames);
+  const Geo g = call_geo(p, nframes);
+  return 5 + ola_stack_launches(g, dst_adjoint_x(p, nullptr), dst_stack(p, g, nullptr));
 }
 
 int vmbd_plan_get_tuning(const vmbd_plan* p, vmbd_tuning* t) {
@@ -1244,8 +1253,8 @@ bool batch_group(BatchGroup& B, vmbd_plan* p, int nframes, const float* x, const
   B.ca_o1 = col_out_policy(g, ColOut{p->Y1, g.sw0}, COL_NT_BYTES_ADJ2);
   B.ca_o2 = col_out_policy(g, ColOut{p->Y2, g.sf0}, COL_NT_BYTES_ADJ2);
   B.ola_adj = dst_adjoint_x(p, xbar);
-  ola_fit_rows(B.ola_adj, (long long)B.ola_adj.O0 * nframes);
   // the grouped OLA launch runs WG threads per workgroup for every group
+  ola_fit_rows(B.ola_adj, (long long)B.ola_adj.O0 * nframes);
   B.stack = dst_stack(p, g, fbar);
   return ok;
 }

@@ -269,6 +269,7 @@ hipError_t launch_rows_c2r_stack(const Geo& g, const StackDst& k, const float2* 
 // the overlap-add takes its weighted summed form
 hipError_t launch_rows_c2r_ola_stack(const Geo& g, const OlaDst& d, const StackDst& k, const float2* tw,
                                      hipStream_t st, int wgs);
+int ola_stack_launches(const Geo& g, const OlaDst& d, const StackDst& k);  // 1 or 2
 // a single-round launch of wgs threads holds every output row's transforms
 int ola_fits(const Geo& g, const OlaDst& d, int wgs);
 // Column pass of a Fourier division (deconv_kernels.hip): operands a[0..na)

@@ -1533,15 +1533,14 @@ __global__ __launch_bounds__(WG) void k_rows_c2r_stack(Geo g, StackDst k, const 
   c2r_stack_body<TW>(g, k, tw, blockIdx.x, blockIdx.y, fl);
 }
 
-template <int TW>
-static int stack_blocks(const StackDst& k) {  // row blocks per patch
-  constexpr int TPW = WG / (TW / 16);
+static int stack_blocks(const Geo& g, const StackDst& k) {  // row blocks per patch
+  const int TPW = WG / (g.Tw / 16);
   return ((k.nrows + 1) / 2 + TPW - 1) / TPW;
 }
 
 template <int TW>
 static hipError_t c2r_stack_t(const Geo& g, const StackDst& k, const float2* tw, hipStream_t st) {
-  const int blocks = stack_blocks<TW>(k);
+  const int blocks = stack_blocks(g, k);
   if (blocks <= 0 || g.P <= 0) return hipSuccess;
   ProfScope ps("rows_c2r_stack", st);
   hipLaunchKernelGGL(k_rows_c2r_stack<TW>, dim3((unsigned)g.P, (unsigned)blocks), dim3(WG), 0, st, g, k, tw);
@@ -1581,23 +1580,36 @@ __global__ __launch_bounds__(WG, (TW >= 512 ? 3 : TW >= 64 ? 4 : 1)) void k_rows
   }
 }
 
+// workgroups of that launch; 0 where the two take launches of their own
+static long long ola_stack_blocks(const Geo& g, const OlaDst& d, const StackDst& k) {
+  const int nst = stack_blocks(g, k);
+  if (!d.sumr || !d.wrow || nst <= 0 || d.O0 <= 0 || d.O1 <= 0) return 0;
+  const long long n = (long long)((d.O0 + d.sumr - 1) / d.sumr) * (g.P / g.Pf) + (long long)g.P * nst;
+  return n > INT_MAX ? 0 : n;
+}
+
+int ola_stack_launches(const Geo& g, const OlaDst& d0, const StackDst& k) {
+  OlaDst d = d0;
+  ola_fit_rows(d, (long long)d.O0 * (g.P / g.Pf));
+  return ola_stack_blocks(g, d, k) ? 1 : 2;
+}
+
 template <int TW>
 static hipError_t c2r_ola_stack_t(const Geo& g, const OlaDst& d0, const StackDst& k, const float2* tw, hipStream_t st,
                                   int wgs) {
   const int frames = g.P / g.Pf;
   OlaDst d = d0;
   ola_fit_rows(d, (long long)d.O0 * frames);
-  const int nst = stack_blocks<TW>(k);
-  const long long nbr = d.sumr ? (d.O0 + d.sumr - 1) / d.sumr : 0;
-  const long long nsum = nbr * frames, n = nsum + (long long)g.P * nst;
-  if (!d.sumr || !d.wrow || nst <= 0 || d.O0 <= 0 || d.O1 <= 0 || n > INT_MAX) {
+  const long long n = ola_stack_blocks(g, d, k);
+  if (!n) {
     const hipError_t e = launch_rows_c2r_ola(g, d0, tw, st, wgs);
     return e != hipSuccess ? e : launch_rows_c2r_stack(g, k, tw, st);
   }
+  const int nbr = (d.O0 + d.sumr - 1) / d.sumr;
   const size_t shm = std::max(ola_shared_bytes(g, d), StackLds<TW>::v * sizeof(float2));
   ProfScope ps("rows_c2r_ola_win_stack", st);
-  hipLaunchKernelGGL(k_rows_c2r_sum_stack<TW>, dim3((unsigned)n), dim3(WG), shm, st, g, d, k, (int)nsum,
-                     fast_div((int)nbr), tw);
+  hipLaunchKernelGGL(k_rows_c2r_sum_stack<TW>, dim3((unsigned)n), dim3(WG), shm, st, g, d, k, nbr * frames,
+                     fast_div(nbr), tw);
   return hipGetLastError();
 }
 
