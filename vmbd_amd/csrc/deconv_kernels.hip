@@ -102,16 +102,13 @@ __global__ __launch_bounds__(WG, 2) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
   twiddles_init<TH>(T, t, tw);
 
   // the column's row bin; the thread's column frequencies, one table entry
-  // each, loaded ahead of the operands where that costs no wavefront (the one
-  // sine per frequency of DIV_X; loaded where they are used, they take 2 of the
-  // 20 us of a 1024^2 frame)
-  constexpr bool AHEAD = OP == DIV_X && TH <= 256;
+  // each, in flight with the first operand's transform where keeping them costs
+  // no wavefront.  1024^2, us per call of 'direct' (two divisions) / 'gdirect' /
+  // 'sparse' (nine): 83.3 / 80.2 / 613; loaded where they are used 87.0 / 82.3 /
+  // 625
+  constexpr bool AHEAD = OP != DIV_SPROD && TH <= 256;
   const Freq hx = div_freq<OP>(min(c, NB - 2), g.Tw, tw);
   Freq ahead[16];
-  if constexpr (AHEAD) {
-#pragma unroll
-    for (int m = 0; m < 16; ++m) ahead[m] = div_freq<OP>(t + TPT * m, TH, tw);
-  }
   const float2* twf = tw;
   auto hy = [&](int m) { return AHEAD ? ahead[m] : div_freq<OP>(t + TPT * m, TH, twf); };
   const ColIn ins[4] = {a0, a1, a2, a3};
@@ -129,6 +126,12 @@ __global__ __launch_bounds__(WG, 2) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
       col_load_spec<TH>(v, ins[j], p, c, NB, t);
     } else {
       col_load<TH>(v, ins[j], p, c, NB, t, grp, row0, cx);
+      if constexpr (AHEAD) {
+        if (j == 0) {
+#pragma unroll
+          for (int m = 0; m < 16; ++m) ahead[m] = div_freq<OP>(t + TPT * m, TH, tw);
+        }
+      }
       if (wact) fft<TH, -1>(v, sl, t, T);
     }
     if (packed) {
