@@ -14,6 +14,9 @@ struct alignas(8) float2 {
 };
 inline float2 make_float2(float x, float y) { return float2{x, y}; }
 
+// the hardware's reciprocal, at its worst: one unit in the last place off
+inline float __builtin_amdgcn_rcpf(float x) { return std::nextafter(1.0f / x, 4.0f * x); }
+
 struct HostIndex {
   unsigned x;
 };
