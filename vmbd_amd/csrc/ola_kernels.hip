@@ -398,7 +398,7 @@ struct ColsLds {
   // both products and the twiddles of three passes: those live in LDS, behind
   // the work area (in registers 25 of them spilled per lane; a 768 x 1024
   // group of 6 x 12 patches: 322 us with the table, 376 without).  At 256
-  // points 6 registers spill and the table costs more than that (one 1024^2
+  // points 5 registers spill and the table costs more than that (one 1024^2
   // frame 21.0 us with it, 20.2 without).
   static constexpr bool twl = OP == COL_ADJ2 && TH >= 512;
   static constexpr int v = work + (twl ? TwiddlesLds<TH>::floats2 : 0);
