@@ -418,37 +418,13 @@ struct RowTiles {
   }
 };
 
-// This block's share of the TV sum, four pixels per thread in flight.  Rows of
-// more than 512 pixels go to the blocks whole, where there is one for each (a
-// row's later pieces are then in flight with its first: 2048^2 12.5 us, in tiles
-// 18.8); narrower and fewer rows in tiles of 1024 pixels, or of 256 where those
-// would leave blocks without one (32 images of 512^2: 45 us by rows, 36 in
-// tiles; 3200 of 41 x 41: 264 and 20; three rows of 200000: 154 and 8).
+// This block's share of the TV sum, four pixels per thread in flight, in tiles
+// of 1024 pixels, or of 256 where those would leave blocks without one.  With
+// whole rows to a block and four pieces of a row in flight, us, before and now:
+// 1024^2 7.7 / 7.7, 2048^2 12.5 / 12.2, 4096^2 54.6 / 34.9, 32 images of 512^2
+// 45 / 20.6, 3200 of 41 x 41 264 / 15.0, three rows of 200000 154 / 7.5.
 __device__ __forceinline__ double tv_rows(const float* __restrict__ x, long long rows, int H, int W, float eps2) {
   double v = 0.0;
-  if (W > 512 && rows >= (int)gridDim.x) {
-    for (long long rho = blockIdx.x; rho < rows; rho += gridDim.x) {
-      const int i = (int)(rho % H);
-      const float* s = x + rho * W;
-      const bool down = i + 1 < H;
-      for (int j0 = threadIdx.x; j0 < W; j0 += 4 * TB) {
-        float c[4], r[4], d[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int j = min(j0 + e * TB, W - 1);
-          c[e] = s[j];
-          r[e] = s[min(j + 1, W - 1)];
-          d[e] = down ? s[j + W] : c[e];
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float a = r[e] - c[e], b = d[e] - c[e];
-          if (j0 + e * TB < W) v += (double)sqrtf(a * a + b * b + eps2);
-        }
-      }
-    }
-    return v;
-  }
   RowTiles t(rows, H, W, rows * W >= 4LL * TB * gridDim.x ? 4 * TB : TB);
   int col[4], row[4];  // of this thread's pixels within a tile
 #pragma unroll
@@ -462,19 +438,22 @@ __device__ __forceinline__ double tv_rows(const float* __restrict__ x, long long
     const float* s = x + t.first();
     const int n = t.count(), j0 = t.c * t.T;
     float c[4], r[4], d[4];
+    bool right[4], below[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {  // no load behind a test: a missing neighbour is the pixel itself
+    for (int e = 0; e < 4; ++e) {  // no load behind a test: a missing neighbour reads the pixel itself
       const int q = min((int)threadIdx.x + e * TB, n - 1);
       int i = t.i + row[e];
       if (i >= H) i -= H;
       const bool in = (int)threadIdx.x + e * TB < n;
+      right[e] = in && j0 + col[e] + 1 < W;
+      below[e] = in && i + 1 < H;
       c[e] = s[q];
-      r[e] = s[q + (in && j0 + col[e] + 1 < W ? 1 : 0)];
-      d[e] = s[(long long)q + (in && i + 1 < H ? W : 0)];
+      r[e] = s[q + (right[e] ? 1 : 0)];
+      d[e] = s[(long long)q + (below[e] ? W : 0)];
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float a = r[e] - c[e], b = d[e] - c[e];
+    for (int e = 0; e < 4; ++e) {  // (and counts 0, whatever the pixel: inf - inf is not 0)
+      const float a = right[e] ? r[e] - c[e] : 0.f, b = below[e] ? d[e] - c[e] : 0.f;
       if ((int)threadIdx.x + e * TB < n) v += (double)sqrtf(a * a + b * b + eps2);
     }
   }
