@@ -101,16 +101,25 @@ __global__ __launch_bounds__(WG, 2) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
   Twiddles<TH> T;
   twiddles_init<TH>(T, t, tw);
 
-  // the column's row bin; the thread's column frequencies, one table entry
-  // each, in flight with the first operand's transform where keeping them costs
-  // no wavefront.  1024^2, us per call of 'direct' (two divisions) / 'gdirect' /
-  // 'sparse' (nine): 83.3 / 80.2 / 613; loaded where they are used 87.0 / 82.3 /
-  // 625
-  constexpr bool AHEAD = OP != DIV_SPROD && TH <= 256;
+  // the column's row bin; the column frequencies, one table entry each, set up
+  // in LDS for all columns of the workgroup beside the first operand's loads
+  // (16 loads per thread are 256 per CU and round, 16 cycles each).  DIV_X keeps
+  // the sines only, which leaves four workgroups per CU; DIV_G has registers for
+  // its thread's entries up to 256 points.  us per call, 1024^2 / 700 x 900 (512
+  // points): 'direct' 82.0 / 67.6, in registers 83.3 / 75; 'gdirect' in registers
+  // 80.2, in LDS 82.0 / 54.9; 'sparse' 607 / 434, loaded where used 625 / 476.
   const Freq hx = div_freq<OP>(min(c, NB - 2), g.Tw, tw);
-  Freq ahead[16];
-  const float2* twf = tw;
-  auto hy = [&](int m) { return AHEAD ? ahead[m] : div_freq<OP>(t + TPT * m, TH, twf); };
+  constexpr bool SINE = OP == DIV_X, REG = OP == DIV_G && TH <= 256, LDS = !REG && OP != DIV_SPROD;
+  __shared__ std::conditional_t<SINE, float, Freq> fq[LDS ? TH : 1];
+  Freq own[REG ? 16 : 1];
+  auto hy = [&](int m) {
+    if constexpr (SINE)
+      return Freq{fq[t + TPT * m], 0.f};
+    else if constexpr (REG)
+      return own[m];
+    else
+      return fq[t + TPT * m];
+  };
   const ColIn ins[4] = {a0, a1, a2, a3};
   // Operands are consumed one at a time: transformed (row-pass outputs) or
   // loaded (spectra), staged when the column is the packed one, and folded
@@ -126,11 +135,19 @@ __global__ __launch_bounds__(WG, 2) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
       col_load_spec<TH>(v, ins[j], p, c, NB, t);
     } else {
       col_load<TH>(v, ins[j], p, c, NB, t, grp, row0, cx);
-      if constexpr (AHEAD) {
-        if (j == 0) {
+      if (REG && j == 0) {
 #pragma unroll
-          for (int m = 0; m < 16; ++m) ahead[m] = div_freq<OP>(t + TPT * m, TH, tw);
+        for (int m = 0; m < 16; ++m) own[REG ? m : 0] = div_freq<OP>(t + TPT * m, TH, tw);
+      }
+      if (LDS && j == 0) {
+        for (int k = threadIdx.x; k < TH; k += WG) {
+          const Freq h = div_freq<OP>(k, TH, tw);
+          if constexpr (SINE)
+            fq[k] = h.s;
+          else
+            fq[k] = h;
         }
+        __syncthreads();
       }
       if (wact) fft<TH, -1>(v, sl, t, T);
     }
@@ -173,9 +190,6 @@ __global__ __launch_bounds__(WG, 2) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
       }
     }
   }
-  // loads of their own here and below: kept from the operands' loop, the
-  // entries would cost a wavefront of DIV_S
-  if constexpr (!AHEAD) asm volatile("" : "+s"(twf));
   float2 Z[16];
 #pragma unroll
   for (int m = 0; m < 16; ++m) {
@@ -190,7 +204,6 @@ __global__ __launch_bounds__(WG, 2) void k_cols_div(Geo g, ColIn a0, ColIn a1, C
       Z[m] = num[m];
     }
   }
-  if constexpr (!AHEAD) asm volatile("" : "+s"(twf));
   if (packed) {
     // both Hermitian parts of every staged operand, the division of each
     // part (row bins 0 and Tw/2), the quotient packed again
